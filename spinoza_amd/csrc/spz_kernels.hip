@@ -381,41 +381,6 @@ __global__ void k_finish1(const double *__restrict__ partials, double *__restric
 }
 
 // ---------------------------------------------------------------------------
-// Inverse-CDF sampling: one thread per uniform (rule restated in the oracle).
-// ---------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(kThreads)
-k_sample(const T *__restrict__ re, const T *__restrict__ im, uint64_t N,
-         const double *__restrict__ P, const double *__restrict__ W, uint64_t nb,
-         int64_t lastnz, const double *__restrict__ U, uint64_t k, uint64_t *__restrict__ out)
-{
-    uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= k) return;
-    double total = P[nb];
-    double x = U[s] * total;
-    uint64_t lo = 0, hi = nb;
-    while (lo < hi) {
-        uint64_t mid = lo + (hi - lo) / 2;
-        if (P[mid + 1] > x) hi = mid; else lo = mid + 1;
-    }
-    uint64_t b = lo < nb ? lo : (uint64_t)lastnz;
-    double acc = P[b];
-    uint64_t j0 = b * kRB, j1 = j0 + kRB;
-    if (j1 > N) j1 = N;
-    int64_t pick = -1, lastw = -1;
-    for (uint64_t j = j0; j < j1; j++) {
-        double xr = re[j], xi = im[j];
-        double w = xr * xr + xi * xi;
-        if (w > 0.0) lastw = (int64_t)j;
-        acc = acc + w;
-        if (acc > x) { pick = (int64_t)j; break; }
-    }
-    if (pick < 0) pick = lastw;
-    out[s] = (uint64_t)pick;
-    (void)W;
-}
-
-// ---------------------------------------------------------------------------
 // Dispatch helpers
 // ---------------------------------------------------------------------------
 template <typename T, int AK>
@@ -741,34 +706,11 @@ int ising_energy_noalloc(const spz_state_s *s, double hx, double *out)
     return SPZ_OK;
 }
 
-int norm_block_partials(const spz_state_s *s, std::vector<double> &W)
+// Level-1 pairs of |psi|^2, one per block of 4096 indices, left in
+// rt().d_partials (for sampling).
+int norm_level1(const spz_state_s *s, uint64_t *nb)
 {
-    uint64_t nb;
-    SPZ_TRY(reduce_level1(s, nullptr, TERM_NORM, 0, 0, 0.0, &nb));
-    std::vector<double> pairs(2 * nb);
-    SPZ_HIP(hipMemcpyAsync(pairs.data(), rt().d_partials, sizeof(double) * 2 * nb,
-                           hipMemcpyDeviceToHost, rt().stream));
-    SPZ_HIP(hipStreamSynchronize(rt().stream));
-    W.resize(nb);
-    for (uint64_t b = 0; b < nb; b++) W[b] = pairs[2 * b] + pairs[2 * b + 1];
-    return SPZ_OK;
-}
-
-int launch_sample(const spz_state_s *s, const double *d_prefix, uint64_t nb, int64_t lastnz,
-                  const double *d_u, uint64_t k, uint64_t *d_out)
-{
-    unsigned g = (unsigned)((k + kThreads - 1) / kThreads);
-    LaunchTimer tm(SPZ_K_OTHER, 0.0);
-    if (s->prec == SPZ_F64)
-        hipLaunchKernelGGL((k_sample<double>), dim3(g), dim3(kThreads), 0, rt().stream,
-                           (const double *)s->re, (const double *)s->im, s->N, d_prefix, nullptr,
-                           nb, lastnz, d_u, k, d_out);
-    else
-        hipLaunchKernelGGL((k_sample<float>), dim3(g), dim3(kThreads), 0, rt().stream,
-                           (const float *)s->re, (const float *)s->im, s->N, d_prefix, nullptr,
-                           nb, lastnz, d_u, k, d_out);
-    SPZ_HIP(hipGetLastError());
-    return SPZ_OK;
+    return reduce_level1(s, nullptr, TERM_NORM, 0, 0, 0.0, nb);
 }
 
 }  // namespace spz

@@ -611,38 +611,7 @@ int spz_sample(spz_state s, const double *uniforms, uint64_t k, uint64_t *out)
     SPZ_TRY(check_state(s));
     if (k == 0) return SPZ_OK;
     if (!uniforms || !out) return fail(SPZ_ERR_ARG, "null uniforms/output");
-    std::vector<double> W;
-    SPZ_TRY(norm_block_partials(s, W));
-    uint64_t nb = W.size();
-    std::vector<double> P(nb + 1);
-    P[0] = 0.0;
-    int64_t lastnz = -1;
-    for (uint64_t b = 0; b < nb; b++) {
-        P[b + 1] = P[b] + W[b];
-        if (W[b] > 0.0) lastnz = (int64_t)b;
-    }
-    if (lastnz < 0) return fail(SPZ_ERR_PROB, "sampling a zero state");
-    double *dP = nullptr, *dU = nullptr;
-    uint64_t *dO = nullptr;
-    SPZ_HIP(hipMalloc(&dP, (nb + 1) * sizeof(double)));
-    if (hipMalloc(&dU, k * sizeof(double)) != hipSuccess || hipMalloc(&dO, k * sizeof(uint64_t)) != hipSuccess) {
-        hipFree(dP);
-        if (dU) hipFree(dU);
-        return fail(SPZ_ERR_OOM, "sampling scratch allocation failed");
-    }
-    int rc = SPZ_OK;
-    if (hipMemcpyAsync(dP, P.data(), (nb + 1) * sizeof(double), hipMemcpyHostToDevice, g_rt.stream) != hipSuccess ||
-        hipMemcpyAsync(dU, uniforms, k * sizeof(double), hipMemcpyHostToDevice, g_rt.stream) != hipSuccess)
-        rc = fail(SPZ_ERR_HIP, "sampling upload failed");
-    if (rc == SPZ_OK) rc = launch_sample(s, dP, nb, lastnz, dU, k, dO);
-    if (rc == SPZ_OK &&
-        hipMemcpyAsync(out, dO, k * sizeof(uint64_t), hipMemcpyDeviceToHost, g_rt.stream) != hipSuccess)
-        rc = fail(SPZ_ERR_HIP, "sampling download failed");
-    hipStreamSynchronize(g_rt.stream);
-    hipFree(dP);
-    hipFree(dU);
-    hipFree(dO);
-    return rc;
+    return sample_state(s, uniforms, k, out);
 }
 
 int spz_profile_enable(int on)

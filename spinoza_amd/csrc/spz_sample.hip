@@ -1,0 +1,395 @@
+// spz_sample.hip -- inverse-CDF sampling of |psi|^2 (replaces
+// reservoir_sampling, core.rs:125-129).
+//
+// The rule (the oracle restates it): W_b is the compensated partial of block
+// b of 4096 indices, P the running sums of W in block order; a uniform u asks
+// for x = u P_nb, picks the first block with P_{b+1} > x and then the first j
+// of it with P_b + w_0 + ... + w_j > x, all sums in index order.  Both sums are
+// chains of dependent additions that fix the rounding, so they cannot be
+// reassociated; what is parallel is everything around them.
+//
+// What bounded it: one thread per uniform walked its block alone, 4096
+// dependent loads and additions at memory latency (859 us for 4096 samples of
+// 20 qubits, 734 us for 1000 of 17), with the block sums carried to the host
+// and back and six allocations around it.  Here the samples are counted into
+// their blocks (atomic ranks, one scan, one scatter) and one workgroup per
+// block that has any forms the block's 4096 running sums once in LDS (loads
+// and squares by the whole workgroup, the chain by one lane at the FP64
+// addition latency) and answers all of its samples by bisection: a running
+// sum of non-negative terms never decreases, so the first one above x is
+// where the walk stopped.  (A NaN or infinite weight makes the total NaN, no
+// sum compares above x, and every sample falls to the last index of positive
+// weight, as in the walk.)
+#include <string.h>
+
+#include <algorithm>
+
+#include "spz_internal.h"
+
+namespace spz {
+
+namespace {
+
+constexpr int kT = 256;
+constexpr uint32_t kBlock = 4096;      // indices per block of the sampling rule
+constexpr uint32_t kPiece = 1u << 20;  // uniforms per round (bounds the scratch)
+
+struct SampleMeta {
+    int64_t lastnz;    // last block with a positive weight (-1: none)
+    double total;      // P_nb
+    uint32_t nslots;   // blocks that hold samples of this round
+    uint32_t pad;
+};
+
+struct Slot {
+    uint32_t block, start, count;
+};
+
+// The running sums of `steps` groups of kStep LDS values, by one lane: ck[i] is
+// the sum up to and with group i.  One dependent addition per value, the reads
+// one group ahead of it.  Only every kStep-th sum is stored (a store per value
+// would double the LDS traffic and make that, not the addition, the pace:
+// 12.7 against 5 ns per value); whoever needs one in between adds at most
+// kStep terms to the sum before, the same additions in the same order.
+constexpr uint32_t kStep = 16;
+
+__device__ __forceinline__ double chain(const double *v, uint32_t steps, double acc, double *ck)
+{
+    double t[kStep], nx[kStep];
+#pragma unroll
+    for (uint32_t k = 0; k < kStep; k++) t[k] = v[k];
+    for (uint32_t i = 0; i < steps; i++) {
+        const uint32_t n = i + 1 < steps ? (i + 1) * kStep : 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kStep; k++) nx[k] = v[n + k];
+#pragma unroll
+        for (uint32_t k = 0; k < kStep; k++) acc = acc + t[k];
+        ck[i] = acc;
+#pragma unroll
+        for (uint32_t k = 0; k < kStep; k++) t[k] = nx[k];
+    }
+    return acc;
+}
+
+// P[0..nb] from the level-1 pairs, the total and the last positive block; also
+// clears the blocks' sample counts.  One workgroup: the chain over blocks is
+// serial, the next chunk's pairs are loaded while it runs.
+constexpr int kPT = 1024;
+constexpr uint32_t kPC = 2048;  // blocks per chunk
+
+__global__ void __launch_bounds__(kPT)
+k_block_prefix(const double *__restrict__ pairs, uint64_t nb, double *__restrict__ P,
+               uint32_t *__restrict__ counts, SampleMeta *__restrict__ meta)
+{
+    __shared__ __align__(16) double v[kPC];
+    __shared__ double ck[kPC / kStep], carry;
+    __shared__ long long last;
+    const uint32_t tid = threadIdx.x;
+    if (tid == 0) {
+        carry = 0.0;
+        last = -1;
+        P[0] = 0.0;
+    }
+    double w[kPC / kPT];
+    long long mine = -1;
+    auto fetch = [&](uint64_t base) {
+#pragma unroll
+        for (uint32_t e = 0; e < kPC / kPT; e++) {
+            const uint64_t b = base + e * kPT + tid;
+            w[e] = b < nb ? pairs[2 * b] + pairs[2 * b + 1] : 0.0;
+            if (b < nb) counts[b] = 0u;
+        }
+    };
+    fetch(0);
+    for (uint64_t base = 0; base < nb; base += kPC) {
+        const uint32_t cnt = (uint32_t)(nb - base < kPC ? nb - base : kPC);
+#pragma unroll
+        for (uint32_t e = 0; e < kPC / kPT; e++) {
+            v[e * kPT + tid] = w[e];
+            if (w[e] > 0.0) mine = (long long)(base + e * kPT + tid);
+        }
+        if (base + kPC < nb) fetch(base + kPC);
+        __syncthreads();
+        const double before = carry;
+        __syncthreads();
+        if (tid == 0) carry = chain(v, (cnt + kStep - 1) / kStep, before, ck);
+        __syncthreads();
+#pragma unroll
+        for (uint32_t e = 0; e < kPC / kPT; e++) {
+            const uint32_t i = e * kPT + tid;
+            if (i < cnt) {
+                const uint32_t g = i / kStep;
+                double acc = g ? ck[g - 1] : before;
+                for (uint32_t j = g * kStep; j <= i; j++) acc = acc + v[j];
+                P[base + i + 1] = acc;
+            }
+        }
+        __syncthreads();
+    }
+    if (mine >= 0) atomicMax(&last, mine);
+    __syncthreads();
+    if (tid == 0) {
+        meta->lastnz = last;
+        meta->total = carry;
+        meta->nslots = 0;
+    }
+}
+
+// The block of every uniform, and its rank among the block's samples.
+__global__ void __launch_bounds__(kT)
+k_sample_block(const double *__restrict__ P, uint64_t nb, const SampleMeta *__restrict__ meta,
+               const double *__restrict__ U, uint32_t k, uint32_t *__restrict__ counts,
+               uint32_t *__restrict__ blk, uint32_t *__restrict__ rank)
+{
+    const uint32_t s = blockIdx.x * kT + threadIdx.x;
+    if (s >= k || meta->lastnz < 0) return;
+    const double x = U[s] * meta->total;
+    uint64_t lo = 0, hi = nb;
+    while (lo < hi) {
+        const uint64_t mid = lo + (hi - lo) / 2;
+        if (P[mid + 1] > x) hi = mid;
+        else lo = mid + 1;
+    }
+    const uint32_t b = (uint32_t)(lo < nb ? lo : (uint64_t)meta->lastnz);
+    blk[s] = b;
+    rank[s] = atomicAdd(&counts[b], 1u);
+}
+
+// Exclusive scan of the counts (in place: counts[b] becomes the block's first
+// position) and the list of blocks that hold samples.  One workgroup.
+__global__ void __launch_bounds__(kPT)
+k_sample_scan(uint32_t *__restrict__ counts, uint64_t nb, Slot *__restrict__ slots,
+              SampleMeta *__restrict__ meta)
+{
+    __shared__ uint32_t ws[kPT / 64], wz[kPT / 64];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    uint32_t base_s = 0, base_z = 0;
+    for (uint64_t b0 = 0; b0 < nb; b0 += kPT) {
+        const uint64_t b = b0 + tid;
+        const uint32_t c = b < nb ? counts[b] : 0u;
+        uint32_t s = c, z = c ? 1u : 0u;  // inclusive scans over the wavefront
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t us = __shfl_up(s, d), uz = __shfl_up(z, d);
+            if (lane >= (uint32_t)d) {
+                s += us;
+                z += uz;
+            }
+        }
+        if (lane == 63) {
+            ws[wave] = s;
+            wz[wave] = z;
+        }
+        __syncthreads();
+        uint32_t os = base_s, oz = base_z;
+        for (uint32_t w = 0; w < kPT / 64; w++) {
+            if (w < wave) {
+                os += ws[w];
+                oz += wz[w];
+            }
+            base_s += ws[w];
+            base_z += wz[w];
+        }
+        if (b < nb) counts[b] = os + s - c;
+        if (c) slots[oz + z - 1] = Slot{(uint32_t)b, os + s - c, c};
+        __syncthreads();
+    }
+    if (tid == 0) meta->nslots = base_z;
+}
+
+__global__ void __launch_bounds__(kT)
+k_sample_order(const uint32_t *__restrict__ starts, const SampleMeta *__restrict__ meta,
+               const uint32_t *__restrict__ blk, const uint32_t *__restrict__ rank, uint32_t k,
+               uint32_t *__restrict__ order)
+{
+    const uint32_t s = blockIdx.x * kT + threadIdx.x;
+    if (s < k && meta->lastnz >= 0) order[starts[blk[s]] + rank[s]] = s;
+}
+
+// One workgroup per block that holds samples; a sample bisects the group sums,
+// then walks its group.
+template <typename T>
+__global__ void __launch_bounds__(kT)
+k_sample_pick(const T *__restrict__ re, const T *__restrict__ im, uint64_t N,
+              const double *__restrict__ P, const SampleMeta *__restrict__ meta,
+              const Slot *__restrict__ slots, const uint32_t *__restrict__ order,
+              const double *__restrict__ U, uint64_t *__restrict__ out)
+{
+    __shared__ __align__(16) double v[kBlock];
+    __shared__ double ck[kBlock / kStep];  // sum up to and with step i
+    __shared__ int last;
+    if (blockIdx.x >= meta->nslots) return;  // uniform over the workgroup
+    const Slot sl = slots[blockIdx.x];
+    const uint32_t tid = threadIdx.x;
+    const uint64_t j0 = (uint64_t)sl.block * kBlock;
+    const uint32_t cnt = (uint32_t)(N - j0 < kBlock ? N - j0 : kBlock);
+    const uint32_t steps = (cnt + kStep - 1) / kStep;
+    if (tid == 0) last = -1;
+    int mine = -1;
+    constexpr uint32_t E = kBlock / kT;
+    if (cnt == kBlock) {  // all loads in flight together
+        T a[E], b[E];
+#pragma unroll
+        for (uint32_t e = 0; e < E; e++) {
+            a[e] = re[j0 + e * kT + tid];
+            b[e] = im[j0 + e * kT + tid];
+        }
+#pragma unroll
+        for (uint32_t e = 0; e < E; e++) {
+            const double x = a[e], y = b[e];
+            const double w = x * x + y * y;
+            v[e * kT + tid] = w;
+            if (w > 0.0) mine = (int)(e * kT + tid);
+        }
+    } else {  // a state smaller than a block: its last step is padded with zeros
+        for (uint32_t i = tid; i < steps * kStep; i += kT) {
+            double w = 0.0;
+            if (i < cnt) {
+                const double x = re[j0 + i], y = im[j0 + i];
+                w = x * x + y * y;
+                if (w > 0.0) mine = (int)i;
+            }
+            v[i] = w;
+        }
+    }
+    __syncthreads();
+    if (mine >= 0) atomicMax(&last, mine);
+    if (tid == 0) chain(v, steps, P[sl.block], ck);
+    __syncthreads();
+    const double total = meta->total;
+    for (uint32_t i = tid; i < sl.count; i += kT) {
+        const uint32_t s = order[sl.start + i];
+        const double x = U[s] * total;
+        uint32_t lo = 0, hi = steps;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (ck[mid] > x) hi = mid;
+            else lo = mid + 1;
+        }
+        uint64_t pick;
+        if (lo < steps) {
+            double acc = lo ? ck[lo - 1] : P[sl.block];
+            uint32_t j = lo * kStep;
+            acc = acc + v[j];
+            while (!(acc > x)) acc = acc + v[++j];  // (ends at ck[lo] > x at the latest)
+            pick = j0 + j;
+        } else {
+            pick = last >= 0 ? j0 + (uint64_t)last : ~0ull;
+        }
+        out[s] = pick;
+    }
+}
+
+// Device and pinned scratch, grown as needed under the library lock; what is
+// over kKeep bytes is given back at the end of the call.
+struct Scratch {
+    void *dev = nullptr, *host = nullptr;
+    size_t dev_cap = 0, host_cap = 0;
+};
+Scratch g_scr;
+constexpr size_t kKeep = 64u << 20;
+
+int reserve(size_t dev_bytes, size_t host_bytes)
+{
+    if (dev_bytes > g_scr.dev_cap) {
+        if (g_scr.dev) SPZ_HIP(hipFree(g_scr.dev));
+        g_scr.dev = nullptr;
+        g_scr.dev_cap = 0;
+        if (hipMalloc(&g_scr.dev, dev_bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            g_scr.dev = nullptr;
+            return fail(SPZ_ERR_OOM, "sampling scratch allocation failed");
+        }
+        g_scr.dev_cap = dev_bytes;
+    }
+    if (host_bytes > g_scr.host_cap) {
+        if (g_scr.host) SPZ_HIP(hipHostFree(g_scr.host));
+        g_scr.host = nullptr;
+        g_scr.host_cap = 0;
+        if (hipHostMalloc(&g_scr.host, host_bytes, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            g_scr.host = nullptr;
+            return fail(SPZ_ERR_OOM, "sampling staging allocation failed");
+        }
+        g_scr.host_cap = host_bytes;
+    }
+    return SPZ_OK;
+}
+
+size_t up(size_t b) { return (b + 255) & ~(size_t)255; }
+
+int sample_rounds(const spz_state_s *s, uint64_t nb, const double *uniforms, uint64_t k,
+                  uint64_t *out)
+{
+    const uint32_t piece = (uint32_t)std::min<uint64_t>(k, kPiece);
+    const uint64_t slots_max = std::min<uint64_t>(piece, nb);
+    // device layout: out and meta together (one copy back), then the rest
+    const size_t o_out = 0, o_meta = up(piece * 8ull), o_u = o_meta + 256;
+    const size_t o_blk = o_u + up(piece * 8ull), o_rank = o_blk + up(piece * 4ull);
+    const size_t o_ord = o_rank + up(piece * 4ull), o_slot = o_ord + up(piece * 4ull);
+    const size_t o_cnt = o_slot + up(slots_max * sizeof(Slot)), o_p = o_cnt + up(nb * 4ull);
+    const size_t dev_bytes = o_p + up((nb + 1) * 8ull);
+    SPZ_TRY(reserve(dev_bytes, o_u));
+    char *d = (char *)g_scr.dev, *h = (char *)g_scr.host;
+    SampleMeta *meta = (SampleMeta *)(d + o_meta);
+    double *U = (double *)(d + o_u), *P = (double *)(d + o_p);
+    uint32_t *blk = (uint32_t *)(d + o_blk), *rank = (uint32_t *)(d + o_rank),
+             *order = (uint32_t *)(d + o_ord), *counts = (uint32_t *)(d + o_cnt);
+    Slot *slots = (Slot *)(d + o_slot);
+    uint64_t *dout = (uint64_t *)(d + o_out);
+    hipStream_t st = rt().stream;
+    LaunchTimer tm(SPZ_K_OTHER, 0.0);
+    for (uint64_t at = 0; at < k; at += piece) {
+        const uint32_t m = (uint32_t)std::min<uint64_t>(piece, k - at);
+        // (the previous round was waited for: the staging buffer is free)
+        memcpy(h, uniforms + at, m * sizeof(double));
+        SPZ_HIP(hipMemcpyAsync(U, h, m * sizeof(double), hipMemcpyHostToDevice, st));
+        const unsigned g = (m + kT - 1) / kT;
+        hipLaunchKernelGGL(k_block_prefix, dim3(1), dim3(kPT), 0, st, rt().d_partials, nb, P,
+                           counts, meta);
+        hipLaunchKernelGGL(k_sample_block, dim3(g), dim3(kT), 0, st, P, nb, meta, U, m, counts,
+                           blk, rank);
+        hipLaunchKernelGGL(k_sample_scan, dim3(1), dim3(kPT), 0, st, counts, nb, slots, meta);
+        hipLaunchKernelGGL(k_sample_order, dim3(g), dim3(kT), 0, st, counts, meta, blk, rank, m,
+                           order);
+        const unsigned gs = (unsigned)std::min<uint64_t>(m, nb);
+        if (s->prec == SPZ_F64)
+            hipLaunchKernelGGL((k_sample_pick<double>), dim3(gs), dim3(kT), 0, st,
+                               (const double *)s->re, (const double *)s->im, s->N, P, meta, slots,
+                               order, U, dout);
+        else
+            hipLaunchKernelGGL((k_sample_pick<float>), dim3(gs), dim3(kT), 0, st,
+                               (const float *)s->re, (const float *)s->im, s->N, P, meta, slots,
+                               order, U, dout);
+        SPZ_HIP(hipGetLastError());
+        SPZ_HIP(hipMemcpyAsync(h, d, o_u, hipMemcpyDeviceToHost, st));
+        SPZ_HIP(hipStreamSynchronize(st));
+        if (((const SampleMeta *)(h + o_meta))->lastnz < 0)
+            return fail(SPZ_ERR_PROB, "sampling a zero state");
+        memcpy(out + at, h, m * sizeof(uint64_t));
+    }
+    return SPZ_OK;
+}
+
+}  // namespace
+
+int sample_state(const spz_state_s *s, const double *uniforms, uint64_t k, uint64_t *out)
+{
+    uint64_t nb;
+    SPZ_TRY(norm_level1(s, &nb));
+    const int rc = sample_rounds(s, nb, uniforms, k, out);
+    if (rc != SPZ_OK) (void)hipStreamSynchronize(rt().stream);  // the scratch is idle again
+    if (g_scr.dev_cap > kKeep) {
+        (void)hipFree(g_scr.dev);
+        g_scr.dev = nullptr;
+        g_scr.dev_cap = 0;
+    }
+    if (g_scr.host_cap > kKeep) {
+        (void)hipHostFree(g_scr.host);
+        g_scr.host = nullptr;
+        g_scr.host_cap = 0;
+    }
+    return rc;
+}
+
+}  // namespace spz
