@@ -23,7 +23,7 @@
 #include <vector>
 
 #include "spz_inplace.h"
-#include "spz_internal.h"
+#include "spz_reduce.h"
 #include "spz_tile.h"
 
 namespace spz {
@@ -566,20 +566,30 @@ int adjoint_grad(spz_state_s *s, const spz_op *ops, uint64_t n_ops, double hx, i
     SPZ_TRY(sc.states_like(s));
     spz_state_s *const wk = &sc.work, *const lm = &sc.lam;  // psi copy, lambda
     SPZ_TRY(spz_state_copy(wk, s));
-    {
-        LaunchTimer tm(SPZ_K_ADJOINT, (double)s->N * (s->prec == SPZ_F64 ? 16.0 : 8.0) * (n + 2));
-        if (s->prec == SPZ_F64)
-            hipLaunchKernelGGL((k_ising_apply<double>), dim3(blocks_for(s->N, kT)), dim3(kT), 0,
-                               rt().stream, (const double *)s->re, (const double *)s->im,
-                               (double *)lm->re, (double *)lm->im, s->N, n, hx);
-        else
-            hipLaunchKernelGGL((k_ising_apply<float>), dim3(blocks_for(s->N, kT)), dim3(kT), 0,
-                               rt().stream, (const float *)s->re, (const float *)s->im,
-                               (float *)lm->re, (float *)lm->im, s->N, n, hx);
-        SPZ_HIP(hipGetLastError());
-    }
     double e = 0.0;
-    SPZ_TRY(reduce(s, lm, TERM_DOT_RE, 0, 0, 0.0, &e));
+    if (s->N >= kRB) {  // H psi and the energy's first level in one pass
+        const uint64_t nb = s->N / kRB;
+        SPZ_TRY(ensure_partials(nb));
+        {
+            LaunchTimer tm(SPZ_K_ADJOINT, 2.0 * (double)s->N * (s->prec == SPZ_F64 ? 16.0 : 8.0));
+            SPZ_TRY(ising_level1(s, hx, lm->re, lm->im, rt().d_partials));
+        }
+        SPZ_TRY(reduce_finish(rt().d_partials, nb, &e));
+    } else {
+        {
+            LaunchTimer tm(SPZ_K_ADJOINT, (double)s->N * (s->prec == SPZ_F64 ? 16.0 : 8.0) * (n + 2));
+            if (s->prec == SPZ_F64)
+                hipLaunchKernelGGL((k_ising_apply<double>), dim3(blocks_for(s->N, kT)), dim3(kT), 0,
+                                   rt().stream, (const double *)s->re, (const double *)s->im,
+                                   (double *)lm->re, (double *)lm->im, s->N, n, hx);
+            else
+                hipLaunchKernelGGL((k_ising_apply<float>), dim3(blocks_for(s->N, kT)), dim3(kT), 0,
+                                   rt().stream, (const float *)s->re, (const float *)s->im,
+                                   (float *)lm->re, (float *)lm->im, s->N, n, hx);
+            SPZ_HIP(hipGetLastError());
+        }
+        SPZ_TRY(reduce(s, lm, TERM_DOT_RE, 0, 0, 0.0, &e));
+    }
     if (energy) *energy = e;
     // ---- reverse sweep -------------------------------------------------------
     const uint64_t per_block = (uint64_t)kT * kGPerThread;

@@ -1,0 +1,343 @@
+// spz_expect.hip -- expectations of many qubits in one pass, and the Ising
+// energy and H psi, for states of at least one reduction block (4096
+// amplitudes).
+//
+// A workgroup owns one block of the reduction tree and holds it in registers:
+// thread t has amplitudes t + 256 e, e = 0..15.  The partner j ^ 2^q of an
+// amplitude is then in another lane of the wavefront (q < 6), in another
+// register of the same thread (8 <= q < 12), or in another wavefront or block
+// (loaded).  Every term and every addition is the reduction tree's own, in its
+// order, so results are bit-identical to one pass per target.
+//
+// What bounded it: one pass over the state, one second-level launch, one copy
+// and one wait per target (23 qubits: 69 passes of 22-28 us and 70 round
+// trips for x, y and z).  Now kExpectGroup targets share a pass, all targets of
+// a call share one second-level launch per pass and one wait, and results land
+// in pinned memory.  x, y and z of all 23 qubits and the energy: 3.08 -> 0.75
+// ms; a pass of 8 targets takes 28 us for z (one state read, then additions)
+// and 64 us for x or y.
+#include <algorithm>
+
+#include "spz_reduce.h"
+
+namespace spz {
+
+namespace {
+
+struct Targets {
+    int32_t q[kExpectGroup];
+    int32_t count;
+};
+
+__device__ __forceinline__ double lane_xor(double x, int mask) { return __shfl_xor(x, mask); }
+
+// Block that workgroup i handles: workgroup i runs on XCD i % 8, and each XCD
+// takes a contiguous eighth of the blocks, so that the partner blocks of the
+// lower block bits are read by the same XCD at about the same time (its L2).
+__device__ __forceinline__ uint64_t xcd_block(uint32_t i, uint64_t nb)
+{
+    return nb >= 8 ? (uint64_t)(i & 7u) * (nb >> 3) + (i >> 3) : i;
+}
+
+// One target's terms: p[e] is the partner of amplitude e.
+template <char OBS>
+__device__ __forceinline__ double expect_term(bool bit, double a, double b, double c, double d)
+{
+    if constexpr (OBS == 'x') {
+        return a * c + b * d;
+    } else {  // (Y psi)_1 = i psi_0, (Y psi)_0 = -i psi_1
+        const double vr = bit ? -d : d, vi = bit ? c : -c;
+        return a * vr + b * vi;
+    }
+}
+
+template <char OBS, int BIT>
+__device__ __forceinline__ void expect_reg(const double *a, const double *b, double &s, double &c)
+{
+#pragma unroll
+    for (int e = 0; e < kRE; e++)
+        add_term(s, c, expect_term<OBS>((e & BIT) != 0, a[e], b[e], a[e ^ BIT], b[e ^ BIT]));
+}
+
+template <typename T, char OBS>
+__global__ void __launch_bounds__(kRT)
+k_expect(const T *__restrict__ re, const T *__restrict__ im, uint64_t nb, Targets tg,
+         double *__restrict__ partials)
+{
+    __shared__ double S[kExpectGroup][kRT], C[kExpectGroup][kRT];
+    const uint32_t tid = threadIdx.x;
+    const uint64_t blk = xcd_block(blockIdx.x, nb), base = blk * kRB;
+    double a[kRE], b[kRE];
+#pragma unroll
+    for (int e = 0; e < kRE; e++) {
+        a[e] = re[base + e * kRT + tid];
+        b[e] = im[base + e * kRT + tid];
+    }
+    if constexpr (OBS == 'z') {
+#pragma unroll
+        for (int e = 0; e < kRE; e++) a[e] = a[e] * a[e] + b[e] * b[e];
+    }
+    for (int t = 0; t < tg.count; t++) {
+        const int q = tg.q[t];
+        double s = 0.0, c = 0.0;
+        if constexpr (OBS == 'z') {  // a (-a) + b (-b) is exactly -(a a + b b)
+            if (q >= 8 && q < 12) {
+#pragma unroll
+                for (int e = 0; e < kRE; e++)
+                    add_term(s, c, ((uint32_t)e >> (q - 8)) & 1u ? -a[e] : a[e]);
+            } else {
+                const bool bit = (((base + tid) >> q) & 1) != 0;
+#pragma unroll
+                for (int e = 0; e < kRE; e++) add_term(s, c, bit ? -a[e] : a[e]);
+            }
+        } else if (q < 6) {
+            const bool bit = ((tid >> q) & 1u) != 0;
+#pragma unroll
+            for (int e = 0; e < kRE; e++) {
+                const double x = lane_xor(a[e], 1 << q), y = lane_xor(b[e], 1 << q);
+                add_term(s, c, expect_term<OBS>(bit, a[e], b[e], x, y));
+            }
+        } else if (q == 8) {
+            expect_reg<OBS, 1>(a, b, s, c);
+        } else if (q == 9) {
+            expect_reg<OBS, 2>(a, b, s, c);
+        } else if (q == 10) {
+            expect_reg<OBS, 4>(a, b, s, c);
+        } else if (q == 11) {
+            expect_reg<OBS, 8>(a, b, s, c);
+        } else {
+            // An amplitude and its partner have the same X and Y term, so a
+            // thread and its partner thread (q = 6, 7: another wavefront),
+            // and a block and its partner block, have the same sums: the
+            // side with the bit clear forms them for both.
+            const uint64_t j0 = base + tid;
+            if ((j0 >> q) & 1) continue;
+            const uint64_t p0 = j0 | (1ull << q);
+            T x[kRE], y[kRE];
+#pragma unroll
+            for (int e = 0; e < kRE; e++) {
+                x[e] = re[p0 + e * kRT];
+                y[e] = im[p0 + e * kRT];
+            }
+#pragma unroll
+            for (int e = 0; e < kRE; e++)
+                add_term(s, c, expect_term<OBS>(false, a[e], b[e], x[e], y[e]));
+            if (q < 8) {
+                S[t][tid | (1u << q)] = s;
+                C[t][tid | (1u << q)] = c;
+            }
+        }
+        S[t][tid] = s;
+        C[t][tid] = c;
+    }
+    __syncthreads();
+    // the halving tree of every target at once
+    for (int lh = 7; lh >= 0; lh--) {
+        const uint32_t h = 1u << lh;
+        for (uint32_t i = tid; i < (uint32_t)tg.count << lh; i += kRT) {
+            const uint32_t t = i >> lh, k = i & (h - 1);
+            double ns, e;
+            two_sum(S[t][k], S[t][k + h], ns, e);
+            C[t][k] = (C[t][k] + C[t][k + h]) + e;
+            S[t][k] = ns;
+        }
+        __syncthreads();
+    }
+    if ((int)tid < tg.count) {
+        const int q = tg.q[tid];
+        double *p = partials + 2 * (uint64_t)tid * nb;
+        if (OBS == 'z' || q < 12 || !((base >> q) & 1)) {
+            p[2 * blk] = S[tid][0];
+            p[2 * blk + 1] = C[tid][0];
+            if (OBS != 'z' && q >= 12) {
+                const uint64_t other = blk | (1ull << (q - 12));
+                p[2 * other] = S[tid][0];
+                p[2 * other + 1] = C[tid][0];
+            }
+        }
+    }
+}
+
+// Block t finishes target t.
+__global__ void __launch_bounds__(kRT)
+k_finish(const double *__restrict__ partials, uint64_t nb, double *__restrict__ out)
+{
+    __shared__ double S[kRT], C[kRT];
+    const double r = reduce_pairs(partials + 2 * (uint64_t)blockIdx.x * nb, nb, S, C);
+    if (threadIdx.x == 0) out[blockIdx.x] = r;
+}
+
+// xr += partner over qubits LO..LO+3 held in registers (bit 1 << k of e).
+template <int BIT>
+__device__ __forceinline__ void reg_sum(const double *a, const double *b, double *xr, double *xi)
+{
+#pragma unroll
+    for (int e = 0; e < kRE; e++) {
+        xr[e] = xr[e] + a[e ^ BIT];
+        xi[e] = xi[e] + b[e ^ BIT];
+    }
+}
+
+// H psi = (sum Z_i Z_{i+1} + hx sum X_i) psi on one block: the X sum of each
+// amplitude runs over the qubits in order; the block's energy terms
+// Re conj(psi_j) (H psi)_j go to its level-1 pair.  STORE keeps H psi, and the
+// terms then use it as stored.
+//
+// Bound: the partner loads of the qubits above the block (one state read each,
+// from L2 where the partner block is in flight on the same XCD, else from the
+// memory-side cache): 11 reads of 134 MB at 23 qubits in 192 us (195 with one
+// thread per term; wavefront, register and loaded partners cost the same
+// there).  With H psi kept, 24 qubits: 464 us for both, where a pass for H psi
+// (504) and one for the energy (99) took 603.
+template <typename T, bool STORE>
+__global__ void __launch_bounds__(kRT) __attribute__((amdgpu_waves_per_eu(3, 3)))
+k_ising(const T *__restrict__ re, const T *__restrict__ im, T *__restrict__ lr,
+        T *__restrict__ li, uint64_t nb, int n, double hx, double *__restrict__ partials)
+{
+    __shared__ double S[kRT], C[kRT];
+    const uint32_t tid = threadIdx.x;
+    const uint64_t blk = xcd_block(blockIdx.x, nb), base = blk * kRB;
+    double a[kRE], b[kRE], xr[kRE], xi[kRE];
+#pragma unroll
+    for (int e = 0; e < kRE; e++) {
+        a[e] = re[base + e * kRT + tid];
+        b[e] = im[base + e * kRT + tid];
+        xr[e] = 0.0;
+        xi[e] = 0.0;
+    }
+    auto far = [&](int q) {
+        const uint64_t p0 = (base + tid) ^ (1ull << q);
+        // a quarter of the block at a time keeps three waves per SIMD
+#pragma unroll
+        for (int h = 0; h < kRE; h += kRE / 4) {
+            T x[kRE / 4], y[kRE / 4];
+#pragma unroll
+            for (int e = 0; e < kRE / 4; e++) {
+                x[e] = re[p0 + (h + e) * kRT];
+                y[e] = im[p0 + (h + e) * kRT];
+            }
+#pragma unroll
+            for (int e = 0; e < kRE / 4; e++) {
+                xr[h + e] = xr[h + e] + (double)x[e];
+                xi[h + e] = xi[h + e] + (double)y[e];
+            }
+        }
+    };
+#pragma unroll 1
+    for (int q = 0; q < 6; q++) {
+#pragma unroll
+        for (int e = 0; e < kRE; e++) {
+            xr[e] = xr[e] + lane_xor(a[e], 1 << q);
+            xi[e] = xi[e] + lane_xor(b[e], 1 << q);
+        }
+    }
+    far(6);
+    far(7);
+    reg_sum<1>(a, b, xr, xi);
+    reg_sum<2>(a, b, xr, xi);
+    reg_sum<4>(a, b, xr, xi);
+    reg_sum<8>(a, b, xr, xi);
+#pragma unroll 1
+    for (int q = 12; q < n; q++) far(q);
+    const uint64_t bonds = (1ull << (n - 1)) - 1;
+    double s = 0.0, c = 0.0;
+#pragma unroll
+    for (int e = 0; e < kRE; e++) {
+        const uint64_t j = base + e * kRT + tid;
+        // aligned bonds count +1, opposed ones -1: an exact integer
+        const int czz = (n - 1) - 2 * __builtin_popcountll((j ^ (j >> 1)) & bonds);
+        double vr = (double)czz * a[e] + hx * xr[e];
+        double vi = (double)czz * b[e] + hx * xi[e];
+        if constexpr (STORE) {
+            lr[j] = (T)vr;
+            li[j] = (T)vi;
+            vr = (double)(T)vr;
+            vi = (double)(T)vi;
+        }
+        add_term(s, c, a[e] * vr + b[e] * vi);
+    }
+    S[tid] = s;
+    C[tid] = c;
+    __syncthreads();
+    tree256(S, C);
+    if (tid == 0) {
+        partials[2 * blk] = S[0];
+        partials[2 * blk + 1] = C[0];
+    }
+}
+
+template <typename T>
+void launch_expect(const spz_state_s *s, char obs, uint64_t nb, const Targets &tg, double *part)
+{
+    const T *re = (const T *)s->re, *im = (const T *)s->im;
+    const dim3 g((unsigned)nb), b(kRT);
+    hipStream_t st = rt().stream;
+    if (obs == 'x')
+        hipLaunchKernelGGL((k_expect<T, 'x'>), g, b, 0, st, re, im, nb, tg, part);
+    else if (obs == 'y')
+        hipLaunchKernelGGL((k_expect<T, 'y'>), g, b, 0, st, re, im, nb, tg, part);
+    else
+        hipLaunchKernelGGL((k_expect<T, 'z'>), g, b, 0, st, re, im, nb, tg, part);
+}
+
+}  // namespace
+
+int reduce_finish(const double *part, uint64_t nb, double *out)
+{
+    hipStream_t st = rt().stream;
+    hipLaunchKernelGGL(k_finish, dim3(1), dim3(kRT), 0, st, part, nb, rt().h_result);
+    SPZ_HIP(hipGetLastError());
+    SPZ_HIP(hipStreamSynchronize(st));
+    *out = rt().h_result[0];
+    return SPZ_OK;
+}
+
+int expect_many(const spz_state_s *s, char observable, const int32_t *targets, uint64_t n_targets,
+                double *out)
+{
+    const uint64_t nb = s->N / kRB;
+    // targets per pass: all kExpectGroup while their pairs take at most 64 MiB
+    const uint64_t room = (64ull << 20) / (16 * nb);
+    const int group = (int)std::max<uint64_t>(1, std::min<uint64_t>(kExpectGroup, room));
+    SPZ_TRY(ensure_partials(nb * std::min<uint64_t>(group, n_targets)));
+    const double bytes = (double)s->N * (s->prec == SPZ_F64 ? 16.0 : 8.0);
+    for (uint64_t r = 0; r < n_targets; r += kResults) {
+        const uint64_t m = std::min<uint64_t>(kResults, n_targets - r);
+        for (uint64_t t = 0; t < m; t += group) {
+            Targets tg;
+            tg.count = (int32_t)std::min<uint64_t>(group, m - t);
+            for (int k = 0; k < tg.count; k++) tg.q[k] = targets[r + t + k];
+            LaunchTimer tm(SPZ_K_REDUCE, bytes);
+            if (s->prec == SPZ_F64) launch_expect<double>(s, observable, nb, tg, rt().d_partials);
+            else launch_expect<float>(s, observable, nb, tg, rt().d_partials);
+            hipLaunchKernelGGL(k_finish, dim3(tg.count), dim3(kRT), 0, rt().stream,
+                               rt().d_partials, nb, rt().h_result + t);
+            SPZ_HIP(hipGetLastError());
+        }
+        SPZ_HIP(hipStreamSynchronize(rt().stream));
+        for (uint64_t t = 0; t < m; t++) out[r + t] = rt().h_result[t];
+    }
+    return SPZ_OK;
+}
+
+int ising_level1(const spz_state_s *s, double hx, void *lr, void *li, double *part)
+{
+    const uint64_t nb = s->N / kRB;
+    const dim3 g((unsigned)nb), b(kRT);
+    hipStream_t st = rt().stream;
+#define SPZ_IS(T, ST)                                                                            \
+    hipLaunchKernelGGL((k_ising<T, ST>), g, b, 0, st, (const T *)s->re, (const T *)s->im, (T *)lr, \
+                       (T *)li, nb, s->n, hx, part)
+    if (s->prec == SPZ_F64) {
+        if (lr) SPZ_IS(double, true);
+        else SPZ_IS(double, false);
+    } else {
+        if (lr) SPZ_IS(float, true);
+        else SPZ_IS(float, false);
+    }
+#undef SPZ_IS
+    SPZ_HIP(hipGetLastError());
+    return SPZ_OK;
+}
+
+}  // namespace spz

@@ -40,16 +40,16 @@ int fail(int code, const std::string &msg);
 // ---------------------------------------------------------------------------
 // Runtime (one device, one stream)
 // ---------------------------------------------------------------------------
+constexpr int kResults = 64;
 struct Runtime {
     bool ready = false;
     int device = 0;
     int cu_count = 0;
     hipStream_t stream = nullptr;
-    // reduction scratch: block partial pairs + final result
+    // reduction scratch: block partial pairs; results land in pinned memory
     double *d_partials = nullptr;
     size_t partial_cap = 0;      // in pairs
-    double *d_result = nullptr;  // 4 doubles
-    double *h_result = nullptr;  // pinned, 4 doubles
+    double *h_result = nullptr;  // pinned, kResults doubles
     // timing
     bool profiling = false;
     struct Pending { int cls; hipEvent_t a, b; double bytes; };

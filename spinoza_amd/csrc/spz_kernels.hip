@@ -15,13 +15,14 @@
 
 #include <type_traits>
 
-#include "spz_internal.h"
+#include "spz_reduce.h"
 
 namespace spz {
 
 namespace {
 
 constexpr int kThreads = 256;
+static_assert(kThreads == kRT, "the reductions share the kernels' block size");
 
 enum Mode { MODE_VEC = 0, MODE_T0 = 1, MODE_SCALAR = 2 };
 
@@ -238,20 +239,8 @@ k_dense(T *__restrict__ re, T *__restrict__ im, uint64_t units, int t, int contr
 }
 
 // ---------------------------------------------------------------------------
-// Fixed-tree compensated reduction (T = 256 threads, E = 16 terms each).
+// Fixed-tree compensated reduction (spz_reduce.h).
 // ---------------------------------------------------------------------------
-constexpr int kRE = 16;
-constexpr uint64_t kRB = (uint64_t)kThreads * kRE;
-
-__device__ __forceinline__ void two_sum(double a, double b, double &s, double &e)
-{
-    double ss = a + b;
-    double bb = ss - a;
-    double aa = ss - bb;
-    e = (a - aa) + (b - bb);
-    s = ss;
-}
-
 template <typename T, typename T2, int TERM>
 __device__ __forceinline__ double term(const T *__restrict__ re, const T *__restrict__ im,
                                        const T2 *__restrict__ re2, const T2 *__restrict__ im2,
@@ -307,20 +296,6 @@ __device__ __forceinline__ double term(const T *__restrict__ re, const T *__rest
     }
 }
 
-__device__ __forceinline__ void tree256(double *S, double *C)
-{
-    const int tid = threadIdx.x;
-    for (int h = kThreads / 2; h >= 1; h >>= 1) {
-        if (tid < h) {
-            double s, e;
-            two_sum(S[tid], S[tid + h], s, e);
-            C[tid] = (C[tid] + C[tid + h]) + e;
-            S[tid] = s;
-        }
-        __syncthreads();
-    }
-}
-
 // T2: storage type of the second state (dot products of an FP32 and an FP64
 // state are summed in FP64 like the rest).
 template <typename T, typename T2, int TERM>
@@ -352,32 +327,6 @@ k_reduce1(const T *__restrict__ re, const T *__restrict__ im, const T2 *__restri
         partials[2 * blockIdx.x] = S[0];
         partials[2 * blockIdx.x + 1] = C[0];
     }
-}
-
-__global__ void __launch_bounds__(kThreads)
-k_reduce2(const double *__restrict__ partials, uint64_t nb, double *__restrict__ out)
-{
-    __shared__ double S[kThreads], C[kThreads];
-    const int tid = threadIdx.x;
-    double s = 0.0, c = 0.0;
-    for (uint64_t j = tid; j < nb; j += kThreads) {
-        double ps = partials[2 * j], pc = partials[2 * j + 1];
-        double ns, e;
-        two_sum(s, ps, ns, e);
-        c = (c + pc) + e;
-        s = ns;
-    }
-    S[tid] = s;
-    C[tid] = c;
-    __syncthreads();
-    tree256(S, C);
-    if (tid == 0) out[0] = S[0] + C[0];
-}
-
-// Single-block finish when there is one level-1 block.
-__global__ void k_finish1(const double *__restrict__ partials, double *__restrict__ out)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) out[0] = partials[0] + partials[1];
 }
 
 // ---------------------------------------------------------------------------
@@ -642,34 +591,30 @@ int reduce(const spz_state_s *a, const spz_state_s *b, int term, int q0, int q1,
            double *out)
 {
     uint64_t nb;
-    SPZ_TRY(reduce_level1(a, b, term, q0, q1, hx, &nb));
-    hipStream_t st = rt().stream;
-    if (nb == 1)
-        hipLaunchKernelGGL(k_finish1, dim3(1), dim3(1), 0, st, rt().d_partials, rt().d_result);
-    else
-        hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kThreads), 0, st, rt().d_partials, nb,
-                           rt().d_result);
-    SPZ_HIP(hipGetLastError());
-    SPZ_HIP(hipMemcpyAsync(rt().h_result, rt().d_result, sizeof(double), hipMemcpyDeviceToHost, st));
-    SPZ_HIP(hipStreamSynchronize(st));
-    *out = rt().h_result[0];
-    return SPZ_OK;
+    if (term == TERM_ISING && a->N >= kRB) {
+        nb = a->N / kRB;
+        SPZ_TRY(ensure_partials(nb));
+        LaunchTimer tm(SPZ_K_REDUCE, (double)a->N * amp_bytes(a));
+        SPZ_TRY(ising_level1(a, hx, nullptr, nullptr, rt().d_partials));
+    } else {
+        SPZ_TRY(reduce_level1(a, b, term, q0, q1, hx, &nb));
+    }
+    return reduce_finish(rt().d_partials, nb, out);
 }
 
 // ---------------------------------------------------------------------------
 // Ising energy without allocation (spz_ising_energy_noalloc)
 // ---------------------------------------------------------------------------
-// The block partials and the result live in a file-scope device array of fixed
+// The block partials live in a file-scope device array of fixed
 // size instead of the grow-only scratch that reduce() allocates: 2^18 blocks
 // of 4096 terms (states up to 2^30 amplitudes, 30 qubits), 4 MiB of partial
-// pairs plus the result.  Host code reaches it only through the address that
+// pairs.  Host code reaches it only through the address that
 // hipGetSymbolAddress returns (the array's name is a host-side stand-in);
 // that address is taken once, when the library initialises on its device.
 // Every call shares the array; the library lock serialises calls within a
 // process, and each call overwrites every pair it reads (no clearing needed).
 constexpr uint64_t kStaticBlocks = 1ull << 18;
-constexpr uint64_t kStaticResult = 2 * kStaticBlocks;  // index of the result slot
-static __device__ __align__(256) double scratch[2 * kStaticBlocks + 32];
+static __device__ __align__(256) double scratch[2 * kStaticBlocks];
 static double *g_static_scratch = nullptr;
 
 int static_scratch_init()
@@ -688,22 +633,15 @@ int ising_energy_noalloc(const spz_state_s *s, double hx, double *out)
     if (nb > kStaticBlocks)
         return fail(SPZ_ERR_ARG, "state too large for spz_ising_energy_noalloc (at most 2^30 "
                                  "amplitudes; use spz_ising_energy)");
-    double *part = g_static_scratch, *res = g_static_scratch + kStaticResult;
-    const int rc = s->prec == SPZ_F64
-                       ? reduce_launch<double>(s, nullptr, TERM_ISING, 0, 0, hx, M, nb, part)
-                       : reduce_launch<float>(s, nullptr, TERM_ISING, 0, 0, hx, M, nb, part);
-    SPZ_TRY(rc);
-    hipStream_t st = rt().stream;
-    if (nb == 1)
-        hipLaunchKernelGGL(k_finish1, dim3(1), dim3(1), 0, st, part, res);
+    double *part = g_static_scratch;
+    if (M >= kRB)
+        SPZ_TRY(ising_level1(s, hx, nullptr, nullptr, part));
     else
-        hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kThreads), 0, st, part, nb, res);
-    SPZ_HIP(hipGetLastError());
-    // the pinned result slot was allocated when the library initialised
-    SPZ_HIP(hipMemcpyAsync(rt().h_result, res, sizeof(double), hipMemcpyDeviceToHost, st));
-    SPZ_HIP(hipStreamSynchronize(st));
-    *out = rt().h_result[0];
-    return SPZ_OK;
+        SPZ_TRY(s->prec == SPZ_F64
+                    ? reduce_launch<double>(s, nullptr, TERM_ISING, 0, 0, hx, M, nb, part)
+                    : reduce_launch<float>(s, nullptr, TERM_ISING, 0, 0, hx, M, nb, part));
+    // the pinned result slots were allocated when the library initialised
+    return reduce_finish(part, nb, out);
 }
 
 // Level-1 pairs of |psi|^2, one per block of 4096 indices, left in

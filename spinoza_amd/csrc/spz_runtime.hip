@@ -5,7 +5,7 @@
 #include <algorithm>
 #include <mutex>
 
-#include "spz_internal.h"
+#include "spz_reduce.h"
 
 namespace spz {
 
@@ -44,8 +44,7 @@ int ensure_init()
     g_rt.cu_count = prop.multiProcessorCount;
     // A default-priority stream; blocking w.r.t. the null stream.
     SPZ_HIP(hipStreamCreate(&g_rt.stream));
-    SPZ_HIP(hipMalloc(&g_rt.d_result, 4 * sizeof(double)));
-    SPZ_HIP(hipHostMalloc(&g_rt.h_result, 4 * sizeof(double), hipHostMallocDefault));
+    SPZ_HIP(hipHostMalloc(&g_rt.h_result, kResults * sizeof(double), hipHostMallocDefault));
     SPZ_TRY(static_scratch_init());
     g_rt.ready = true;
     return SPZ_OK;
@@ -560,11 +559,12 @@ int spz_xyz_expectation_value(spz_state s, char observable, const int32_t *targe
     else if (observable == 'z') term = TERM_Z;
     else return fail(SPZ_ERR_ARG, std::string("observable ") + observable + " not supported");
     if (n_targets && (!targets || !out)) return fail(SPZ_ERR_ARG, "null targets/output");
-    for (uint64_t i = 0; i < n_targets; i++) {
-        int t = targets[i];
-        if (t < 0 || t >= s->n) return fail(SPZ_ERR_QUBIT, "target qubit out of range");
-        SPZ_TRY(reduce(s, nullptr, term, t, 0, 0.0, &out[i]));
-    }
+    for (uint64_t i = 0; i < n_targets; i++)
+        if (targets[i] < 0 || targets[i] >= s->n)
+            return fail(SPZ_ERR_QUBIT, "target qubit out of range");
+    if (s->N >= kRB) return expect_many(s, observable, targets, n_targets, out);
+    for (uint64_t i = 0; i < n_targets; i++)
+        SPZ_TRY(reduce(s, nullptr, term, targets[i], 0, 0.0, &out[i]));
     return SPZ_OK;
 }
 
