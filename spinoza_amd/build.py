@@ -40,6 +40,7 @@ COMMON = [
 # source); the compiler reaches 4 without spills and warns that 6 was not met.
 _TILE_FLAGS = ["-mllvm", "-simplifycfg-sink-common=false", "-Wno-pass-failed"]
 EXTRA = {
+    "spz_adj_tile.hip": _TILE_FLAGS,   # reverse sweeps of the adjoint
     "spz_tile.hip": _TILE_FLAGS,       # exact arithmetic
     "spz_tile_fast.hip": _TILE_FLAGS,  # AUTO arithmetic (compiled in parallel)
 }

@@ -7,13 +7,14 @@
 //   and for P(theta) = diag(1, e^{i theta}), dE/dtheta_k = -2 Im <lambda_k|Pi_1~|psi_k>
 //   (G~, Pi_1~: the operator restricted to amplitudes whose controls are met).
 //
-// Reverse sweep.  Consecutive ops whose targets fit in 3 qubits form a group
-// that costs one pass over psi and lambda: per element (the 8 amplitudes that
-// differ in those qubits) each op adds its gradient term (TwoSum-compensated
-// FP64 per thread, a halving tree per block, one more block over the block
-// partials, written to a device gradient array) and then applies U_k^dag to
-// both states.  Runs of 4 or more parameter-free ops are undone with the
-// fused tile executor, once on psi and once on lambda.
+// Reverse sweep.  States of more than 12 qubits are undone in tile sweeps over
+// psi and lambda together (spz_adj_tile.hip).  Smaller ones fit in the caches
+// and are undone in groups: consecutive ops whose targets fit in 3 qubits cost
+// one launch over psi and lambda, in which each op of an element (the 8
+// amplitudes that differ in those qubits) adds its gradient term
+// (TwoSum-compensated FP64 per thread, a halving tree per block, one more block
+// over the block partials, written to a device gradient array) and then applies
+// U_k^dag to both states.
 #include <math.h>
 #include <string.h>
 
@@ -22,6 +23,7 @@
 #include <mutex>
 #include <vector>
 
+#include "spz_adj_tile.h"
 #include "spz_inplace.h"
 #include "spz_reduce.h"
 #include "spz_tile.h"
@@ -30,6 +32,25 @@ namespace spz {
 
 int execute_ops(spz_state_s *s, const spz_op *ops, uint64_t n_ops, spz_tracker *trk,
                 const spz_exec_opts *opts, uint8_t *outcomes);
+
+static bool has_param(int kind)
+{
+    return kind == SPZ_RX || kind == SPZ_RY || kind == SPZ_RZ || kind == SPZ_P;
+}
+
+// The inverse of one op (gates.rs:78-92): rotations and P negate theta,
+// U(theta, phi, lambda)^-1 = U(-theta, -lambda, -phi), the rest are self-inverse.
+spz_op inverse_op(const spz_op &o)
+{
+    spz_op r = o;
+    if (has_param(o.kind)) r.theta = -o.theta;
+    if (o.kind == SPZ_U) {
+        r.theta = -o.theta;
+        r.phi = -o.lambda;
+        r.lambda = -o.phi;
+    }
+    return r;
+}
 
 namespace {
 
@@ -332,11 +353,6 @@ uint32_t kind_bit_of(int ak)
     }
 }
 
-bool has_param(int kind)
-{
-    return kind == SPZ_RX || kind == SPZ_RY || kind == SPZ_RZ || kind == SPZ_P;
-}
-
 int grad_kind(int kind)
 {
     switch (kind) {
@@ -346,20 +362,6 @@ int grad_kind(int kind)
     case SPZ_P: return GK_P;
     default: return GK_NONE;
     }
-}
-
-// The inverse of one op (gates.rs:78-92): rotations and P negate theta,
-// U(theta, phi, lambda)^-1 = U(-theta, -lambda, -phi), the rest are self-inverse.
-spz_op inverse_op(const spz_op &o)
-{
-    spz_op r = o;
-    if (has_param(o.kind)) r.theta = -o.theta;
-    if (o.kind == SPZ_U) {
-        r.theta = -o.theta;
-        r.phi = -o.lambda;
-        r.lambda = -o.phi;
-    }
-    return r;
 }
 
 int launch_group(spz_state_s *psi, spz_state_s *lam, int nq, uint64_t nel, const PosList &pl,
@@ -383,6 +385,79 @@ int launch_group(spz_state_s *psi, spz_state_s *lam, int nq, uint64_t nel, const
     return SPZ_OK;
 }
 
+// Undo ops[lo_lim, ii) on wk and lm in groups (states of at most kAdjK qubits).
+int undo_groups(spz_state_s *wk, spz_state_s *lm, const spz_op *ops, uint64_t lo_lim, uint64_t ii,
+                double *part, double *gdev)
+{
+    const uint64_t per_block = (uint64_t)kT * kGPerThread;
+    const double amp = wk->prec == SPZ_F64 ? 16.0 : 8.0;
+    while (ii > lo_lim) {
+        const uint64_t hi = ii - 1;
+        const spz_op &o = ops[hi];
+        uint64_t lo = hi;
+        if (o.kind == SPZ_SWAP) {  // self-inverse, no parameter
+            SPZ_TRY(apply_gate(wk, SPZ_SWAP, 0, 0, 0, o.target, o.t1, o.ones, o.zeros));
+            SPZ_TRY(apply_gate(lm, SPZ_SWAP, 0, 0, 0, o.target, o.t1, o.ones, o.zeros));
+            ii = lo;
+            continue;
+        }
+        // greedy group: ops hi, hi-1, ... while the targets fit in kGMaxQ qubits
+        GroupDesc gd;
+        memset(&gd, 0, sizeof gd);
+        GradIdx gi;
+        int nq = 0, ngrad = 0;
+        uint64_t qmask = 0, all_ones = ~0ull, all_zeros = ~0ull;
+        for (uint64_t k = hi + 1; k-- > lo_lim;) {
+            const spz_op &g = ops[k];
+            if (g.kind == SPZ_SWAP || gd.nop == kGMaxOps) break;
+            const uint64_t tb = 1ull << g.target;
+            if (!(qmask & tb)) {
+                if (nq == kGMaxQ) break;
+                gd.q[nq++] = (int8_t)g.target;
+                qmask |= tb;
+            }
+            GroupOp &go = gd.op[gd.nop];
+            const spz_op inv = inverse_op(g);
+            Coef kc;
+            SPZ_TRY(make_coef(inv.kind, inv.theta, inv.phi, inv.lambda, &kc));
+            go.ak = kc.ak;
+            go.kb = kind_bit_of(kc.ak);
+            if (!go.kb) return fail(SPZ_ERR_GATE, "adjoint: unsupported arithmetic");
+            memcpy(go.c, kc.c, sizeof go.c);
+            go.gk = grad_kind(g.kind);
+            for (int b = 0; b < nq; b++)
+                if (gd.q[b] == g.target) go.tq = b;
+            go.cm = g.ones | g.zeros;
+            go.ones = g.ones;
+            all_ones &= g.ones;
+            all_zeros &= g.zeros;
+            gi.i[gd.nop] = go.gk != GK_NONE ? (int64_t)k : -1;
+            ngrad += go.gk != GK_NONE;
+            gd.nop++;
+            lo = k;
+        }
+        // common controls outside Q are fixed positions of every element
+        all_ones &= ~qmask;
+        all_zeros &= ~qmask;
+        gd.base_ones = all_ones;
+        PosList pl;
+        const int np = build_poslist(qmask | all_ones | all_zeros, &pl);
+        const uint64_t nel = wk->N >> np;
+        const unsigned g = blocks_for(nel, per_block);
+        {
+            LaunchTimer tm(SPZ_K_ADJOINT, 2.0 * 2.0 * (double)(nel << nq) * amp);
+            SPZ_TRY(launch_group(wk, lm, nq, nel, pl, gd, part, g));
+        }
+        if (ngrad) {  // one block per op; ops without a gradient write nothing
+            hipLaunchKernelGGL(k_adj_finish, dim3(gd.nop), dim3(kT), 0, rt().stream, part,
+                               (uint64_t)g, gi, gdev);
+            SPZ_HIP(hipGetLastError());
+        }
+        ii = lo;
+    }
+    return SPZ_OK;
+}
+
 // Owns a scratch state; not copyable, so it can live in a vector only
 // behind a unique_ptr (a copy would free the state twice).
 struct OwnedState {
@@ -393,10 +468,33 @@ struct OwnedState {
     ~OwnedState() { if (s) spz_state_destroy(s); }
 };
 
-int make_like(const spz_state_s *s, OwnedState &o)
-{
-    return spz_state_create(s->n, s->prec, &o.s);
-}
+// Checkpoint states kept between calls of one shape (allocating and freeing
+// them costs a device synchronisation each): given back when a call has
+// another shape, and at the end of a call that needs more than kCkptKeep bytes.
+constexpr size_t kCkptKeep = (size_t)4 << 30;
+
+struct CkptPool {
+    std::vector<std::unique_ptr<OwnedState>> st;
+
+    int get(size_t i, const spz_state_s *like, spz_state_s **out)
+    {
+        if (!st.empty() && (st[0]->s->n != like->n || st[0]->s->prec != like->prec)) st.clear();
+        while (st.size() <= i) {
+            auto o = std::make_unique<OwnedState>();
+            SPZ_TRY(spz_state_create(like->n, like->prec, &o->s));
+            st.push_back(std::move(o));
+        }
+        *out = st[i]->s;
+        return SPZ_OK;
+    }
+
+    void trim()
+    {
+        if (st.empty()) return;
+        const size_t each = (size_t)st[0]->s->N * (st[0]->s->prec == SPZ_F64 ? 16 : 8);
+        if (each * st.size() > kCkptKeep) st.clear();
+    }
+};
 
 // Scratch kept between calls (hipFree synchronises the device, and small
 // circuits would otherwise spend most of their time allocating): four
@@ -410,6 +508,7 @@ struct AdjScratch {
     spz_state_s work, lam;  // views into arr
     void *grad = nullptr, *part = nullptr, *dmax = nullptr;
     size_t grad_cap = 0, part_cap = 0;
+    CkptPool ckpts;
 
     int reserve_states(int n, int prec)
     {
@@ -483,6 +582,7 @@ size_t grad_bytes(uint64_t n_ops) { return std::max<uint64_t>(n_ops, 1) * sizeof
 
 size_t part_bytes(uint64_t N)
 {
+    if (N > (1ull << kAdjK)) return adj_part_bytes(N);
     const uint64_t per_block = (uint64_t)kT * kGPerThread;
     return ((N / 2 + per_block - 1) / per_block + 1) * 2 * kGMaxOps * sizeof(double);
 }
@@ -538,173 +638,99 @@ int adjoint_grad(spz_state_s *s, const spz_op *ops, uint64_t n_ops, double hx, i
     if (n_ops && (!ops || !grad)) return fail(SPZ_ERR_ARG, "null ops/grad");
     for (uint64_t i = 0; i < n_ops; i++) SPZ_TRY(validate_adjoint_op(s->n, ops[i], i, true, 64));
     const int n = s->n;
+    AdjScratch &sc = adj_scratch();
+    std::lock_guard<std::mutex> lock(sc.mu);
+    struct Trim {
+        CkptPool &p;
+        ~Trim() { p.trim(); }
+    } trim{sc.ckpts};
     // ---- forward pass with checkpoints ---------------------------------------
-    std::vector<std::unique_ptr<OwnedState>> ckpts;
+    std::vector<spz_state_s *> ckpts;
     std::vector<uint64_t> ckpt_at;  // checkpoint j holds psi after op ckpt_at[j]
     spz_exec_opts eo;
     memset(&eo, 0, sizeof eo);
     eo.mode = SPZ_EXEC_AUTO;
-    if (ckpt_every > 0 && n_ops > 0) {
-        uint64_t done = 0;
-        while (done < n_ops) {
-            uint64_t len = std::min<uint64_t>((uint64_t)ckpt_every, n_ops - done);
-            SPZ_TRY(execute_ops(s, ops + done, len, nullptr, &eo, nullptr));
-            done += len;
-            if (done < n_ops) {
-                ckpts.push_back(std::make_unique<OwnedState>());
-                SPZ_TRY(make_like(s, *ckpts.back()));
-                SPZ_TRY(spz_state_copy(ckpts.back()->s, s));
-                ckpt_at.push_back(done - 1);
-            }
+    const uint64_t step = ckpt_every > 0 ? (uint64_t)ckpt_every : std::max<uint64_t>(n_ops, 1);
+    for (uint64_t done = 0; done < n_ops;) {
+        const uint64_t len = std::min<uint64_t>(step, n_ops - done);
+        SPZ_TRY(execute_ops(s, ops + done, len, nullptr, &eo, nullptr));
+        done += len;
+        if (done < n_ops) {
+            spz_state_s *c = nullptr;
+            SPZ_TRY(sc.ckpts.get(ckpts.size(), s, &c));
+            SPZ_TRY(spz_state_copy(c, s));
+            ckpts.push_back(c);
+            ckpt_at.push_back(done - 1);
         }
-    } else if (n_ops) {
-        SPZ_TRY(execute_ops(s, ops, n_ops, nullptr, &eo, nullptr));
     }
-    // ---- lambda = H psi, energy --------------------------------------------
-    AdjScratch &sc = adj_scratch();
-    std::lock_guard<std::mutex> lock(sc.mu);
+    // ---- lambda = H psi, energy (read with the gradients at the end) ----------
     SPZ_TRY(sc.states_like(s));
+    SPZ_TRY(sc.buffers(grad_bytes(n_ops), part_bytes(s->N)));
     spz_state_s *const wk = &sc.work, *const lm = &sc.lam;  // psi copy, lambda
-    SPZ_TRY(spz_state_copy(wk, s));
-    double e = 0.0;
+    const double amp = s->prec == SPZ_F64 ? 16.0 : 8.0;
+    double *const e_out = rt().h_result + (kResults - 1);
     if (s->N >= kRB) {  // H psi and the energy's first level in one pass
         const uint64_t nb = s->N / kRB;
         SPZ_TRY(ensure_partials(nb));
         {
-            LaunchTimer tm(SPZ_K_ADJOINT, 2.0 * (double)s->N * (s->prec == SPZ_F64 ? 16.0 : 8.0));
+            LaunchTimer tm(SPZ_K_ADJOINT, 2.0 * (double)s->N * amp);
             SPZ_TRY(ising_level1(s, hx, lm->re, lm->im, rt().d_partials));
         }
-        SPZ_TRY(reduce_finish(rt().d_partials, nb, &e));
+        SPZ_TRY(reduce_finish_to(rt().d_partials, nb, e_out));
     } else {
         {
-            LaunchTimer tm(SPZ_K_ADJOINT, (double)s->N * (s->prec == SPZ_F64 ? 16.0 : 8.0) * (n + 2));
+            LaunchTimer tm(SPZ_K_ADJOINT, 2.0 * (double)s->N * amp);
             if (s->prec == SPZ_F64)
-                hipLaunchKernelGGL((k_ising_apply<double>), dim3(blocks_for(s->N, kT)), dim3(kT), 0,
-                                   rt().stream, (const double *)s->re, (const double *)s->im,
+                hipLaunchKernelGGL((k_ising_apply<double>), dim3(blocks_for(s->N, kT)), dim3(kT),
+                                   0, rt().stream, (const double *)s->re, (const double *)s->im,
                                    (double *)lm->re, (double *)lm->im, s->N, n, hx);
             else
-                hipLaunchKernelGGL((k_ising_apply<float>), dim3(blocks_for(s->N, kT)), dim3(kT), 0,
-                                   rt().stream, (const float *)s->re, (const float *)s->im,
+                hipLaunchKernelGGL((k_ising_apply<float>), dim3(blocks_for(s->N, kT)), dim3(kT),
+                                   0, rt().stream, (const float *)s->re, (const float *)s->im,
                                    (float *)lm->re, (float *)lm->im, s->N, n, hx);
             SPZ_HIP(hipGetLastError());
         }
+        double e = 0.0;
         SPZ_TRY(reduce(s, lm, TERM_DOT_RE, 0, 0, 0.0, &e));
+        *e_out = e;
     }
-    if (energy) *energy = e;
     // ---- reverse sweep -------------------------------------------------------
-    const uint64_t per_block = (uint64_t)kT * kGPerThread;
-    SPZ_TRY(sc.buffers(grad_bytes(n_ops), part_bytes(s->N)));
-    SPZ_HIP(hipMemsetAsync(sc.grad, 0, std::max<uint64_t>(n_ops, 1) * sizeof(double), rt().stream));
+    SPZ_HIP(hipMemsetAsync(sc.grad, 0, grad_bytes(n_ops), rt().stream));
     SPZ_HIP(hipMemsetAsync(sc.dmax, 0, sizeof(unsigned long long), rt().stream));
     double *gdev = (double *)sc.grad, *part = (double *)sc.part;
-    void *dmax_p = sc.dmax;
-    const double amp = s->prec == SPZ_F64 ? 16.0 : 8.0;
-    // run_lo[k]: first index of the run of parameter-free ops that ends at k
-    std::vector<uint64_t> run_lo(n_ops);
-    for (uint64_t k = 0; k < n_ops; k++)
-        run_lo[k] = has_param(ops[k].kind) ? k + 1 : (k > 0 && !has_param(ops[k - 1].kind) ? run_lo[k - 1] : k);
-    const bool tiled = n >= 13;  // the fused executor tiles 12 qubits
-    constexpr uint64_t kMinRun = 4;
-    int next_ck = (int)ckpt_at.size() - 1;
-    uint64_t ii = n_ops;  // ops [0, ii) remain
-    while (ii > 0) {
-        const uint64_t hi = ii - 1;
-        // a block of ops must not step over a checkpoint restore point
-        const uint64_t lo_lim = next_ck >= 0 ? ckpt_at[next_ck] + 1 : 0;
-        const spz_op &o = ops[hi];
-        uint64_t lo = hi;
-        if (tiled && !has_param(o.kind) && hi + 1 - std::max(run_lo[hi], lo_lim) >= kMinRun) {
-            lo = std::max(run_lo[hi], lo_lim);
-            std::vector<spz_op> inv;
-            inv.reserve(hi + 1 - lo);
-            for (uint64_t k = hi + 1; k-- > lo;) inv.push_back(inverse_op(ops[k]));
-            SPZ_TRY(execute_ops(wk, inv.data(), inv.size(), nullptr, &eo, nullptr));
-            SPZ_TRY(execute_ops(lm, inv.data(), inv.size(), nullptr, &eo, nullptr));
-        } else if (o.kind == SPZ_SWAP) {  // self-inverse, no parameter
-            SPZ_TRY(apply_gate(wk, SPZ_SWAP, 0, 0, 0, o.target, o.t1, o.ones, o.zeros));
-            SPZ_TRY(apply_gate(lm, SPZ_SWAP, 0, 0, 0, o.target, o.t1, o.ones, o.zeros));
+    const spz_state_s *src = s;  // holds the current psi (wk once anything was undone)
+    for (size_t seg = ckpts.size() + 1; seg-- > 0 && n_ops;) {
+        const uint64_t lo = seg ? ckpt_at[seg - 1] + 1 : 0;
+        const uint64_t hi = seg < ckpts.size() ? ckpt_at[seg] + 1 : n_ops;
+        if (n > kAdjK) {
+            SPZ_TRY(adjoint_undo(src, wk, lm, ops, lo, hi, part, gdev));
         } else {
-            // greedy group: ops hi, hi-1, ... while the targets fit in kGMaxQ qubits
-            GroupDesc gd;
-            memset(&gd, 0, sizeof gd);
-            GradIdx gi;
-            int nq = 0, ngrad = 0;
-            uint64_t qmask = 0, all_ones = ~0ull, all_zeros = ~0ull;
-            for (uint64_t k = hi + 1; k-- > lo_lim;) {
-                const spz_op &g = ops[k];
-                if (g.kind == SPZ_SWAP || gd.nop == kGMaxOps) break;
-                if (k != hi && tiled && !has_param(g.kind) &&
-                    k + 1 - std::max(run_lo[k], lo_lim) >= kMinRun)
-                    break;  // leave a long parameter-free run to the tile executor
-                const uint64_t tb = 1ull << g.target;
-                if (!(qmask & tb)) {
-                    if (nq == kGMaxQ) break;
-                    gd.q[nq++] = (int8_t)g.target;
-                    qmask |= tb;
-                }
-                GroupOp &go = gd.op[gd.nop];
-                double th = g.theta, ph = g.phi, la = g.lambda;
-                if (has_param(g.kind)) th = -th;
-                if (g.kind == SPZ_U) { th = -g.theta; ph = -g.lambda; la = -g.phi; }  // gates.rs:78-92
-                Coef kc;
-                SPZ_TRY(make_coef(g.kind, th, ph, la, &kc));
-                go.ak = kc.ak;
-                go.kb = kind_bit_of(kc.ak);
-                if (!go.kb) return fail(SPZ_ERR_GATE, "adjoint: unsupported arithmetic");
-                memcpy(go.c, kc.c, sizeof go.c);
-                go.gk = grad_kind(g.kind);
-                for (int b = 0; b < nq; b++)
-                    if (gd.q[b] == g.target) go.tq = b;
-                go.cm = g.ones | g.zeros;
-                go.ones = g.ones;
-                all_ones &= g.ones;
-                all_zeros &= g.zeros;
-                gi.i[gd.nop] = go.gk != GK_NONE ? (int64_t)k : -1;
-                ngrad += go.gk != GK_NONE;
-                gd.nop++;
-                lo = k;
-            }
-            // common controls outside Q are fixed positions of every element
-            all_ones &= ~qmask;
-            all_zeros &= ~qmask;
-            gd.base_ones = all_ones;
-            PosList pl;
-            const int np = build_poslist(qmask | all_ones | all_zeros, &pl);
-            const uint64_t nel = s->N >> np;
-            const unsigned g = blocks_for(nel, per_block);
-            {
-                LaunchTimer tm(SPZ_K_ADJOINT, 2.0 * 2.0 * (double)(nel << nq) * amp);
-                SPZ_TRY(launch_group(wk, lm, nq, nel, pl, gd, part, g));
-            }
-            if (ngrad) {  // one block per op; ops without a gradient write nothing
-                hipLaunchKernelGGL(k_adj_finish, dim3(gd.nop), dim3(kT), 0, rt().stream, part,
-                                   (uint64_t)g, gi, gdev);
-                SPZ_HIP(hipGetLastError());
-            }
+            SPZ_TRY(spz_state_copy(wk, const_cast<spz_state_s *>(src)));
+            SPZ_TRY(undo_groups(wk, lm, ops, lo, hi, part, gdev));
         }
-        // work now holds psi_{lo-1}: restore from a checkpoint taken after op lo-1
-        if (next_ck >= 0 && lo >= 1 && ckpt_at[next_ck] == lo - 1) {
-            spz_state_s *ck = ckpts[next_ck]->s;
-            if (s->prec == SPZ_F64)
-                hipLaunchKernelGGL((k_maxdiff<double>), dim3(maxdiff_grid(s->N)), dim3(kT), 0,
-                                   rt().stream, (const double *)wk->re,
-                                   (const double *)wk->im, (const double *)ck->re,
-                                   (const double *)ck->im, s->N, (unsigned long long *)dmax_p);
-            else
-                hipLaunchKernelGGL((k_maxdiff<float>), dim3(maxdiff_grid(s->N)), dim3(kT), 0,
-                                   rt().stream, (const float *)wk->re,
-                                   (const float *)wk->im, (const float *)ck->re,
-                                   (const float *)ck->im, s->N, (unsigned long long *)dmax_p);
-            SPZ_HIP(hipGetLastError());
-            SPZ_TRY(spz_state_copy(wk, ck));
-            next_ck--;
-        }
-        ii = lo;
+        if (!seg) break;
+        // wk holds the uncomputed psi: compare it with the checkpoint, go on from that
+        const spz_state_s *ck = ckpts[seg - 1];
+        if (s->prec == SPZ_F64)
+            hipLaunchKernelGGL((k_maxdiff<double>), dim3(maxdiff_grid(s->N)), dim3(kT), 0,
+                               rt().stream, (const double *)wk->re, (const double *)wk->im,
+                               (const double *)ck->re, (const double *)ck->im, s->N,
+                               (unsigned long long *)sc.dmax);
+        else
+            hipLaunchKernelGGL((k_maxdiff<float>), dim3(maxdiff_grid(s->N)), dim3(kT), 0,
+                               rt().stream, (const float *)wk->re, (const float *)wk->im,
+                               (const float *)ck->re, (const float *)ck->im, s->N,
+                               (unsigned long long *)sc.dmax);
+        SPZ_HIP(hipGetLastError());
+        src = ck;
     }
-    SPZ_HIP(hipMemcpyAsync(grad, gdev, n_ops * sizeof(double), hipMemcpyDeviceToHost, rt().stream));
+    if (n_ops)
+        SPZ_HIP(hipMemcpyAsync(grad, gdev, n_ops * sizeof(double), hipMemcpyDeviceToHost,
+                               rt().stream));
     unsigned long long mx = 0;
-    SPZ_HIP(hipMemcpyAsync(&mx, dmax_p, sizeof mx, hipMemcpyDeviceToHost, rt().stream));
+    SPZ_HIP(hipMemcpyAsync(&mx, sc.dmax, sizeof mx, hipMemcpyDeviceToHost, rt().stream));
     SPZ_HIP(hipStreamSynchronize(rt().stream));
+    if (energy) *energy = *e_out;
     if (drift) {
         double d;
         memcpy(&d, &mx, sizeof d);

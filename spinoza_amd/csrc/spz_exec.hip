@@ -20,6 +20,7 @@
 #include <cmath>
 #include <vector>
 
+#include "spz_adj_tile.h"
 #include "spz_internal.h"
 #include "spz_tile.h"
 
@@ -86,6 +87,7 @@ struct SG {
     bool diag;
     uint64_t nd;  // qubits acted on non-diagonally (the target of a 2x2 gate)
     uint64_t dm;  // qubits acted on diagonally (controls, diagonal targets)
+    int64_t grad; // reverse sweeps: index of its gradient (-1: none)
 };
 
 bool is_barrier(const spz_op &o)
@@ -126,6 +128,7 @@ int lower(const spz_state_s *s, const spz_op &o, const spz_tracker *trk, int idx
     g->diag = is_diagonal(g->k.ak);
     g->nd = g->diag ? 0 : tb;
     g->dm = (ones | zeros) | (g->diag ? tb : 0);
+    g->grad = -1;
     return SPZ_OK;
 }
 
@@ -140,6 +143,8 @@ struct Sweep {
     int gate;                  // plain: index into the run
     TileDesc desc;
     size_t op_begin, op_count; // range in the program buffer
+    size_t slot_begin;         // reverse sweeps: range in the list of gradients
+    int slots;
     // fast sweeps: the frame a next tile sweep can take over (Z part and
     // phase; the X part is always applied at the store)
     bool can_carry;
@@ -387,6 +392,10 @@ struct Planner {
     bool fast = false;   // AUTO arithmetic (see launch_tile): H factors carried
     bool swaps = false;  // in-wavefront layout changes when they reach the set
     bool bad = false;
+    // Reverse sweeps of the adjoint: every gate runs in a sweep (a single one
+    // too), and a sweep takes at most max_grads gates with a gradient.
+    int max_grads = 0;
+    std::vector<uint32_t> grads;  // the sweeps' gradients, slot by slot
     uint64_t frame_gates = 0;  // gates absorbed into Pauli frames
     uint64_t split_ops = 0;    // second halves of gates run as two half-angle ops
     std::vector<TileOp> prog;
@@ -926,6 +935,7 @@ struct Planner {
             }
         for (; i < 16; i++) sw.desc.spos[i] = 64;
         sw.op_begin = prog.size();
+        sw.slot_begin = grads.size();
         std::vector<int> seq, RS, THR;
         std::vector<Change> changes;
         sequence(run, order, lbit, seq, changes, RS, THR);
@@ -1114,6 +1124,10 @@ struct Planner {
                     op.sel = 1u << slot;
                     op.grp |= pred ? TG_PAIRP : TG_PAIR;
                 }
+                if (g.grad >= 0) {
+                    grads.push_back((uint32_t)g.grad);
+                    op.pad = (uint32_t)(grads.size() - sw.slot_begin);
+                }
                 prog.push_back(op);
             }
             if (zafter) fr.z ^= tb;  // (on phi: the frame takes it on its right)
@@ -1204,6 +1218,7 @@ struct Planner {
             sw.carry_w = (fr.w + 2 * __builtin_popcountll(fr.x & fr.z)) & 3;
         }
         sw.op_count = prog.size() - sw.op_begin;
+        sw.slots = (int)(grads.size() - sw.slot_begin);
         sw.desc.nops = (int32_t)sw.op_count;
         sweeps.push_back(sw);
     }
@@ -1216,7 +1231,13 @@ struct Planner {
             uint64_t smask;
             std::vector<int> order = collect(run, rem, smask);
             if (order.size() >= 2) endgame(run, rem, smask, order);
-            if (order.size() < 2) {
+            if (max_grads) {  // a prefix of the order is a valid sweep
+                int left = max_grads;
+                size_t keep = 0;
+                while (keep < order.size() && (run[order[keep]].grad < 0 || left-- > 0)) keep++;
+                order.resize(keep);
+            }
+            if (order.size() < 2 && !max_grads) {
                 // nothing to fuse: the first remaining gate runs on the plain path
                 Sweep sw;
                 memset(&sw, 0, sizeof sw);
@@ -1239,9 +1260,9 @@ struct Planner {
 // whose sweeps have not finished: execute calls return without a device
 // synchronisation, in stream order like every other entry point.
 struct ProgSlot {
-    TileOp *host = nullptr;
-    TileOp *dev = nullptr;
-    size_t cap = 0;
+    char *host = nullptr;
+    char *dev = nullptr;
+    size_t cap = 0;  // bytes
     hipEvent_t done = nullptr;
     bool pending = false;
 };
@@ -1249,7 +1270,9 @@ ProgSlot g_slots[2];
 int g_slot_next = 0;
 std::mutex g_slot_mu;
 
-int upload_program(const std::vector<TileOp> &prog, ProgSlot **out)
+// The program, and after it a list of 32-bit indices, into the next slot.
+int upload_program(const std::vector<TileOp> &prog, const std::vector<uint32_t> &idx,
+                   ProgSlot **out)
 {
     ProgSlot &sl = g_slots[g_slot_next];
     g_slot_next ^= 1;
@@ -1258,24 +1281,38 @@ int upload_program(const std::vector<TileOp> &prog, ProgSlot **out)
         sl.pending = false;
     }
     if (!sl.done) SPZ_HIP(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));
-    if (prog.size() > sl.cap) {
+    const size_t pb = prog.size() * sizeof(TileOp), ib = idx.size() * sizeof(uint32_t);
+    if (pb + ib > sl.cap) {
         if (sl.dev) SPZ_HIP(hipFree(sl.dev));
         if (sl.host) SPZ_HIP(hipHostFree(sl.host));
         sl.dev = nullptr;
         sl.host = nullptr;
         sl.cap = 0;
-        const size_t cap = std::max(prog.size(), (size_t)4096);
-        if (hipMalloc(&sl.dev, cap * sizeof(TileOp)) != hipSuccess ||
-            hipHostMalloc(&sl.host, cap * sizeof(TileOp), hipHostMallocDefault) != hipSuccess)
+        const size_t cap = std::max(pb + ib, 4096 * sizeof(TileOp));
+        if (hipMalloc(&sl.dev, cap) != hipSuccess ||
+            hipHostMalloc(&sl.host, cap, hipHostMallocDefault) != hipSuccess)
             return fail(SPZ_ERR_OOM, "tile program allocation failed");
         sl.cap = cap;
     }
-    memcpy(sl.host, prog.data(), prog.size() * sizeof(TileOp));
-    SPZ_HIP(hipMemcpyAsync(sl.dev, sl.host, prog.size() * sizeof(TileOp), hipMemcpyHostToDevice,
-                           rt().stream));
+    memcpy(sl.host, prog.data(), pb);
+    if (ib) memcpy(sl.host + pb, idx.data(), ib);
+    SPZ_HIP(hipMemcpyAsync(sl.dev, sl.host, pb + ib, hipMemcpyHostToDevice, rt().stream));
     *out = &sl;
     return SPZ_OK;
 }
+
+// Marks a slot busy until the stream passes the point where it goes out of
+// scope, on every exit after the upload (an error return included, with the
+// copy in flight).
+struct Release {
+    ProgSlot *sl;
+    ~Release()
+    {
+        if (!sl) return;
+        if (hipEventRecord(sl->done, rt().stream) == hipSuccess) sl->pending = true;
+        else (void)hipStreamSynchronize(rt().stream);
+    }
+};
 
 int run_fused(spz_state_s *s, const std::vector<SG> &run, int K, bool strict)
 {
@@ -1328,19 +1365,9 @@ int run_fused(spz_state_s *s, const std::vector<SG> &run, int K, bool strict)
     }
     std::lock_guard<std::mutex> lk(g_slot_mu);
     ProgSlot *slot = nullptr;
-    if (!pl.prog.empty()) SPZ_TRY(upload_program(pl.prog, &slot));
-    const TileOp *d_prog = slot ? slot->dev : nullptr;
-    // on every exit after the upload: mark the slot busy until the stream
-    // passes this point (an error return included, with the copy in flight)
-    struct Release {
-        ProgSlot *sl;
-        ~Release()
-        {
-            if (!sl) return;
-            if (hipEventRecord(sl->done, rt().stream) == hipSuccess) sl->pending = true;
-            else (void)hipStreamSynchronize(rt().stream);
-        }
-    } release{slot};
+    if (!pl.prog.empty()) SPZ_TRY(upload_program(pl.prog, {}, &slot));
+    const TileOp *d_prog = slot ? (const TileOp *)slot->dev : nullptr;
+    Release release{slot};
     for (const Sweep &sw : pl.sweeps) {
         if (sw.tile) {
             SPZ_TRY(launch_tile(s, K, sw.desc, d_prog + sw.op_begin, pl.fast));
@@ -1506,6 +1533,65 @@ int run_dense5(spz_state_s *s, const std::vector<SG> &run)
 }
 
 }  // namespace
+
+// (spz_adj_tile.h)
+int adjoint_undo(const spz_state_s *src, spz_state_s *psi, spz_state_s *lam, const spz_op *ops,
+                 uint64_t lo, uint64_t hi, double *part, double *grad)
+{
+    std::vector<SG> run;
+    run.reserve(hi - lo);
+    auto add = [&](const spz_op &o, int64_t slot) -> int {
+        SG g;
+        SPZ_TRY(lower(psi, o, nullptr, (int)run.size(), &g));
+        g.grad = slot;
+        run.push_back(g);
+        return SPZ_OK;
+    };
+    for (uint64_t k = hi; k-- > lo;) {
+        const spz_op o = inverse_op(ops[k]);
+        if (o.kind == SPZ_SWAP) {  // three CX, the middle one with the SWAP's controls
+            spz_op x;
+            memset(&x, 0, sizeof x);
+            x.kind = SPZ_X;
+            x.target = o.target;
+            x.ones = 1ull << o.t1;
+            spz_op y = x;
+            y.target = o.t1;
+            y.ones = o.ones | (1ull << o.target);
+            y.zeros = o.zeros;
+            SPZ_TRY(add(x, -1));
+            SPZ_TRY(add(y, -1));
+            SPZ_TRY(add(x, -1));
+            continue;
+        }
+        const bool par = o.kind == SPZ_RX || o.kind == SPZ_RY || o.kind == SPZ_RZ || o.kind == SPZ_P;
+        SPZ_TRY(add(o, par ? (int64_t)k : -1));
+    }
+    Planner pl;
+    pl.n = psi->n;
+    pl.K = kAdjK;
+    pl.LOGW = kAdjK - 4;
+    pl.RB = 4;
+    pl.klo = std::min(env_int("SPZ_TILE_KLO", 4), kAdjK);
+    pl.improve = env_int("SPZ_TILE_SEARCH", 16);
+    pl.strict = false;
+    pl.max_grads = kAdjSlots;
+    pl.plan(run);
+    if (pl.bad) return fail(SPZ_ERR_ARG, "tile planner produced a gate outside the register layout");
+    std::lock_guard<std::mutex> lk(g_slot_mu);
+    ProgSlot *slot = nullptr;
+    SPZ_TRY(upload_program(pl.prog, pl.grads, &slot));
+    Release release{slot};
+    const TileOp *d_prog = (const TileOp *)slot->dev;
+    const uint32_t *d_idx = (const uint32_t *)(slot->dev + pl.prog.size() * sizeof(TileOp));
+    const uint64_t tiles = psi->N >> kAdjK;
+    for (const Sweep &sw : pl.sweeps) {
+        SPZ_TRY(launch_adj_tile(src, psi, lam, sw.desc, d_prog + sw.op_begin, sw.slots, part));
+        SPZ_TRY(launch_adj_sum(part, tiles, d_idx + sw.slot_begin, sw.slots, grad));
+        src = psi;
+    }
+    return SPZ_OK;
+}
 
 int execute_plain(spz_state_s *s, const spz_op *ops, uint64_t n_ops, spz_tracker *trk,
                   uint8_t *outcomes)

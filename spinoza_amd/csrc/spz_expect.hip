@@ -282,12 +282,17 @@ void launch_expect(const spz_state_s *s, char obs, uint64_t nb, const Targets &t
 
 }  // namespace
 
+int reduce_finish_to(const double *part, uint64_t nb, double *pinned)
+{
+    hipLaunchKernelGGL(k_finish, dim3(1), dim3(kRT), 0, rt().stream, part, nb, pinned);
+    SPZ_HIP(hipGetLastError());
+    return SPZ_OK;
+}
+
 int reduce_finish(const double *part, uint64_t nb, double *out)
 {
-    hipStream_t st = rt().stream;
-    hipLaunchKernelGGL(k_finish, dim3(1), dim3(kRT), 0, st, part, nb, rt().h_result);
-    SPZ_HIP(hipGetLastError());
-    SPZ_HIP(hipStreamSynchronize(st));
+    SPZ_TRY(reduce_finish_to(part, nb, rt().h_result));
+    SPZ_HIP(hipStreamSynchronize(rt().stream));
     *out = rt().h_result[0];
     return SPZ_OK;
 }

@@ -90,7 +90,9 @@ int expect_many(const spz_state_s *s, char observable, const int32_t *targets, u
 // Level-1 pairs of the Ising energy into `part` and, with lr and li, the
 // amplitudes of H psi (states of at least 4096 amplitudes).
 int ising_level1(const spz_state_s *s, double hx, void *lr, void *li, double *part);
-// Second level over `nb` pairs into *out (waits for the result).
+// Second level over `nb` pairs into *out (waits for the result), or into a
+// pinned slot of rt().h_result without a wait.
 int reduce_finish(const double *part, uint64_t nb, double *out);
+int reduce_finish_to(const double *part, uint64_t nb, double *pinned);
 
 }  // namespace spz
