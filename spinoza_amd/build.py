@@ -1,4 +1,5 @@
-"""Build the gfx950 shared library ``spinoza_amd/libspinoza_amd.so`` in-tree.
+"""Build the gfx950 shared library ``spinoza_amd/libspinoza_amd.so`` and the
+CPython extension ``spinoza_amd/_encode.so`` (op dicts to C records) in-tree.
 
 Every ``csrc/*.hip`` file is compiled by hipcc for gfx950 only, then linked
 into one shared library exporting the C ABI of ``include/spinoza_amd.h``.
@@ -14,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -63,6 +65,20 @@ def sources():
 HOST = ["-O2", "-fPIC", "-std=c++17", "-Wall", "-I", os.path.join(ROOT, "include")]
 
 
+def _build_extension():
+    """The op encoder, a small C extension of the running interpreter."""
+    out = os.path.join(HERE, "_encode.so")
+    cmd = [os.environ.get("CC", "gcc"), "-O2", "-fPIC", "-shared", "-Wall", "-Wextra",
+           "-Wno-missing-field-initializers", "-I", sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "py", "encode.c"), "-o", out + ".tmp"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"compiling the op encoder failed:\n{r.stdout}\n{r.stderr}")
+    if r.stderr.strip():
+        sys.stderr.write(r.stderr)
+    os.replace(out + ".tmp", out)
+
+
 def _compile(src):
     obj = os.path.join(BUILD, os.path.basename(src) + ".o")
     if src.endswith(".cpp"):
@@ -93,6 +109,7 @@ def build(verbose=False, incremental=False):
     """Compile every source (or, with incremental=True, only those whose
     object is out of date) and link the library."""
     os.makedirs(BUILD, exist_ok=True)
+    _build_extension()
     srcs = sources()
     todo = [s for s in srcs if _stale(s)] if incremental else srcs
     with concurrent.futures.ThreadPoolExecutor(max_workers=max(1, min(8, len(todo)))) as ex:

@@ -401,6 +401,12 @@ struct Planner {
     std::vector<TileOp> prog;
     std::vector<Sweep> sweeps;
 
+    // What the searches read of a gate, packed (a run's SG records are an order
+    // of magnitude larger, and the searches pass over them thousands of times).
+    struct Acts {
+        uint64_t nd, dm;
+    };
+
     // A gate that a fast sweep absorbs into its frame needs no register slot.
     bool absorbed(const SG &g) const
     {
@@ -448,16 +454,16 @@ struct Planner {
     // Gates of `rem` that one sweep over the fixed tile set `smask` can take
     // (program order, skipping past blocked gates); stops once every tile
     // qubit is blocked.  With `out`, also lists them.
-    size_t take_fixed(const std::vector<SG> &run, const std::vector<int> &rem, uint64_t smask,
-                      std::vector<int> *out) const
+    static size_t take_fixed(const std::vector<Acts> &acts, const std::vector<int> &rem,
+                             uint64_t smask, std::vector<int> *out)
     {
         uint64_t bnd = 0, bd = 0;
         size_t cnt = 0;
-        for (int idx : rem) {
-            const SG &g = run[idx];
+        for (size_t i = 0; i < rem.size(); i++) {
+            const Acts &g = acts[i];
             if (!(g.nd & (bnd | bd)) && !(g.dm & bnd) && !(g.nd & ~smask)) {
                 cnt++;
-                if (out) out->push_back(idx);
+                if (out) out->push_back(rem[i]);
             } else {
                 bnd |= g.nd;
                 bd |= g.dm;
@@ -465,6 +471,13 @@ struct Planner {
             }
         }
         return cnt;
+    }
+
+    static std::vector<Acts> acts_of(const std::vector<SG> &run, const std::vector<int> &rem)
+    {
+        std::vector<Acts> acts(rem.size());
+        for (size_t i = 0; i < rem.size(); i++) acts[i] = {run[rem[i]].nd, run[rem[i]].dm};
+        return acts;
     }
 
     // Local search over the tile set: swap a free tile qubit for a qubit that
@@ -481,6 +494,7 @@ struct Planner {
             if (++seen >= 4 * (size_t)n * 8) break;
         }
         cand &= ~fixed;
+        const std::vector<Acts> acts = acts_of(run, rem);
         size_t best = order.size();
         bool moved = false;
         for (int pass = 0; pass < improve; pass++) {
@@ -490,7 +504,7 @@ struct Planner {
                 for (int b = 0; b < n && !better; b++) {
                     if (((smask >> b) & 1) || !((cand >> b) & 1)) continue;
                     const uint64_t m2 = (smask & ~(1ull << a)) | (1ull << b);
-                    const size_t c2 = take_fixed(run, rem, m2, nullptr);
+                    const size_t c2 = take_fixed(acts, rem, m2, nullptr);
                     if (c2 > best) {
                         best = c2;
                         smask = m2;
@@ -502,7 +516,7 @@ struct Planner {
         }
         if (moved) {
             order.clear();
-            take_fixed(run, rem, smask, &order);
+            take_fixed(acts, rem, smask, &order);
         }
     }
 
@@ -556,6 +570,7 @@ struct Planner {
         uint64_t cand = 0;
         for (int idx : rem) cand |= run[idx].nd;
         cand &= ~fixed;
+        const std::vector<Acts> acts = acts_of(run, rem);
         double best = base;
         uint64_t bm = smask;
         std::vector<int> bo;
@@ -565,7 +580,7 @@ struct Planner {
                 if (((smask >> b) & 1) || !((cand >> b) & 1)) continue;
                 const uint64_t m2 = (smask & ~(1ull << a)) | (1ull << b);
                 std::vector<int> o2;
-                take_fixed(run, rem, m2, &o2);
+                take_fixed(acts, rem, m2, &o2);
                 if (o2.size() < 2) continue;
                 const double c = tail_cost(run, minus(rem, o2));
                 if (c < best) {
@@ -669,48 +684,49 @@ struct Planner {
         for (auto [j, tb] : sw) std::swap(rs[j], thr[tb]);
     }
 
-    // Dependency graph of a sweep's gates: a -> b (a before b) when they share
-    // a qubit on which at least one acts non-diagonally.
-    void deps_of(const std::vector<SG> &run, const std::vector<int> &order,
-                 std::vector<std::vector<int>> &succ, std::vector<int> &indeg) const
-    {
-        const int m = (int)order.size();
-        succ.assign(m, {});
-        indeg.assign(m, 0);
-        for (int a = 0; a < m; a++) {
-            const SG &x = run[order[a]];
-            for (int b = a + 1; b < m; b++) {
-                const SG &y = run[order[b]];
-                if ((x.nd & (y.nd | y.dm)) || (x.dm & y.nd)) {
-                    succ[a].push_back(b);
-                    indeg[b]++;
-                }
-            }
-        }
-    }
+    // A gate still to run in the sweep: what it acts on, and the local bit that
+    // must be in a register for it (0: none).  Gates keep their program order,
+    // so one forward pass with masks of what the passed-over gates act on
+    // decides everything a dependency graph would: a gate waits for an earlier
+    // one when they share a qubit on which at least one acts non-diagonally.
+    struct Todo {
+        uint64_t nd, dm;
+        uint32_t need;
+        int at;  // index into `order`
+    };
 
-    // Gates that run, in dependency order, under register bits rs before a
-    // pair gate on another bit blocks every remaining one.
-    int runs_under(const std::vector<SG> &run, const std::vector<int> &order, const int *lbit,
-                   const std::vector<std::vector<int>> &succ, std::vector<int> indeg,
-                   std::vector<char> done, uint32_t rs) const
+    // Gates that run under register bits rs before the others are stuck (or
+    // fewer, once it is certain that they are fewer than `least`).  `all`: the
+    // qubits the gates act on.
+    static int runs_under(const std::vector<Todo> &todo, uint32_t rs, uint64_t all, int least)
     {
-        const int m = (int)order.size();
-        int cnt = 0;
-        bool progress = true;
-        while (progress) {
-            progress = false;
-            for (int a = 0; a < m; a++) {
-                if (done[a] || indeg[a]) continue;
-                const SG &g = run[order[a]];
-                if (needs_reg(g) && !((rs >> lbit[g.target]) & 1)) continue;
-                done[a] = 1;
+        uint64_t bnd = 0, bd = 0;
+        int cnt = 0, spare = (int)todo.size() - least;
+        for (const Todo &g : todo) {
+            if (!(g.nd & (bnd | bd)) && !(g.dm & bnd) && !(g.need & ~rs)) {
                 cnt++;
-                for (int b : succ[a]) indeg[b]--;
-                progress = true;
+            } else {
+                bnd |= g.nd;
+                bd |= g.dm;
+                if (--spare < 0 || bnd == all) break;
             }
         }
         return cnt;
+    }
+
+    // Register targets still to run, weighted by readiness.
+    void pair_score(const std::vector<Todo> &todo, std::vector<long> &score) const
+    {
+        score.assign(K, 0);
+        uint64_t bnd = 0, bd = 0;
+        for (const Todo &g : todo) {
+            if (g.need) {
+                const bool ready = !(g.nd & (bnd | bd)) && !(g.dm & bnd);
+                score[__builtin_ctz(g.need)] += ready ? 1000 : 1;
+            }
+            bnd |= g.nd;
+            bd |= g.dm;
+        }
     }
 
     // The RB register bits (from `lo` up) to switch to: every RB-subset of
@@ -720,15 +736,11 @@ struct Planner {
     // swaps is charged less than one that needs an LDS transpose (in gates
     // that could have run: a transpose costs about four gates, a swap about
     // half of one).
-    std::vector<int> best_set(const std::vector<SG> &run, const std::vector<int> &order,
-                              const int *lbit, const std::vector<std::vector<int>> &succ,
-                              const std::vector<int> &indeg, const std::vector<char> &done,
-                              const std::vector<long> &score, int lo,
+    std::vector<int> best_set(const std::vector<Todo> &todo, const std::vector<long> &score, int lo,
                               const std::vector<int> *cur_rs = nullptr,
                               const std::vector<int> *cur_thr = nullptr) const
     {
-        int left = 0;
-        for (char d : done) left += !d;
+        const int left = (int)todo.size();
         std::vector<int> bits;
         for (int b = lo; b < K; b++) bits.push_back(b);
         std::stable_sort(bits.begin(), bits.end(),
@@ -737,18 +749,23 @@ struct Planner {
         uint32_t best = 0;
         double best_val = -1e30;
         long best_sc = -1;
+        uint64_t all = 0;
+        for (const Todo &g : todo) all |= g.nd | g.dm;
+        std::vector<int> want;
+        std::vector<std::pair<int, int>> sw;
         for (uint32_t sub = 0; sub < (1u << T); sub++) {
             if (__builtin_popcount(sub) != RB) continue;
             uint32_t rs = 0;
             long sc = 0;
-            std::vector<int> want;
             for (int i = 0; i < T; i++)
                 if ((sub >> i) & 1) {
                     rs |= 1u << bits[i];
                     sc += score[bits[i]];
-                    want.push_back(bits[i]);
                 }
-            int cnt = runs_under(run, order, lbit, succ, indeg, done, rs);
+            // (a count whose value would stay below best_val cannot win: at
+            // most 1 is added to it, and without swaps 4 are taken off)
+            int cnt = runs_under(todo, rs, all,
+                                 (int)std::max(0.0, best_val + (cur_rs && !swaps ? 3.0 : -1.0)));
             // a set that finishes the sweep and keeps the low bits on lanes
             // saves the change back before the store
             if (cnt == left && !(rs & ((1u << klo) - 1))) cnt++;
@@ -756,8 +773,15 @@ struct Planner {
             if (cnt == 0) continue;
             double val = cnt;
             if (cur_rs && cur_thr) {
-                std::vector<std::pair<int, int>> sw;
-                val -= swap_path(*cur_rs, *cur_thr, want, &sw) ? 0.5 * (double)sw.size() : 4.0;
+                bool swap = false;
+                if (swaps) {
+                    want.clear();
+                    sw.clear();
+                    for (int i = 0; i < T; i++)
+                        if ((sub >> i) & 1) want.push_back(bits[i]);
+                    swap = swap_path(*cur_rs, *cur_thr, want, &sw);
+                }
+                val -= swap ? 0.5 * (double)sw.size() : 4.0;
             }
             if (val > best_val || (val == best_val && sc > best_sc)) {
                 best = rs;
@@ -800,22 +824,14 @@ struct Planner {
                 if (RS[j] == b) return true;
             return false;
         };
-        // pair-gate targets still to run, weighted by readiness
-        auto pair_score = [&](const std::vector<int> &indeg, const std::vector<char> *done) {
-            std::vector<long> score(K, 0);
-            for (int a = 0; a < m; a++) {
-                if (done && (*done)[a]) continue;
-                const SG &g = run[order[a]];
-                if (needs_reg(g)) score[lbit[g.target]] += indeg[a] == 0 ? 1000 : 1;
-            }
-            return score;
-        };
-        std::vector<std::vector<int>> succ0;
-        std::vector<int> indeg0;
-        deps_of(run, order, succ0, indeg0);
-        std::vector<long> score0 = pair_score(indeg0, nullptr);
-        if (!strict && K - klo >= RB)
-            RS = best_set(run, order, lbit, succ0, indeg0, std::vector<char>(m, 0), score0, klo);
+        std::vector<Todo> todo(m);
+        for (int a = 0; a < m; a++) {
+            const SG &g = run[order[a]];
+            todo[a] = {g.nd, g.dm, needs_reg(g) ? 1u << lbit[g.target] : 0u, a};
+        }
+        std::vector<long> score0;
+        pair_score(todo, score0);
+        if (!strict && K - klo >= RB) RS = best_set(todo, score0, klo);
         std::vector<int> THR = thread_layout(RS, &score0, klo);
         rs_in = RS;
         thr_in = THR;
@@ -882,32 +898,31 @@ struct Planner {
             }
             return;
         }
-        std::vector<std::vector<int>> &succ = succ0;
-        std::vector<int> &indeg = indeg0;
-        std::vector<char> done(m, 0);
-        int left = m;
-        while (left > 0) {
-            bool progress = true;
-            while (progress) {
-                progress = false;
-                for (int a = 0; a < m; a++) {
-                    if (done[a] || indeg[a]) continue;
-                    const SG &g = run[order[a]];
-                    if (needs_reg(g) && !in_rs(lbit[g.target])) continue;
-                    seq.push_back(order[a]);
-                    done[a] = 1;
-                    left--;
-                    for (int b : succ[a]) indeg[b]--;
-                    progress = true;
+        std::vector<Todo> stuck;
+        std::vector<long> score;
+        for (;;) {
+            // every gate that runs under the current register bits, in order
+            uint32_t rs = 0;
+            for (int j = 0; j < RB; j++) rs |= 1u << RS[j];
+            uint64_t bnd = 0, bd = 0;
+            stuck.clear();
+            for (const Todo &g : todo) {
+                if (!(g.nd & (bnd | bd)) && !(g.dm & bnd) && !(g.need & ~rs)) {
+                    seq.push_back(order[g.at]);
+                } else {
+                    stuck.push_back(g);
+                    bnd |= g.nd;
+                    bd |= g.dm;
                 }
             }
-            if (left == 0) break;
+            todo.swap(stuck);
+            if (todo.empty()) break;
             // next layout: score target bits of the remaining non-diagonal
             // gates, ready ones first; among the RB-subsets of the best
             // scored bits, take the one under which the most gates run
             // before the next change, less the cost of reaching it
-            std::vector<long> score = pair_score(indeg, &done);
-            std::vector<int> nx = best_set(run, order, lbit, succ, indeg, done, score, 0, &RS, &THR);
+            pair_score(todo, score);
+            std::vector<int> nx = best_set(todo, score, 0, &RS, &THR);
             change_to(nx, score);
             if ((int)changes.size() > 2 * m + 8) {  // every change runs a gate: cannot happen
                 bad = true;
@@ -1068,9 +1083,9 @@ struct Planner {
                     return -1;
                 };
                 uint32_t mro = 0, mrz = 0;  // controls on register-index bits (read 1 / 0)
-                for (int q = 0; q < n; q++) {
-                    const bool one = (g.ones >> q) & 1, zero = (g.zeros >> q) & 1;
-                    if (!one && !zero) continue;
+                for (uint64_t ctl = g.ones | g.zeros; ctl; ctl &= ctl - 1) {
+                    const int q = __builtin_ctzll(ctl);
+                    const bool one = (g.ones >> q) & 1;
                     const int b = lbit[q];
                     if (b < 0) {
                         if (one) op.eo |= 1ull << q;

@@ -8,33 +8,24 @@ import ctypes
 
 import numpy as np
 
+from . import _encode
 from . import _native as N
 
 
 def encode_ops(ops):
+    if not isinstance(ops, (list, tuple)):
+        ops = list(ops)
     n = len(ops)
     arr = (N.Op_t * max(n, 1))()
     keep = []
-    for i, d in enumerate(ops):
-        o = arr[i]
-        o.kind = int(d["kind"])
-        o.target = int(d.get("target", 0))
-        o.theta = float(d.get("theta", 0.0))
-        o.phi = float(d.get("phi", 0.0))
-        o.lam = float(d.get("lam", 0.0))
-        o.t1 = int(d.get("t1", 0))
-        o.flags = N.OPF_CLASSICAL if d.get("classical") else 0
-        o.ones = int(d.get("ones", 0))
-        o.zeros = int(d.get("zeros", 0))
-        o.u = float(d.get("u", 1.0))
-        if "matrix" in d:
-            u = np.asarray(d["matrix"], dtype=complex)
-            re = np.ascontiguousarray(u.real)
-            im = np.ascontiguousarray(u.imag)
-            keep += [re, im]
-            o.m = int(u.shape[0]).bit_length() - 1
-            o.u_re = re.ctypes.data
-            o.u_im = im.ctypes.data
+    for i in _encode.fill(ops, arr):
+        u = np.asarray(ops[i]["matrix"], dtype=complex)
+        re = np.ascontiguousarray(u.real)
+        im = np.ascontiguousarray(u.imag)
+        keep += [re, im]
+        arr[i].m = int(u.shape[0]).bit_length() - 1
+        arr[i].u_re = re.ctypes.data
+        arr[i].u_im = im.ctypes.data
     return arr, keep
 
 
@@ -51,7 +42,7 @@ def run_ops(state, ops, mode=N.EXEC_AUTO, tracker=None, tile_qubits=0, encoded=N
     N.check(N.lib().spz_execute(state._h, arr, n, ctypes.byref(tr), ctypes.byref(opts),
                                 outcomes))
     del keep
-    return [int(outcomes[i]) for i in range(n)]
+    return outcomes[:n]
 
 
 def plan_stats(n, ops, mode=N.EXEC_AUTO, tile_qubits=0, precision="f64"):
