@@ -43,6 +43,7 @@ COMMON = [
 _TILE_FLAGS = ["-mllvm", "-simplifycfg-sink-common=false", "-Wno-pass-failed"]
 EXTRA = {
     "spz_adj_tile.hip": _TILE_FLAGS,   # reverse sweeps of the adjoint
+    "spz_chip.hip": _TILE_FLAGS,       # sweeps of many or small circuits
     "spz_tile.hip": _TILE_FLAGS,       # exact arithmetic
     "spz_tile_fast.hip": _TILE_FLAGS,  # AUTO arithmetic (compiled in parallel)
 }

@@ -20,10 +20,11 @@ int launch_adj_tile(const spz_state_s *src, spz_state_s *psi, spz_state_s *lam, 
 int launch_adj_sum(const double *part, uint64_t tiles, const uint32_t *d_idx, int slots,
                    double *grad);
 
-// Bytes of partial sums that adjoint_undo needs for a state of N amplitudes.
+// Bytes of partial sums that adjoint_undo needs for a state of N amplitudes
+// (more than one tile; a smaller one needs 2 kChipRows doubles per op).
 inline size_t adj_part_bytes(uint64_t N) { return (N >> kAdjK) * kAdjSlots * 2 * sizeof(double); }
 
-// Undo ops[lo, hi) (validated; more than kAdjK qubits, hi > lo) on psi, whose
+// Undo ops[lo, hi) (validated, hi > lo) on psi, whose
 // amplitudes are taken from src (another state or psi itself), and on lam, and
 // write dE/dtheta of each parametric one to the device array grad[0, hi).
 int adjoint_undo(const spz_state_s *src, spz_state_s *psi, spz_state_s *lam, const spz_op *ops,

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "spz_adj_tile.h"
+#include "spz_chip.h"
 #include "spz_internal.h"
 #include "spz_tile.h"
 
@@ -395,6 +396,9 @@ struct Planner {
     // Reverse sweeps of the adjoint: every gate runs in a sweep (a single one
     // too), and a sweep takes at most max_grads gates with a gradient.
     int max_grads = 0;
+    // Cheap planning (spz_chip.h): every sweep is a tile sweep, the next register
+    // bits are simply the best-scored ones.
+    bool quick = false;
     std::vector<uint32_t> grads;  // the sweeps' gradients, slot by slot
     uint64_t frame_gates = 0;  // gates absorbed into Pauli frames
     uint64_t split_ops = 0;    // second halves of gates run as two half-angle ops
@@ -745,6 +749,11 @@ struct Planner {
         for (int b = lo; b < K; b++) bits.push_back(b);
         std::stable_sort(bits.begin(), bits.end(),
                          [&](int x, int y) { return score[x] > score[y]; });
+        if (quick) {
+            std::vector<int> out(bits.begin(), bits.begin() + RB);
+            std::sort(out.begin(), out.end());
+            return out;
+        }
         const int T = std::min((int)bits.size(), std::max(RB, 8));
         uint32_t best = 0;
         double best_val = -1e30;
@@ -868,6 +877,8 @@ struct Planner {
                     std::vector<int> nx;
                     std::vector<long> score(K, 0);
                     for (int p2 = pos; p2 < m; p2++) {
+                        // (scores only place lanes 4 and 5, for swaps)
+                        if (!swaps && (int)nx.size() == RB) break;
                         const SG &h = run[order[p2]];
                         if (h.diag) continue;
                         int hb = lbit[h.target];
@@ -1252,7 +1263,7 @@ struct Planner {
                 while (keep < order.size() && (run[order[keep]].grad < 0 || left-- > 0)) keep++;
                 order.resize(keep);
             }
-            if (order.size() < 2 && !max_grads) {
+            if (order.size() < 2 && !max_grads && !quick) {
                 // nothing to fuse: the first remaining gate runs on the plain path
                 Sweep sw;
                 memset(&sw, 0, sizeof sw);
@@ -1285,9 +1296,14 @@ ProgSlot g_slots[2];
 int g_slot_next = 0;
 std::mutex g_slot_mu;
 
-// The program, and after it a list of 32-bit indices, into the next slot.
-int upload_program(const std::vector<TileOp> &prog, const std::vector<uint32_t> &idx,
-                   ProgSlot **out)
+// Several blocks of bytes into the next slot, each at a 256-byte boundary;
+// `at` receives their device addresses.
+struct Bytes {
+    const void *p;
+    size_t n;
+};
+
+int reserve_slot(size_t total, ProgSlot **out)
 {
     ProgSlot &sl = g_slots[g_slot_next];
     g_slot_next ^= 1;
@@ -1296,24 +1312,45 @@ int upload_program(const std::vector<TileOp> &prog, const std::vector<uint32_t> 
         sl.pending = false;
     }
     if (!sl.done) SPZ_HIP(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));
-    const size_t pb = prog.size() * sizeof(TileOp), ib = idx.size() * sizeof(uint32_t);
-    if (pb + ib > sl.cap) {
+    if (total > sl.cap) {
         if (sl.dev) SPZ_HIP(hipFree(sl.dev));
         if (sl.host) SPZ_HIP(hipHostFree(sl.host));
         sl.dev = nullptr;
         sl.host = nullptr;
         sl.cap = 0;
-        const size_t cap = std::max(pb + ib, 4096 * sizeof(TileOp));
+        const size_t cap = std::max(total, 4096 * sizeof(TileOp));
         if (hipMalloc(&sl.dev, cap) != hipSuccess ||
             hipHostMalloc(&sl.host, cap, hipHostMallocDefault) != hipSuccess)
             return fail(SPZ_ERR_OOM, "tile program allocation failed");
         sl.cap = cap;
     }
-    memcpy(sl.host, prog.data(), pb);
-    if (ib) memcpy(sl.host + pb, idx.data(), ib);
-    SPZ_HIP(hipMemcpyAsync(sl.dev, sl.host, pb + ib, hipMemcpyHostToDevice, rt().stream));
     *out = &sl;
     return SPZ_OK;
+}
+
+size_t aligned(size_t n) { return (n + 255) & ~(size_t)255; }
+
+int upload(const std::vector<Bytes> &parts, ProgSlot **out, std::vector<char *> *at)
+{
+    size_t total = 0;
+    for (const Bytes &b : parts) total += aligned(b.n);
+    ProgSlot *sl;
+    SPZ_TRY(reserve_slot(total, &sl));
+    size_t o = 0;
+    for (const Bytes &b : parts) {
+        if (b.n) memcpy(sl->host + o, b.p, b.n);
+        at->push_back(sl->dev + o);
+        o += aligned(b.n);
+    }
+    SPZ_HIP(hipMemcpyAsync(sl->dev, sl->host, total, hipMemcpyHostToDevice, rt().stream));
+    *out = sl;
+    return SPZ_OK;
+}
+
+template <typename T>
+Bytes bytes_of(const std::vector<T> &v)
+{
+    return {v.data(), v.size() * sizeof(T)};
 }
 
 // Marks a slot busy until the stream passes the point where it goes out of
@@ -1380,9 +1417,10 @@ int run_fused(spz_state_s *s, const std::vector<SG> &run, int K, bool strict)
     }
     std::lock_guard<std::mutex> lk(g_slot_mu);
     ProgSlot *slot = nullptr;
-    if (!pl.prog.empty()) SPZ_TRY(upload_program(pl.prog, {}, &slot));
-    const TileOp *d_prog = slot ? (const TileOp *)slot->dev : nullptr;
+    std::vector<char *> at;
+    if (!pl.prog.empty()) SPZ_TRY(upload({bytes_of(pl.prog)}, &slot, &at));
     Release release{slot};
+    const TileOp *d_prog = slot ? (const TileOp *)at[0] : nullptr;
     for (const Sweep &sw : pl.sweeps) {
         if (sw.tile) {
             SPZ_TRY(launch_tile(s, K, sw.desc, d_prog + sw.op_begin, pl.fast));
@@ -1549,38 +1587,167 @@ int run_dense5(spz_state_s *s, const std::vector<SG> &run)
 
 }  // namespace
 
+// A SWAP as three CX, the middle one with the SWAP's controls.
+void swap_as_cx(const spz_op &o, spz_op out[3])
+{
+    spz_op x;
+    memset(&x, 0, sizeof x);
+    x.kind = SPZ_X;
+    x.target = o.target;
+    x.ones = 1ull << o.t1;
+    spz_op y = x;
+    y.target = o.t1;
+    y.ones = o.ones | (1ull << o.target);
+    y.zeros = o.zeros;
+    out[0] = out[2] = x;
+    out[1] = y;
+}
+
+// Validated ops as a run on n qubits: forward, or undone from the last to the
+// first with the index of each one's gradient (SWAPs as CX).
+static int lower_run(int n, const spz_op *ops, uint64_t lo, uint64_t hi, bool reverse,
+                     std::vector<SG> &run)
+{
+    spz_state_s st;  // shape only
+    st.n = n;
+    st.N = 1ull << n;
+    run.clear();
+    run.reserve(hi - lo);
+    auto add = [&](const spz_op &o, int64_t grad) -> int {
+        SG g;
+        SPZ_TRY(lower(&st, o, nullptr, (int)run.size(), &g));
+        g.grad = grad;
+        run.push_back(g);
+        return SPZ_OK;
+    };
+    for (uint64_t i = lo; i < hi; i++) {
+        const uint64_t k = reverse ? hi - 1 - (i - lo) : i;
+        const spz_op o = reverse ? inverse_op(ops[k]) : ops[k];
+        if (o.kind == SPZ_SWAP) {
+            spz_op cx[3];
+            swap_as_cx(o, cx);
+            for (const spz_op &c : cx) SPZ_TRY(add(c, -1));
+            continue;
+        }
+        const bool par = reverse && (o.kind == SPZ_RX || o.kind == SPZ_RY || o.kind == SPZ_RZ ||
+                                     o.kind == SPZ_P);
+        SPZ_TRY(add(o, par ? (int64_t)k : -1));
+    }
+    return SPZ_OK;
+}
+
+// Lowers ops from *j on into a run, up to the next barrier (*j moves there).
+static int collect_run(const spz_state_s *s, const spz_op *ops, uint64_t n_ops,
+                       const spz_tracker *trk, bool small, uint64_t *j, std::vector<SG> &run);
+
+static int plan_chip(int n, const std::vector<SG> &run, bool strict, bool reverse, ChipPlan &out)
+{
+    Planner pl;
+    pl.n = std::max(n, kChipK);  // fewer qubits: the tile's other bits stay |0>
+    pl.K = kChipK;
+    pl.LOGW = kChipK - 4;
+    pl.RB = 4;
+    pl.klo = 4;
+    pl.strict = strict;
+    pl.quick = true;
+    if (reverse) pl.max_grads = 1 << 30;
+    pl.plan(run);
+    if (pl.bad) return fail(SPZ_ERR_ARG, "tile planner produced a gate outside the register layout");
+    out.sweeps.clear();
+    for (const Sweep &sw : pl.sweeps)
+        out.sweeps.push_back({sw.desc, (uint32_t)sw.op_begin, (uint32_t)sw.op_count,
+                              (uint32_t)sw.slot_begin, (uint32_t)sw.slots});
+    out.prog.swap(pl.prog);
+    out.grads.swap(pl.grads);
+    return SPZ_OK;
+}
+
+// (spz_chip.h)
+int chip_plan(int n, const spz_op *ops, uint64_t n_ops, bool reverse, ChipPlan &out)
+{
+    std::vector<SG> run;
+    SPZ_TRY(lower_run(std::max(n, kChipK), ops, 0, n_ops, reverse, run));
+    return plan_chip(n, run, false, reverse, out);
+}
+
+// A run on a state of at most kChipK qubits: one launch.  Program order is
+// kept, so the amplitudes are bit-identical to one launch per gate (FP32
+// storage: rounded once, at the end).
+static int run_chip(spz_state_s *s, const std::vector<SG> &run)
+{
+    ChipPlan cp;
+    SPZ_TRY(plan_chip(s->n, run, true, false, cp));
+    std::lock_guard<std::mutex> lk(g_slot_mu);
+    std::vector<ChipSweep> d(cp.sweeps.size());
+    ProgSlot *slot = nullptr;
+    SPZ_TRY(reserve_slot(aligned(cp.prog.size() * sizeof(TileOp)) +
+                             aligned(d.size() * sizeof(ChipSweep)), &slot));
+    Release release{slot};
+    const size_t o_d = aligned(cp.prog.size() * sizeof(TileOp));
+    for (size_t i = 0; i < d.size(); i++) {
+        memset(&d[i], 0, sizeof d[i]);
+        chip_geometry(cp.sweeps[i], s->n, s->prec, d[i]);
+        d[i].sr = d[i].pr = s->re;
+        d[i].si = d[i].pi = s->im;
+        d[i].ops = (const TileOp *)slot->dev + cp.sweeps[i].op_begin;
+        d[i].flags = CHIP_STORE;
+    }
+    memcpy(slot->host, cp.prog.data(), cp.prog.size() * sizeof(TileOp));
+    memcpy(slot->host + o_d, d.data(), d.size() * sizeof(ChipSweep));
+    SPZ_HIP(hipMemcpyAsync(slot->dev, slot->host, o_d + d.size() * sizeof(ChipSweep),
+                           hipMemcpyHostToDevice, rt().stream));
+    for (size_t i = 0; i < d.size(); i++) {  // (one: every qubit is in the tile)
+        LaunchTimer tm(SPZ_K_TILE, 2.0 * (double)s->N * (s->prec == SPZ_F64 ? 16.0 : 8.0));
+        SPZ_TRY(launch_chip_sweeps(s->prec, false, (const ChipSweep *)(slot->dev + o_d) + i, 1, 1, 0));
+    }
+    return SPZ_OK;
+}
+
 // (spz_adj_tile.h)
 int adjoint_undo(const spz_state_s *src, spz_state_s *psi, spz_state_s *lam, const spz_op *ops,
                  uint64_t lo, uint64_t hi, double *part, double *grad)
 {
     std::vector<SG> run;
-    run.reserve(hi - lo);
-    auto add = [&](const spz_op &o, int64_t slot) -> int {
-        SG g;
-        SPZ_TRY(lower(psi, o, nullptr, (int)run.size(), &g));
-        g.grad = slot;
-        run.push_back(g);
-        return SPZ_OK;
-    };
-    for (uint64_t k = hi; k-- > lo;) {
-        const spz_op o = inverse_op(ops[k]);
-        if (o.kind == SPZ_SWAP) {  // three CX, the middle one with the SWAP's controls
-            spz_op x;
-            memset(&x, 0, sizeof x);
-            x.kind = SPZ_X;
-            x.target = o.target;
-            x.ones = 1ull << o.t1;
-            spz_op y = x;
-            y.target = o.t1;
-            y.ones = o.ones | (1ull << o.target);
-            y.zeros = o.zeros;
-            SPZ_TRY(add(x, -1));
-            SPZ_TRY(add(y, -1));
-            SPZ_TRY(add(x, -1));
-            continue;
+    const bool chip = psi->n <= kChipK;
+    SPZ_TRY(lower_run(chip ? kChipK : psi->n, ops, lo, hi, true, run));
+    if (chip) {
+        ChipPlan cp;
+        SPZ_TRY(plan_chip(psi->n, run, false, true, cp));
+        std::vector<ChipSweep> d(cp.sweeps.size());
+        std::vector<ChipSum> sums;
+        const size_t o_d = aligned(cp.prog.size() * sizeof(TileOp));
+        const size_t o_s = o_d + aligned(d.size() * sizeof(ChipSweep));
+        const size_t total = o_s + aligned(cp.grads.size() * sizeof(ChipSum));
+        std::lock_guard<std::mutex> lk(g_slot_mu);
+        ProgSlot *slot = nullptr;
+        SPZ_TRY(reserve_slot(total, &slot));
+        Release release{slot};
+        for (size_t i = 0; i < d.size(); i++) {
+            memset(&d[i], 0, sizeof d[i]);
+            chip_geometry(cp.sweeps[i], psi->n, psi->prec, d[i]);
+            d[i].sr = src->re;
+            d[i].si = src->im;
+            d[i].pr = psi->re;
+            d[i].pi = psi->im;
+            d[i].qr = lam->re;
+            d[i].qi = lam->im;
+            d[i].ops = (const TileOp *)slot->dev + cp.sweeps[i].op_begin;
+            d[i].part = part + 2 * kChipRows * (size_t)cp.sweeps[i].slot_begin;
+            d[i].flags = CHIP_STORE;
+            src = psi;
         }
-        const bool par = o.kind == SPZ_RX || o.kind == SPZ_RY || o.kind == SPZ_RZ || o.kind == SPZ_P;
-        SPZ_TRY(add(o, par ? (int64_t)k : -1));
+        for (size_t k = 0; k < cp.grads.size(); k++)
+            sums.push_back({part + 2 * kChipRows * k, kChipRows, cp.grads[k]});
+        memcpy(slot->host, cp.prog.data(), cp.prog.size() * sizeof(TileOp));
+        memcpy(slot->host + o_d, d.data(), d.size() * sizeof(ChipSweep));
+        if (!sums.empty()) memcpy(slot->host + o_s, sums.data(), sums.size() * sizeof(ChipSum));
+        SPZ_HIP(hipMemcpyAsync(slot->dev, slot->host, total, hipMemcpyHostToDevice, rt().stream));
+        for (size_t i = 0; i < d.size(); i++) {
+            LaunchTimer tm(SPZ_K_ADJOINT, 4.0 * (double)psi->N * (psi->prec == SPZ_F64 ? 16.0 : 8.0));
+            SPZ_TRY(launch_chip_sweeps(psi->prec, true, (const ChipSweep *)(slot->dev + o_d) + i, 1,
+                                       1, 0));
+        }
+        return launch_chip_sums((const ChipSum *)(slot->dev + o_s), (uint32_t)sums.size(), grad);
     }
     Planner pl;
     pl.n = psi->n;
@@ -1595,10 +1762,11 @@ int adjoint_undo(const spz_state_s *src, spz_state_s *psi, spz_state_s *lam, con
     if (pl.bad) return fail(SPZ_ERR_ARG, "tile planner produced a gate outside the register layout");
     std::lock_guard<std::mutex> lk(g_slot_mu);
     ProgSlot *slot = nullptr;
-    SPZ_TRY(upload_program(pl.prog, pl.grads, &slot));
+    std::vector<char *> at;
+    SPZ_TRY(upload({bytes_of(pl.prog), bytes_of(pl.grads)}, &slot, &at));
     Release release{slot};
-    const TileOp *d_prog = (const TileOp *)slot->dev;
-    const uint32_t *d_idx = (const uint32_t *)(slot->dev + pl.prog.size() * sizeof(TileOp));
+    const TileOp *d_prog = (const TileOp *)at[0];
+    const uint32_t *d_idx = (const uint32_t *)at[1];
     const uint64_t tiles = psi->N >> kAdjK;
     for (const Sweep &sw : pl.sweeps) {
         SPZ_TRY(launch_adj_tile(src, psi, lam, sw.desc, d_prog + sw.op_begin, sw.slots, part));
@@ -1632,6 +1800,23 @@ int tile_width(const spz_exec_opts *opts, int n, int *K_out)
     return SPZ_OK;
 }
 
+// Whether a state takes the one-launch path: at most kChipK qubits, and no
+// tile width asked for.
+static bool small_path(const spz_exec_opts *opts, int n)
+{
+    return n <= kChipK && !(opts && opts->tile_qubits) && env_int("SPZ_TILE_K", 0) == 0;
+}
+
+// A SWAP that the one-launch path can take into a run: valid, and (its control
+// flags are resolved like a gate's) not under classical control.
+static bool plain_swap(const spz_op &o, int n)
+{
+    if (o.kind != SPZ_SWAP || (o.flags & SPZ_OPF_CLASSICAL)) return false;
+    if (o.target < 0 || o.target >= n || o.t1 < 0 || o.t1 >= n || o.target == o.t1) return false;
+    const uint64_t sw = (1ull << o.target) | (1ull << o.t1), c = o.ones | o.zeros;
+    return !(c & sw) && !(o.ones & o.zeros) && !(c >> n);
+}
+
 // Planning only (no device work): how the tile executor would split `ops`.
 int plan_info(int n, int prec, const spz_op *ops, uint64_t n_ops, const spz_exec_opts *opts,
               spz_plan_info *out)
@@ -1649,21 +1834,30 @@ int plan_info(int n, int prec, const spz_op *ops, uint64_t n_ops, const spz_exec
     st.n = n;
     st.prec = prec;
     st.N = 1ull << n;
+    const bool small = small_path(opts, n);
     uint64_t i = 0;
     while (i < n_ops) {
-        if (is_barrier(ops[i]) || K < 10) {
+        const bool barrier = is_barrier(ops[i]) && !(small && plain_swap(ops[i], n));
+        if (barrier || (K < 10 && !small)) {
             out->plain_gates++;
             i++;
             continue;
         }
         std::vector<SG> run;
         uint64_t j = i;
-        for (; j < n_ops && !is_barrier(ops[j]); j++) {
-            SG g;
-            int rc = lower(&st, ops[j], nullptr, (int)j, &g);
-            if (rc == -1) continue;
-            if (rc != SPZ_OK) return rc;
-            run.push_back(g);
+        SPZ_TRY(collect_run(&st, ops, n_ops, nullptr, small, &j, run));
+        if (small) {
+            if (!run.empty()) {
+                ChipPlan cp;
+                SPZ_TRY(plan_chip(n, run, true, false, cp));
+                out->sweeps += cp.sweeps.size();
+                for (const TileOp &op : cp.prog) {
+                    if (op.type == TOP_LAYOUT) out->layouts++;
+                    else out->tile_gates++;
+                }
+            }
+            i = j;
+            continue;
         }
         Planner pl;
         pl.n = n;
@@ -1697,6 +1891,34 @@ int plan_info(int n, int prec, const spz_op *ops, uint64_t n_ops, const spz_exec
     return SPZ_OK;
 }
 
+static int collect_run(const spz_state_s *s, const spz_op *ops, uint64_t n_ops,
+                       const spz_tracker *trk, bool small, uint64_t *j, std::vector<SG> &run)
+{
+    for (; *j < n_ops; (*j)++) {
+        const spz_op &o = ops[*j];
+        spz_op cx[3];
+        int n = 1;
+        if (is_barrier(o)) {
+            if (!(small && plain_swap(o, s->n))) break;
+            swap_as_cx(o, cx);
+            n = 3;
+        } else {
+            cx[0] = o;
+        }
+        for (int k = 0; k < n; k++) {
+            SG g;
+            const int rc = lower(s, cx[k], trk, (int)*j, &g);
+            if (rc == -1) continue;  // no-op (unflipped noise, classical control read 0)
+            if (rc != SPZ_OK) {
+                set_error("op " + std::to_string(*j) + ": " + spz_last_error());
+                return rc;
+            }
+            run.push_back(g);
+        }
+    }
+    return SPZ_OK;
+}
+
 int execute_ops(spz_state_s *s, const spz_op *ops, uint64_t n_ops, spz_tracker *trk,
                 const spz_exec_opts *opts, uint8_t *outcomes)
 {
@@ -1708,13 +1930,14 @@ int execute_ops(spz_state_s *s, const spz_op *ops, uint64_t n_ops, spz_tracker *
     if (dense5 && s->n < 12) return execute_plain(s, ops, n_ops, trk, outcomes);
     int K;
     SPZ_TRY(tile_width(opts, s->n, &K));
-    if (K < 10) return execute_plain(s, ops, n_ops, trk, outcomes);
+    const bool small = !dense5 && small_path(opts, s->n);
+    if (K < 10 && !small) return execute_plain(s, ops, n_ops, trk, outcomes);
     const bool strict = mode == SPZ_EXEC_STRICT;
     if (outcomes)
         for (uint64_t i = 0; i < n_ops; i++) outcomes[i] = 255;
     uint64_t i = 0;
     while (i < n_ops) {
-        if (is_barrier(ops[i])) {
+        if (is_barrier(ops[i]) && !(small && plain_swap(ops[i], s->n))) {
             int rc = exec_one_plain(s, ops[i], trk, outcomes ? &outcomes[i] : nullptr);
             if (rc != SPZ_OK) {
                 set_error("op " + std::to_string(i) + ": " + spz_last_error());
@@ -1725,17 +1948,10 @@ int execute_ops(spz_state_s *s, const spz_op *ops, uint64_t n_ops, spz_tracker *
         }
         std::vector<SG> run;
         uint64_t j = i;
-        for (; j < n_ops && !is_barrier(ops[j]); j++) {
-            SG g;
-            int rc = lower(s, ops[j], trk, (int)j, &g);
-            if (rc == -1) continue;  // no-op (unflipped noise, classical control read 0)
-            if (rc != SPZ_OK) {
-                set_error("op " + std::to_string(j) + ": " + spz_last_error());
-                return rc;
-            }
-            run.push_back(g);
-        }
-        if (!run.empty()) SPZ_TRY(dense5 ? run_dense5(s, run) : run_fused(s, run, K, strict));
+        SPZ_TRY(collect_run(s, ops, n_ops, trk, small, &j, run));
+        if (!run.empty())
+            SPZ_TRY(small ? run_chip(s, run)
+                          : dense5 ? run_dense5(s, run) : run_fused(s, run, K, strict));
         i = j;
     }
     return SPZ_OK;

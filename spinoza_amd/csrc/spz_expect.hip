@@ -18,7 +18,7 @@
 // and 64 us for x or y.
 #include <algorithm>
 
-#include "spz_reduce.h"
+#include "spz_ising.h"
 
 namespace spz {
 
@@ -167,21 +167,7 @@ k_finish(const double *__restrict__ partials, uint64_t nb, double *__restrict__ 
     if (threadIdx.x == 0) out[blockIdx.x] = r;
 }
 
-// xr += partner over qubits LO..LO+3 held in registers (bit 1 << k of e).
-template <int BIT>
-__device__ __forceinline__ void reg_sum(const double *a, const double *b, double *xr, double *xi)
-{
-#pragma unroll
-    for (int e = 0; e < kRE; e++) {
-        xr[e] = xr[e] + a[e ^ BIT];
-        xi[e] = xi[e] + b[e ^ BIT];
-    }
-}
-
-// H psi = (sum Z_i Z_{i+1} + hx sum X_i) psi on one block: the X sum of each
-// amplitude runs over the qubits in order; the block's energy terms
-// Re conj(psi_j) (H psi)_j go to its level-1 pair.  STORE keeps H psi, and the
-// terms then use it as stored.
+// H psi and the energy's level-1 pairs, one block per workgroup (spz_ising.h).
 //
 // Bound: the partner loads of the qubits above the block (one state read each,
 // from L2 where the partner block is in flight on the same XCD, else from the
@@ -195,75 +181,17 @@ k_ising(const T *__restrict__ re, const T *__restrict__ im, T *__restrict__ lr,
         T *__restrict__ li, uint64_t nb, int n, double hx, double *__restrict__ partials)
 {
     __shared__ double S[kRT], C[kRT];
-    const uint32_t tid = threadIdx.x;
-    const uint64_t blk = xcd_block(blockIdx.x, nb), base = blk * kRB;
-    double a[kRE], b[kRE], xr[kRE], xi[kRE];
-#pragma unroll
-    for (int e = 0; e < kRE; e++) {
-        a[e] = re[base + e * kRT + tid];
-        b[e] = im[base + e * kRT + tid];
-        xr[e] = 0.0;
-        xi[e] = 0.0;
-    }
-    auto far = [&](int q) {
-        const uint64_t p0 = (base + tid) ^ (1ull << q);
-        // a quarter of the block at a time keeps three waves per SIMD
-#pragma unroll
-        for (int h = 0; h < kRE; h += kRE / 4) {
-            T x[kRE / 4], y[kRE / 4];
-#pragma unroll
-            for (int e = 0; e < kRE / 4; e++) {
-                x[e] = re[p0 + (h + e) * kRT];
-                y[e] = im[p0 + (h + e) * kRT];
-            }
-#pragma unroll
-            for (int e = 0; e < kRE / 4; e++) {
-                xr[h + e] = xr[h + e] + (double)x[e];
-                xi[h + e] = xi[h + e] + (double)y[e];
-            }
-        }
-    };
-#pragma unroll 1
-    for (int q = 0; q < 6; q++) {
-#pragma unroll
-        for (int e = 0; e < kRE; e++) {
-            xr[e] = xr[e] + lane_xor(a[e], 1 << q);
-            xi[e] = xi[e] + lane_xor(b[e], 1 << q);
-        }
-    }
-    far(6);
-    far(7);
-    reg_sum<1>(a, b, xr, xi);
-    reg_sum<2>(a, b, xr, xi);
-    reg_sum<4>(a, b, xr, xi);
-    reg_sum<8>(a, b, xr, xi);
-#pragma unroll 1
-    for (int q = 12; q < n; q++) far(q);
-    const uint64_t bonds = (1ull << (n - 1)) - 1;
-    double s = 0.0, c = 0.0;
-#pragma unroll
-    for (int e = 0; e < kRE; e++) {
-        const uint64_t j = base + e * kRT + tid;
-        // aligned bonds count +1, opposed ones -1: an exact integer
-        const int czz = (n - 1) - 2 * __builtin_popcountll((j ^ (j >> 1)) & bonds);
-        double vr = (double)czz * a[e] + hx * xr[e];
-        double vi = (double)czz * b[e] + hx * xi[e];
-        if constexpr (STORE) {
-            lr[j] = (T)vr;
-            li[j] = (T)vi;
-            vr = (double)(T)vr;
-            vi = (double)(T)vi;
-        }
-        add_term(s, c, a[e] * vr + b[e] * vi);
-    }
-    S[tid] = s;
-    C[tid] = c;
-    __syncthreads();
-    tree256(S, C);
-    if (tid == 0) {
-        partials[2 * blk] = S[0];
-        partials[2 * blk + 1] = C[0];
-    }
+    const uint64_t blk = xcd_block(blockIdx.x, nb);
+    ising_block<T, STORE, false>(re, im, lr, li, blk * kRB, n, 0, hx, partials + 2 * blk, S, C);
+}
+
+template <typename T, bool STORE>
+__global__ void __launch_bounds__(kRT)
+k_ising_small(const T *__restrict__ re, const T *__restrict__ im, T *__restrict__ lr,
+              T *__restrict__ li, uint64_t N, int n, double hx, double *__restrict__ partials)
+{
+    __shared__ double S[kRT], C[kRT];
+    ising_block<T, STORE, true>(re, im, lr, li, 0, n, N, hx, partials, S, C);
 }
 
 template <typename T>
@@ -328,11 +256,18 @@ int expect_many(const spz_state_s *s, char observable, const int32_t *targets, u
 int ising_level1(const spz_state_s *s, double hx, void *lr, void *li, double *part)
 {
     const uint64_t nb = s->N / kRB;
-    const dim3 g((unsigned)nb), b(kRT);
     hipStream_t st = rt().stream;
-#define SPZ_IS(T, ST)                                                                            \
-    hipLaunchKernelGGL((k_ising<T, ST>), g, b, 0, st, (const T *)s->re, (const T *)s->im, (T *)lr, \
-                       (T *)li, nb, s->n, hx, part)
+#define SPZ_IS(T, ST)                                                                              \
+    do {                                                                                           \
+        if (nb)                                                                                    \
+            hipLaunchKernelGGL((k_ising<T, ST>), dim3((unsigned)nb), dim3(kRT), 0, st,               \
+                               (const T *)s->re, (const T *)s->im, (T *)lr, (T *)li, nb, s->n, hx,    \
+                               part);                                                              \
+        else                                                                                       \
+            hipLaunchKernelGGL((k_ising_small<T, ST>), dim3(1), dim3(kRT), 0, st,                    \
+                               (const T *)s->re, (const T *)s->im, (T *)lr, (T *)li, s->N, s->n, hx,  \
+                               part);                                                              \
+    } while (0)
     if (s->prec == SPZ_F64) {
         if (lr) SPZ_IS(double, true);
         else SPZ_IS(double, false);

@@ -13,6 +13,7 @@
 // about 2048 workgroups keeps all 256 CUs busy for any state size.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "spz_reduce.h"
@@ -274,19 +275,6 @@ __device__ __forceinline__ double term(const T *__restrict__ re, const T *__rest
         double x = re[j], y = im[j];
         double w = x * x + y * y;
         return (((j >> q0) ^ (j >> q1)) & 1) ? -w : w;
-    } else if constexpr (TERM == TERM_ISING) {
-        int czz = 0;
-        for (int i = 0; i + 1 < n; i++) czz += (((j >> i) ^ (j >> (i + 1))) & 1) ? -1 : 1;
-        double xr = 0.0, xi = 0.0;
-        for (int i = 0; i < n; i++) {
-            uint64_t p = j ^ (1ull << i);
-            xr = xr + (double)re[p];
-            xi = xi + (double)im[p];
-        }
-        double a = re[j], b = im[j];
-        double lr = (double)czz * a + hx * xr;
-        double li = (double)czz * b + hx * xi;
-        return a * lr + b * li;
     } else if constexpr (TERM == TERM_DOT_RE) {
         double a = re[j], b = im[j], c = re2[j], d = im2[j];
         return a * c + b * d;
@@ -555,7 +543,6 @@ static int reduce_launch(const spz_state_s *a, const spz_state_s *b, int term, i
     case TERM_Y: SPZ_RL(TERM_Y); break;
     case TERM_Z: SPZ_RL(TERM_Z); break;
     case TERM_ZZ: SPZ_RL(TERM_ZZ); break;
-    case TERM_ISING: SPZ_RL(TERM_ISING); break;
     case TERM_DOT_RE: SPZ_RL(TERM_DOT_RE); break;
     case TERM_DOT_IM: SPZ_RL(TERM_DOT_IM); break;
     default: return fail(SPZ_ERR_ARG, "unknown reduction term");
@@ -591,8 +578,8 @@ int reduce(const spz_state_s *a, const spz_state_s *b, int term, int q0, int q1,
            double *out)
 {
     uint64_t nb;
-    if (term == TERM_ISING && a->N >= kRB) {
-        nb = a->N / kRB;
+    if (term == TERM_ISING) {
+        nb = std::max<uint64_t>(a->N / kRB, 1);
         SPZ_TRY(ensure_partials(nb));
         LaunchTimer tm(SPZ_K_REDUCE, (double)a->N * amp_bytes(a));
         SPZ_TRY(ising_level1(a, hx, nullptr, nullptr, rt().d_partials));
@@ -634,12 +621,7 @@ int ising_energy_noalloc(const spz_state_s *s, double hx, double *out)
         return fail(SPZ_ERR_ARG, "state too large for spz_ising_energy_noalloc (at most 2^30 "
                                  "amplitudes; use spz_ising_energy)");
     double *part = g_static_scratch;
-    if (M >= kRB)
-        SPZ_TRY(ising_level1(s, hx, nullptr, nullptr, part));
-    else
-        SPZ_TRY(s->prec == SPZ_F64
-                    ? reduce_launch<double>(s, nullptr, TERM_ISING, 0, 0, hx, M, nb, part)
-                    : reduce_launch<float>(s, nullptr, TERM_ISING, 0, 0, hx, M, nb, part));
+    SPZ_TRY(ising_level1(s, hx, nullptr, nullptr, part));
     // the pinned result slots were allocated when the library initialised
     return reduce_finish(part, nb, out);
 }

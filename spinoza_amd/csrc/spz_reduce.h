@@ -87,8 +87,8 @@ constexpr int kExpectGroup = 8;
 // states of at least 4096 amplitudes).
 int expect_many(const spz_state_s *s, char observable, const int32_t *targets, uint64_t n_targets,
                 double *out);
-// Level-1 pairs of the Ising energy into `part` and, with lr and li, the
-// amplitudes of H psi (states of at least 4096 amplitudes).
+// Level-1 pairs of the Ising energy into `part` (one per 4096 amplitudes, or
+// one) and, with lr and li, the amplitudes of H psi.
 int ising_level1(const spz_state_s *s, double hx, void *lr, void *li, double *part);
 // Second level over `nb` pairs into *out (waits for the result), or into a
 // pinned slot of rt().h_result without a wait.
