@@ -289,7 +289,7 @@ def batch_leg(spz, N, count, seed=5, group_qubits=0, wg_max=0, wg_per_cu=0):
         err = max(err, abs(e - e1), float(np.max(np.abs(g - g1))))
     del states
     return {"circuits": count, "params": nparams, "wg_max_qubits": wg,
-            "wg_per_cu": wg_per_cu if wg_per_cu else 2,  # (0: the library default)
+            "wg_per_cu": wg_per_cu,  # (0: as many as fit)
             "n_small": st["n_small"], "n_large": st["n_large"], "n_group": st["n_group"],
             "total_ms": round(dt * 1e3, 2), "p50_ms": round(st["p50_ms"], 4),
             "p99_ms": round(st["p99_ms"], 4), "grads_per_s": round(nparams / dt, 1),

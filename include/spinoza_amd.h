@@ -269,27 +269,28 @@ typedef struct spz_batch_circuit {
 } spz_batch_circuit;
 
 typedef struct spz_batch_opts {
-    int32_t wg_max_qubits;  /* circuits with n <= this run in the persistent
-                               kernel; 0 = autotuned value (or 14 before
+    int32_t wg_max_qubits;  /* circuits with n <= this (and <= 20) run batched,
+                               one launch per sweep of all of them; 0 =
+                               autotuned value (or 14 before
                                spz_batch_autotune ran)                      */
-    int32_t use_graph;      /* capture the persistent launch in a hipGraph  */
-    int32_t group_qubits;   /* circuits in the persistent kernel with more
-                               qubits run on 2^(n - group_qubits) workgroups
-                               of one XCD; 0 = 12, < 0 = never (values
-                               below 8 count as 8)                          */
-    int32_t wg_per_cu;      /* resident persistent-kernel workgroups per CU:
-                               0 = 2 (a group's members then share their CU
-                               with at most one other circuit, which bounds
-                               the per-circuit tail), < 0 = as many as fit  */
+    int32_t use_graph;      /* accepted; the launches are the same either way */
+    int32_t group_qubits;   /* batched circuits with more qubits run on
+                               2^(n - group_qubits) workgroups (at most one
+                               per tile of 2^12 amplitudes); 0 = 12, < 0 =
+                               always one workgroup (values below 8 count
+                               as 8)                                        */
+    int32_t wg_per_cu;      /* most workgroups resident on a CU (from 2 up);
+                               <= 0 = as many as fit                        */
     int32_t reserved[4];
 } spz_batch_opts;
 
 typedef struct spz_batch_stats {
     double total_ms;        /* wall time of the whole batch                 */
-    double p50_ms, p99_ms;  /* per-circuit processing time                  */
+    double p50_ms, p99_ms;  /* per-circuit processing time (batched: the time
+                               of the chunk that holds the circuit)          */
     uint64_t n_small, n_large;
     int32_t wg_max_qubits;
-    int32_t n_group;        /* circuits run on a group of workgroups        */
+    int32_t n_group;        /* batched circuits above group_qubits           */
 } spz_batch_stats;
 
 /* Energy and adjoint gradient (as spz_adjoint_grad, no checkpoints) of every
@@ -297,14 +298,14 @@ typedef struct spz_batch_stats {
  * may be single-target gates H..U with up to 7 controls (1- or 0-controls,
  * none equal to the target, no qubit both).  Every op of every circuit is
  * checked before any work starts, by the same rule whichever path (the
- * persistent kernel or the single-circuit one) a circuit would take: one bad
+ * batched one or the single-circuit one) a circuit would take: one bad
  * op fails the whole call with SPZ_ERR_GATE / SPZ_ERR_QUBIT.  opts and stats
  * may be NULL. */
 int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const spz_op *ops,
                       double hx, double *energies, double *grads,
                       const spz_batch_opts *opts, spz_batch_stats *stats);
-/* Measure, per qubit count present in the batch, the persistent workgroup
- * kernel against the single-circuit path and keep the switch point for later
+/* Measure, per qubit count present in the batch, the batched sweeps
+ * against the single-circuit path and keep the switch point for later
  * spz_batch_adjoint calls (also returned in *wg_max_qubits). */
 int spz_batch_autotune(const spz_batch_circuit *circuits, uint64_t count, const spz_op *ops,
                        int *wg_max_qubits);

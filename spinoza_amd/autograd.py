@@ -120,10 +120,11 @@ def batch_adjoint(circuits, hx=1.0, wg_max_qubits=0, use_graph=True, group_qubit
     """Energies and adjoint gradients of many independent circuits.
 
     `circuits` is a list of (n, ops); every circuit starts in |0...0>.
-    Circuits up to `wg_max_qubits` run in the persistent kernel, those above
-    `group_qubits` of them on a group of workgroups (0: the defaults; a
-    negative group_qubits keeps every circuit in one workgroup), with
-    `wg_per_cu` resident workgroups per CU (0: 2; negative: as many as fit).
+    Circuits up to `wg_max_qubits` run batched, one launch per sweep of all of
+    them, those above `group_qubits` on several workgroups each (0: the
+    defaults; a negative group_qubits keeps every circuit in one workgroup),
+    with at most `wg_per_cu` workgroups per CU (<= 0: as many as fit).
+    `use_graph` is accepted and changes nothing.
     Returns (energies, [grad_per_op arrays], stats dict)."""
     all_ops, table, off, goff = [], [], 0, 0
     for n, ops in circuits:
@@ -154,8 +155,8 @@ def batch_adjoint(circuits, hx=1.0, wg_max_qubits=0, use_graph=True, group_qubit
 
 
 def batch_autotune(circuits):
-    """Measure and keep the qubit count up to which circuits run one per
-    workgroup (see spz_batch_autotune)."""
+    """Measure and keep the qubit count up to which circuits run batched (see
+    spz_batch_autotune)."""
     all_ops, table, off = [], [], 0
     for n, ops in circuits:
         table.append((n, len(ops), off))

@@ -216,16 +216,6 @@ AdjScratch &adj_scratch()
 
 }  // namespace
 
-// Size the adjoint's scratch for circuits of up to n qubits and n_ops ops, so
-// that later calls allocate (and free) nothing.
-int adjoint_reserve(int n, int prec, uint64_t n_ops)
-{
-    AdjScratch &sc = adj_scratch();
-    std::lock_guard<std::mutex> lock(sc.mu);
-    SPZ_TRY(sc.reserve_states(n, prec));
-    return sc.buffers(grad_bytes(n_ops), std::max(part_bytes(1ull << n, n_ops), part_bytes(1, n_ops)));
-}
-
 // The ops a differentiated circuit may hold: unitary single-target gates H..U
 // (and SWAP where allowed) with 1- and 0-controls; every qubit in range, the
 // target (SWAP: both qubits) not a control, no qubit both a 1- and a

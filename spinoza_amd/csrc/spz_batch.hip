@@ -1,573 +1,322 @@
 // spz_batch.hip -- batched adjoint gradients of many independent circuits
 // (no counterpart in the reference).
 //
-// Circuits up to the switch point run inside a persistent kernel.  Small ones
-// (n <= group_qubits, 12 by default) run whole inside one workgroup: the
-// workgroup takes the next ticket from an atomic queue, keeps psi and lambda in
-// its own slice of a scratch buffer, runs the forward gates, lambda = H psi,
-// the energy, and the reverse sweep with the per-parameter reductions, all
-// separated by workgroup barriers instead of kernel launches.  Larger ones run
-// on a group of 2^(n - group_qubits) workgroups of one XCD: each member owns a
-// contiguous share of every gate's pairs, and the members meet at a group
-// barrier after every gate (a counter in memory; the members' stores reach the
-// XCD's shared L2 before they arrive, and each member drops its CU's L1 copies
-// after it leaves, so no L2 writeback is needed).  Every XCD has its own
-// ticket queue, and a workgroup only takes tickets from the queue of the XCD
-// it runs on, so a group's members always share an L2; tickets are handed out
-// in order, so at most the group at the head of a queue is incomplete and its
-// missing members are the next workgroups to finish their work.  Barrier
-// waits are bounded: a member that waits too long raises an error flag and
-// every workgroup leaves.  Larger circuits use the whole GPU one at a time
-// (the single-circuit path).  The switch point is measured by
+// Circuits up to the switch point are planned as tile sweeps and run level by
+// level (spz_chip.hip): one launch takes the k-th sweep of every circuit of a
+// chunk, so a launch has a tile of 2^12 amplitudes per workgroup whatever the
+// circuits' sizes, a gate costs register arithmetic instead of a pass through
+// the caches, and nothing waits inside a kernel.  A chunk is a set of circuits
+// with about as many tiles as the GPU holds workgroups; its programs are
+// planned and uploaded while the GPU runs the chunk before.  Larger circuits use
+// the single-circuit path one at a time.  The switch point is measured by
 // spz_batch_autotune.
+//
+// What bounded it: a persistent kernel that moved every gate's pairs through
+// the L2 (one workgroup, or a group of workgroups of one XCD with a barrier
+// around every gate that crossed their blocks): 33.3 ms of device time for 128
+// circuits of 10 to 18 qubits, 6.7 ms now (whole call 50.8 -> 10.3 ms).  Chunks
+// of 192 to 1536 tiles measured within 5% of each other.
 #include <math.h>
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
+#include <new>
+#include <system_error>
+#include <thread>
 #include <vector>
 
-#include "spz_internal.h"
+#include "spz_chip.h"
+#include "spz_reduce.h"
 
 namespace spz {
 
 int adjoint_grad(spz_state_s *s, const spz_op *ops, uint64_t n_ops, double hx, int ckpt_every,
                  double *grad, double *energy, double *drift);
-int adjoint_reserve(int n, int prec, uint64_t n_ops);
 int validate_adjoint_op(int n, const spz_op &o, uint64_t idx, bool allow_swap, int max_controls);
 
 namespace {
 
-constexpr int kW = 256;
-constexpr int kMaxControls = 7;  // BOp::pos holds the target and up to 7 controls
-
-// Compact gate record for the persistent kernel.
-struct BOp {
-    int32_t ak_fwd, ak_inv;
-    int32_t target, gk;      // gk: 0 none, 1 X, 2 Y, 3 Z, 4 P (gradient term)
-    int32_t np, pad;
-    int8_t pos[8];           // ascending fixed positions (target + controls)
-    uint64_t ones;
-    double cf[8], ci[8];     // forward / inverse coefficients
-};
-
-struct BCirc {
-    int32_t n, nops;
-    uint64_t op0;            // first BOp
-    uint64_t grad0;          // first gradient slot
-    uint64_t region;         // group circuits: offset (doubles) of psi/lambda in the pool
-    uint64_t part;           // group circuits: offset (pairs) of the partial sums
-    uint32_t bar;            // group circuits: barrier counter index
-    uint32_t pad;
-};
-
-// One unit of work: member `m` of the `g` workgroups that run circuit `c`.
-struct BTicket {
-    uint32_t c;
-    uint16_t m, g;
-};
-
-constexpr unsigned kSpinLimit = 1u << 22;  // bounded barrier waits (~seconds)
-constexpr int kWgPerCu = 2;                // default resident workgroups per CU
-
-__device__ __forceinline__ void b_two_sum(double a, double b, double &s, double &e)
-{
-    double ss = a + b;
-    double bb = ss - a;
-    double aa = ss - bb;
-    e = (a - aa) + (b - bb);
-    s = ss;
-}
-
-// Workgroup sum of (s, c) pairs; result valid in thread 0.
-__device__ double wg_sum(double s, double c, double *S, double *C)
-{
-    const int tid = threadIdx.x;
-    __syncthreads();
-    S[tid] = s;
-    C[tid] = c;
-    __syncthreads();
-    for (int h = kW / 2; h >= 1; h >>= 1) {
-        if (tid < h) {
-            double ns, e;
-            b_two_sum(S[tid], S[tid + h], ns, e);
-            C[tid] = (C[tid] + C[tid + h]) + e;
-            S[tid] = ns;
-        }
-        __syncthreads();
-    }
-    return S[0] + C[0];
-}
-
-// Workgroup (S, C) pair of a compensated sum; valid in thread 0.
-__device__ void wg_pair(double s, double c, double *S, double *C, double &ps, double &pc)
-{
-    const int tid = threadIdx.x;
-    __syncthreads();
-    S[tid] = s;
-    C[tid] = c;
-    __syncthreads();
-    for (int h = kW / 2; h >= 1; h >>= 1) {
-        if (tid < h) {
-            double ns, e;
-            b_two_sum(S[tid], S[tid + h], ns, e);
-            C[tid] = (C[tid] + C[tid + h]) + e;
-            S[tid] = ns;
-        }
-        __syncthreads();
-    }
-    ps = S[0];
-    pc = C[0];
-}
-
-// XCD (XCC) this wavefront runs on: HW_REG_XCC_ID, bits 3:0 (gfx940 family).
-__device__ __forceinline__ unsigned xcc_id()
-{
-    return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15u;
-}
-
-// Group barrier: every member has made its stores visible in the XCD's L2
-// (s_waitcnt vmcnt(0) in every wavefront), one thread counts the arrival and
-// waits for `target` arrivals, then every member drops its CU's L1 lines so
-// that its next loads see the other members' stores (the members share the
-// XCD's L2, so no L2 writeback or invalidation is needed).  Returns false (and
-// raises *err) when the wait runs past kSpinLimit polls or another member
-// already gave up.
-__device__ bool group_barrier(unsigned *ctr, unsigned target, int *err, int *flag)
-{
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int ok = 1;
-        atomicAdd(ctr, 1u);
-        unsigned spins = 0;
-        while (__hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-            __builtin_amdgcn_s_sleep(1);
-            if (++spins > kSpinLimit ||
-                __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                atomicExch(err, 1);
-                ok = 0;
-                break;
-            }
-        }
-        *flag = ok;
-    }
-    __syncthreads();
-    const bool ok = *flag != 0;
-    asm volatile("buffer_inv sc0" ::: "memory");
-    __syncthreads();
-    return ok;
-}
-
-__device__ __forceinline__ void apply_ak(int ak, const double *k, double &a, double &b, double &c,
-                                         double &d)
-{
-    switch (ak) {
-    case AK_H: pair_update(AK_H, k, a, b, c, d); break;
-    case AK_X: pair_update(AK_X, k, a, b, c, d); break;
-    case AK_Y: pair_update(AK_Y, k, a, b, c, d); break;
-    case AK_RX: pair_update(AK_RX, k, a, b, c, d); break;
-    case AK_RY: pair_update(AK_RY, k, a, b, c, d); break;
-    case AK_U: pair_update(AK_U, k, a, b, c, d); break;
-    case AK_NEG: pair_update(AK_NEG, k, a, b, c, d); break;
-    case AK_PHASE: pair_update(AK_PHASE, k, a, b, c, d); break;
-    case AK_RZ: pair_update(AK_RZ, k, a, b, c, d); break;
-    default: pair_update(AK_MAT, k, a, b, c, d); break;
-    }
-}
-
-// Gradient term of op `gk` on one pair (psi: a, b, cc, d; lambda: la..ld).
-__device__ __forceinline__ double grad_term(int gk, double a, double b, double cc, double d,
-                                            double la, double lb, double lc, double ld)
-{
-    if (gk == 1) return (la * d - lb * cc) + (lc * b - ld * a);
-    if (gk == 2) return (lc * a + ld * b) - (la * cc + lb * d);
-    if (gk == 3) return (la * b - lb * a) - (lc * d - ld * cc);
-    return -2.0 * (lc * d - ld * cc);
-}
-
-// lambda_j = (H psi)_j for the open Ising chain; returns Re conj(psi_j) lambda_j.
-__device__ __forceinline__ double ising_row(const double *pr, const double *pi, double *lr,
-                                            double *li, uint64_t j, int n, double hx)
-{
-    int czz = 0;
-    for (int i = 0; i + 1 < n; i++) czz += (((j >> i) ^ (j >> (i + 1))) & 1) ? -1 : 1;
-    double xr = 0.0, xi = 0.0;
-    for (int i = 0; i < n; i++) {
-        const uint64_t p = j ^ (1ull << i);
-        xr = xr + pr[p];
-        xi = xi + pi[p];
-    }
-    const double a = pr[j], b = pi[j];
-    const double vr = (double)czz * a + hx * xr, vi = (double)czz * b + hx * xi;
-    lr[j] = vr;
-    li[j] = vi;
-    return a * vr + b * vi;
-}
-
-// Two ops whose pairs are the same amplitudes, split the same way over the
-// members: equal fixed positions (target and controls) and control values.
-__device__ __forceinline__ bool same_pairs(const BOp &a, const BOp &b)
-{
-    if (a.np != b.np || a.ones != b.ones) return false;
-    for (int i = 0; i < a.np; i++)
-        if (a.pos[i] != b.pos[i]) return false;
-    return true;
-}
-
-// A whole circuit in one workgroup (psi, lambda in the workgroup's slot).
-__device__ void run_single(const BCirc &c, uint64_t ci, const BOp *__restrict__ ops, double hx,
-                           double *pr, double *pi, double *lr, double *li, double *S, double *C,
-                           double *__restrict__ energies, double *__restrict__ grads)
-{
-    const int tid = threadIdx.x;
-    const int n = c.n;
-    const uint64_t N = 1ull << n;
-    for (uint64_t j = tid; j < N; j += kW) {
-        pr[j] = j == 0 ? 1.0 : 0.0;
-        pi[j] = 0.0;
-    }
-    __syncthreads();
-    // forward
-    for (int o = 0; o < c.nops; o++) {
-        const BOp &op = ops[c.op0 + o];
-        const uint64_t tb = 1ull << op.target;
-        const uint64_t np = N >> op.np;
-        for (uint64_t u = tid; u < np; u += kW) {
-            const uint64_t s0 = insert_zeros(u, op.pos, op.np) | op.ones;
-            const uint64_t s1 = s0 | tb;
-            double a = pr[s0], b = pi[s0], cc = pr[s1], d = pi[s1];
-            apply_ak(op.ak_fwd, op.cf, a, b, cc, d);
-            pr[s0] = a; pi[s0] = b; pr[s1] = cc; pi[s1] = d;
-        }
-        __syncthreads();
-    }
-    // lambda = H psi and the energy Re <psi|lambda>
-    double es = 0.0, ec = 0.0;
-    for (uint64_t j = tid; j < N; j += kW) {
-        double ns, er;
-        b_two_sum(es, ising_row(pr, pi, lr, li, j, n, hx), ns, er);
-        es = ns;
-        ec = ec + er;
-    }
-    const double e = wg_sum(es, ec, S, C);
-    if (tid == 0) energies[ci] = e;
-    __syncthreads();
-    // reverse sweep
-    for (int o = c.nops - 1; o >= 0; o--) {
-        const BOp &op = ops[c.op0 + o];
-        const uint64_t tb = 1ull << op.target;
-        const uint64_t np = N >> op.np;
-        const int gk = op.gk;
-        double gs = 0.0, gc = 0.0;
-        for (uint64_t u = tid; u < np; u += kW) {
-            const uint64_t s0 = insert_zeros(u, op.pos, op.np) | op.ones;
-            const uint64_t s1 = s0 | tb;
-            double a = pr[s0], b = pi[s0], cc = pr[s1], d = pi[s1];
-            double la = lr[s0], lb = li[s0], lc = lr[s1], ld = li[s1];
-            if (gk) {
-                double ns, er;
-                b_two_sum(gs, grad_term(gk, a, b, cc, d, la, lb, lc, ld), ns, er);
-                gs = ns;
-                gc = gc + er;
-            }
-            apply_ak(op.ak_inv, op.ci, a, b, cc, d);
-            apply_ak(op.ak_inv, op.ci, la, lb, lc, ld);
-            pr[s0] = a; pi[s0] = b; pr[s1] = cc; pi[s1] = d;
-            lr[s0] = la; li[s0] = lb; lr[s1] = lc; li[s1] = ld;
-        }
-        if (gk) {
-            const double g = wg_sum(gs, gc, S, C);
-            if (tid == 0) grads[c.grad0 + o] = g;
-        }
-        __syncthreads();
-    }
-}
-
-// Member m of the g workgroups running circuit c.  The member owns the m-th
-// contiguous block of N/g amplitudes: it initialises its block and forms
-// lambda on it, and it takes the m-th contiguous share of every gate's pairs,
-// which for a gate whose qubits all lie below log2(N/g) ("local") are exactly
-// the pairs inside its own block.  So the members only meet at a group
-// barrier around non-local gates (before one, because it reads other blocks,
-// and after it), before lambda (which reads every block), after lambda (the
-// reverse sweep overwrites what other members read) and at the end; runs of
-// local gates need none, and neither do two non-local gates in a row on the
-// same fixed positions and control values (RY then RZ on one qubit): a member
-// then reads and writes the same pairs in both, which no other member touches.  Partial sums go to `part` (one (S, C) pair per
-// member for the energy and for every op) and member 0 adds them, in member
-// order, after the last barrier.  Returns false when a barrier gave up.
-__device__ bool run_group(const BCirc &c, uint64_t ci, unsigned m, unsigned g,
-                          const BOp *__restrict__ ops, double hx, double *pool, unsigned *bars,
-                          double *parts, int *err, double *S, double *C, int *flag,
-                          double *__restrict__ energies, double *__restrict__ grads)
-{
-    const int tid = threadIdx.x;
-    const int n = c.n;
-    const uint64_t N = 1ull << n;
-    double *pr = pool + c.region, *pi = pr + N, *lr = pi + N, *li = lr + N;
-    double *part = parts + 2ull * c.part;  // [op 0..nops-1, energy][member][S, C]
-    unsigned *bar = bars + c.bar;
-    unsigned arrivals = 0;
-    auto sync = [&]() {
-        arrivals += g;
-        return group_barrier(bar, arrivals, err, flag);
-    };
-    const uint64_t share = N / g, lo = share * m;
-    const int lb = n - (31 - __builtin_clz(g));  // local qubits: below lb
-    for (uint64_t j = lo + tid; j < lo + share; j += kW) {
-        pr[j] = j == 0 ? 1.0 : 0.0;
-        pi[j] = 0.0;
-    }
-    bool prev_nl = false;
-    for (int o = 0; o < c.nops; o++) {
-        const BOp &op = ops[c.op0 + o];
-        const bool nl = op.pos[op.np - 1] >= lb;
-        const bool same = o > 0 && nl && prev_nl && same_pairs(op, ops[c.op0 + o - 1]);
-        if ((nl || prev_nl) && !same && !sync()) return false;
-        prev_nl = nl;
-        const uint64_t tb = 1ull << op.target;
-        const uint64_t np = N >> op.np, ps = np / g, plo = ps * m;
-        for (uint64_t u = plo + tid; u < plo + ps; u += kW) {
-            const uint64_t s0 = insert_zeros(u, op.pos, op.np) | op.ones;
-            const uint64_t s1 = s0 | tb;
-            double a = pr[s0], b = pi[s0], cc = pr[s1], d = pi[s1];
-            apply_ak(op.ak_fwd, op.cf, a, b, cc, d);
-            pr[s0] = a; pi[s0] = b; pr[s1] = cc; pi[s1] = d;
-        }
-        __syncthreads();
-    }
-    if (!sync()) return false;
-    {
-        double es = 0.0, ec = 0.0;
-        for (uint64_t j = lo + tid; j < lo + share; j += kW) {
-            double ns, er;
-            b_two_sum(es, ising_row(pr, pi, lr, li, j, n, hx), ns, er);
-            es = ns;
-            ec = ec + er;
-        }
-        double ps, pc;
-        wg_pair(es, ec, S, C, ps, pc);
-        if (tid == 0) {
-            part[2 * ((uint64_t)c.nops * g + m)] = ps;
-            part[2 * ((uint64_t)c.nops * g + m) + 1] = pc;
-        }
-    }
-    if (!sync()) return false;
-    prev_nl = false;
-    for (int o = c.nops - 1; o >= 0; o--) {
-        const BOp &op = ops[c.op0 + o];
-        const bool nl = op.pos[op.np - 1] >= lb;
-        const bool same = o + 1 < c.nops && nl && prev_nl && same_pairs(op, ops[c.op0 + o + 1]);
-        if ((nl || prev_nl) && !same && !sync()) return false;
-        prev_nl = nl;
-        const uint64_t tb = 1ull << op.target;
-        const uint64_t np = N >> op.np, ps = np / g, plo = ps * m;
-        const int gk = op.gk;
-        double gs = 0.0, gc = 0.0;
-        for (uint64_t u = plo + tid; u < plo + ps; u += kW) {
-            const uint64_t s0 = insert_zeros(u, op.pos, op.np) | op.ones;
-            const uint64_t s1 = s0 | tb;
-            double a = pr[s0], b = pi[s0], cc = pr[s1], d = pi[s1];
-            double la = lr[s0], lb2 = li[s0], lc = lr[s1], ld = li[s1];
-            if (gk) {
-                double ns, er;
-                b_two_sum(gs, grad_term(gk, a, b, cc, d, la, lb2, lc, ld), ns, er);
-                gs = ns;
-                gc = gc + er;
-            }
-            apply_ak(op.ak_inv, op.ci, a, b, cc, d);
-            apply_ak(op.ak_inv, op.ci, la, lb2, lc, ld);
-            pr[s0] = a; pi[s0] = b; pr[s1] = cc; pi[s1] = d;
-            lr[s0] = la; li[s0] = lb2; lr[s1] = lc; li[s1] = ld;
-        }
-        if (gk) {
-            double ps2, pc2;
-            wg_pair(gs, gc, S, C, ps2, pc2);
-            if (tid == 0) {
-                part[2 * ((uint64_t)o * g + m)] = ps2;
-                part[2 * ((uint64_t)o * g + m) + 1] = pc2;
-            }
-        }
-        __syncthreads();
-    }
-    if (!sync()) return false;
-    if (m == 0) {
-        // energy (slot nops) and every parameter's gradient, members in order
-        for (int o = tid; o <= c.nops; o += kW) {
-            if (o < c.nops && !ops[c.op0 + o].gk) continue;
-            double ts = 0.0, tc = 0.0;
-            for (unsigned k = 0; k < g; k++) {
-                double ns, er;
-                b_two_sum(ts, part[2 * ((uint64_t)o * g + k)], ns, er);
-                tc = (tc + part[2 * ((uint64_t)o * g + k) + 1]) + er;
-                ts = ns;
-            }
-            if (o == c.nops) energies[ci] = ts + tc;
-            else grads[c.grad0 + o] = ts + tc;
-        }
-    }
-    return true;
-}
-
-// Persistent kernel: every workgroup serves the ticket queue of its own XCD
-// (queue q = xcc % nq) until the queue is empty or a group barrier failed.
-__global__ void __launch_bounds__(kW)
-k_batch_adjoint(const BCirc *__restrict__ circs, const BTicket *__restrict__ tickets,
-                const uint32_t *__restrict__ qstart, const uint32_t *__restrict__ qlen, uint32_t nq,
-                const BOp *__restrict__ ops, double hx, double *__restrict__ scratch,
-                uint64_t slot_amps, double *__restrict__ pool, double *__restrict__ parts,
-                unsigned int *__restrict__ counters, int *__restrict__ err,
-                double *__restrict__ energies, double *__restrict__ grads,
-                unsigned long long *__restrict__ ticks)
-{
-    __shared__ double S[kW], C[kW];
-    __shared__ unsigned int cur;
-    __shared__ int flag;
-    const int tid = threadIdx.x;
-    double *pr = scratch + (uint64_t)blockIdx.x * 4 * slot_amps;
-    double *pi = pr + slot_amps, *lr = pi + slot_amps, *li = lr + slot_amps;
-    const uint32_t q = nq > 1 ? xcc_id() % nq : 0u;
-    unsigned int *qctr = counters + q;
-    unsigned int *bars = counters + nq;
-    for (;;) {
-        if (tid == 0) cur = atomicAdd(qctr, 1u);
-        __syncthreads();
-        const uint32_t t = cur;
-        __syncthreads();
-        if (t >= qlen[q]) break;  // uniform: every wavefront leaves together
-        const BTicket tk = tickets[qstart[q] + t];
-        const unsigned long long t_start = wall_clock64();
-        const BCirc c = circs[tk.c];
-        if (tk.g <= 1) {
-            run_single(c, tk.c, ops, hx, pr, pi, lr, li, S, C, energies, grads);
-        } else if (!run_group(c, tk.c, tk.m, tk.g, ops, hx, pool, bars, parts, err, S, C, &flag,
-                              energies, grads)) {
-            break;  // a group barrier gave up: leave (uniform, from the barrier's flag)
-        }
-        if (tid == 0 && ticks && tk.m == 0) {
-            ticks[2 * tk.c] = t_start;
-            ticks[2 * tk.c + 1] = wall_clock64();
-        }
-    }
-}
-
-// XCD of each of `count` workgroups (probe of the device's XCD layout).
-__global__ void k_xcc_probe(unsigned int *out)
-{
-    if (threadIdx.x == 0) out[blockIdx.x] = xcc_id();
-}
-
-// Zero `count` counters (inside a captured graph, where a memset node is
-// avoided) and the error flag.
-__global__ void k_zero_u32(unsigned int *p, uint32_t count, int *err)
-{
-    for (uint32_t i = threadIdx.x; i < count; i += blockDim.x) p[i] = 0u;
-    if (threadIdx.x == 0) *err = 0;
-}
-
-int lower_bop(const spz_op &o, BOp *b)
-{
-    memset(b, 0, sizeof *b);
-    if (o.kind < SPZ_H || o.kind > SPZ_U) return fail(SPZ_ERR_GATE, "batched adjoint: unsupported gate");
-    Coef kf, ki;
-    SPZ_TRY(make_coef(o.kind, o.theta, o.phi, o.lambda, &kf));
-    double th = o.theta, ph = o.phi, la = o.lambda;
-    if (o.kind == SPZ_P || o.kind == SPZ_RX || o.kind == SPZ_RY || o.kind == SPZ_RZ) th = -th;
-    if (o.kind == SPZ_U) { th = -o.theta; ph = -o.lambda; la = -o.phi; }
-    SPZ_TRY(make_coef(o.kind, th, ph, la, &ki));
-    b->ak_fwd = kf.ak;
-    b->ak_inv = ki.ak;
-    for (int j = 0; j < 8; j++) { b->cf[j] = kf.c[j]; b->ci[j] = ki.c[j]; }
-    b->target = o.target;
-    b->gk = o.kind == SPZ_RX ? 1 : o.kind == SPZ_RY ? 2 : o.kind == SPZ_RZ ? 3 : o.kind == SPZ_P ? 4 : 0;
-    const uint64_t fixed = o.ones | o.zeros | (1ull << o.target);
-    int np = 0;
-    for (int q = 0; q < 64; q++)
-        if ((fixed >> q) & 1) {
-            if (np == 8) return fail(SPZ_ERR_GATE, "batched adjoint: more than 7 controls");
-            b->pos[np++] = (int8_t)q;
-        }
-    b->np = np;
-    b->ones = o.ones;
-    return SPZ_OK;
-}
+constexpr int kMaxControls = 7;
+constexpr int kBatchMaxQubits = 20;     // larger circuits fill the GPU on their own
+constexpr uint64_t kChunkTiles = 768;   // three reverse workgroups on each of 256 CUs
+constexpr uint64_t kChunkOps = 20000;   // bounds a chunk's program (128 bytes per op)
+constexpr int kPlanThreads = 8;
+constexpr size_t kKeep = (size_t)1 << 30;  // scratch kept between calls
 
 int g_wg_max_qubits = -1;  // autotuned switch point (-1: not tuned yet)
 
-// A second stream (default priority) for the persistent small-circuit kernel,
-// so that it runs beside the single-circuit path of the larger circuits.
-hipStream_t side_stream()
-{
-    static hipStream_t st = nullptr;
-    if (!st && hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) {
-        (void)hipGetLastError();
-        st = nullptr;
-    }
-    return st;
-}
-
-// Buffers of the persistent launch, kept across calls and grown when a call
-// needs more (a free synchronises the device), and the captured launch, which
-// is launched again while its arguments stay the same (a call with the same
-// batch shape and the same buffers).
-struct BatchBuf {
+// Grow-only device buffers, given back at the end of a call that needed more
+// than kKeep bytes of them (a free synchronises the device).
+struct Buf {
     void *p = nullptr;
     size_t cap = 0;
-};
-struct BatchCache {
-    BatchBuf circ, ops, scr, cnt, err, tk, q, pool, parts, e, g, t;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    std::vector<uint64_t> key;  // the captured launch's arguments
-};
-BatchCache g_bc;
 
-bool grow(BatchBuf &b, size_t bytes)
-{
-    bytes = std::max<size_t>(bytes, 256);
-    if (bytes <= b.cap) return true;
-    if (b.p) (void)hipFree(b.p);
-    b.p = nullptr;
-    b.cap = 0;
-    if (hipMalloc(&b.p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
+    int need(size_t bytes)
+    {
+        if (bytes <= cap) return SPZ_OK;
+        drop();
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return fail(SPZ_ERR_OOM, "batched adjoint scratch allocation failed");
+        }
+        cap = bytes;
+        return SPZ_OK;
     }
-    b.cap = bytes;
-    return true;
+    void drop()
+    {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        cap = 0;
+    }
+};
+
+// A chunk's program goes through one of two pinned staging buffers and device
+// copies, so that the next chunk is planned while this one runs; `done` is
+// recorded after the last kernel that reads the slot.
+struct Slot {
+    char *host = nullptr, *dev = nullptr;
+    size_t cap = 0;
+    hipEvent_t done = nullptr;
+    bool busy = false;
+
+    int open(size_t bytes)
+    {
+        if (busy) {
+            SPZ_HIP(hipEventSynchronize(done));
+            busy = false;
+        }
+        if (!done) SPZ_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+        if (bytes <= cap) return SPZ_OK;
+        drop();
+        if (hipMalloc(&dev, bytes) != hipSuccess ||
+            hipHostMalloc(&host, bytes, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            drop();
+            return fail(SPZ_ERR_OOM, "batched adjoint program allocation failed");
+        }
+        cap = bytes;
+        return SPZ_OK;
+    }
+    void drop()
+    {
+        if (dev) (void)hipFree(dev);
+        if (host) (void)hipHostFree(host);
+        dev = host = nullptr;
+        cap = 0;
+    }
+};
+
+// All of it is used under the library lock.
+struct Scratch {
+    Buf states, parts, out;
+    Slot slots[2];
+    std::vector<hipEvent_t> events;  // pairs of timing events, one per chunk
+};
+Scratch &scratch()
+{
+    static Scratch *s = new Scratch();  // lives until the process ends
+    return *s;
 }
 
-// Number of XCDs, from the XCC ids that workgroups report (0 when the ids do
-// not cover 0..k-1: grouped circuits are then disabled).  Measured once.
-int xcd_count()
+uint64_t tiles_of(int n) { return n > kChipK ? 1ull << (n - kChipK) : 1ull; }
+
+size_t up(size_t n) { return (n + 255) & ~(size_t)255; }
+
+// The sweep of a circuit without ops: it only writes |0...0>.
+ChipPlan::Sweep empty_sweep()
 {
-    static int nx = -1;
-    if (nx >= 0) return nx;
-    nx = 0;
-    const unsigned P = (unsigned)std::max(rt().cu_count, 1) * 8u;
-    unsigned int *d = nullptr;
-    if (hipMalloc(&d, P * sizeof(unsigned int)) != hipSuccess) {
-        (void)hipGetLastError();
-        return nx;
+    ChipPlan::Sweep s;
+    memset(&s, 0, sizeof s);
+    for (int i = 0; i < 16; i++) s.desc.spos[i] = (int8_t)(i < kChipK ? i : 64);
+    for (int i = 0; i < kChipK - 4; i++) {
+        s.desc.tin[i] = (int8_t)i;
+        s.desc.tg[i] = 1ull << i;
     }
-    std::vector<unsigned int> h(P, 0);
-    hipLaunchKernelGGL(k_xcc_probe, dim3(P), dim3(64), 0, rt().stream, d);
-    const bool ok = hipGetLastError() == hipSuccess &&
-                    hipMemcpyAsync(h.data(), d, P * sizeof(unsigned int), hipMemcpyDeviceToHost,
-                                   rt().stream) == hipSuccess &&
-                    hipStreamSynchronize(rt().stream) == hipSuccess;
-    (void)hipFree(d);
-    if (!ok) return nx;
-    unsigned seen = 0, mx = 0;
-    for (unsigned v : h) {
-        if (v >= 16) return nx;
-        seen |= 1u << v;
-        mx = std::max(mx, v);
-    }
-    if (seen == (2u << mx) - 1) nx = (int)mx + 1;
-    return nx;
+    for (uint64_t p = 0; p < 16; p++) s.desc.gr[p] = s.desc.gs[p] = p << (kChipK - 4);
+    return s;
 }
+
+struct Job {
+    uint64_t circuit;   // index in the caller's list
+    uint32_t width;     // workgroups it may use
+};
+
+// Forward and reverse plans of a chunk's circuits.  Planning costs about 0.1 us
+// per op and direction, more than the GPU takes for circuits of up to 12 qubits
+// (180 of them: 6.0 ms planned by one thread, 0.6 ms of sweeps), so a chunk is
+// planned by several threads once it has enough ops to pay for starting them.
+int plan_chunk(const spz_batch_circuit *circuits, const spz_op *ops, const Job *jobs,
+               uint32_t count, std::vector<ChipPlan> &fwd, std::vector<ChipPlan> &rev)
+{
+    uint64_t nops = 0;
+    for (uint32_t c = 0; c < count; c++) nops += (uint64_t)circuits[jobs[c].circuit].n_ops;
+    std::atomic<uint32_t> next{0};
+    std::atomic<int> status{SPZ_OK};
+    auto work = [&]() {
+        try {
+            for (uint32_t c; status == SPZ_OK && (c = next++) < count;) {
+                const spz_batch_circuit &q = circuits[jobs[c].circuit];
+                const spz_op *o = ops + q.op_offset;
+                int rc = chip_plan(q.n, o, (uint64_t)q.n_ops, false, fwd[c]);
+                if (rc == SPZ_OK) rc = chip_plan(q.n, o, (uint64_t)q.n_ops, true, rev[c]);
+                if (rc != SPZ_OK) status = rc;
+            }
+        } catch (const std::bad_alloc &) {
+            status = SPZ_ERR_OOM;
+        }
+    };
+    const unsigned cores = std::max(1u, std::thread::hardware_concurrency());
+    const uint64_t want = std::min<uint64_t>({(uint64_t)kPlanThreads, cores, count, nops / 1000 + 1});
+    std::vector<std::thread> pool;
+    pool.reserve(kPlanThreads);
+    try {
+        for (uint64_t t = 1; t < want; t++) pool.emplace_back(work);
+    } catch (const std::system_error &) {
+        // no more threads to be had: the ones there are do the work
+    }
+    work();
+    for (std::thread &t : pool) t.join();
+    if (status != SPZ_OK) return fail(status, "batched adjoint: planning failed");
+    return SPZ_OK;
+}
+
+// Plans, uploads and launches one chunk; energies go to out[circuit slot],
+// gradients to out[grad0 + grad_offset + op].
+struct Chunk {
+    const spz_batch_circuit *circuits;
+    const spz_op *ops;
+    double hx;
+    size_t lds;
+    uint64_t grad0;
+
+    int run(const Job *jobs, uint32_t count, uint32_t slot0, Scratch &sc, Slot &slot,
+            hipEvent_t begin, hipEvent_t end)
+    {
+        std::vector<ChipPlan> fwd(count), rev(count);
+        uint64_t amps = 0, pairs = 0, nops = 0;
+        size_t nf = 0, nr = 0, ns = 0, lf = 0, lr = 0;
+        uint32_t width = 0, blocks = 0;
+        SPZ_TRY(plan_chunk(circuits, ops, jobs, count, fwd, rev));
+        for (uint32_t c = 0; c < count; c++) {
+            const spz_batch_circuit &q = circuits[jobs[c].circuit];
+            if (fwd[c].sweeps.empty()) fwd[c].sweeps.push_back(empty_sweep());
+            const uint64_t t = tiles_of(q.n);
+            amps += 4 * (t << kChipK);
+            pairs += rev[c].grads.size() * t * kChipRows + t;
+            nops += fwd[c].prog.size() + rev[c].prog.size();
+            nf += fwd[c].sweeps.size();
+            nr += rev[c].sweeps.size();
+            ns += rev[c].grads.size() + 1;
+            lf = std::max(lf, fwd[c].sweeps.size());
+            lr = std::max(lr, rev[c].sweeps.size());
+            width = std::max(width, jobs[c].width);
+            blocks = std::max(blocks, (uint32_t)t);
+        }
+        SPZ_TRY(sc.states.need(amps * sizeof(double)));
+        SPZ_TRY(sc.parts.need(pairs * 2 * sizeof(double)));
+        const size_t o_f = up(nops * sizeof(TileOp)), o_i = o_f + up(nf * sizeof(ChipSweep));
+        const size_t o_r = o_i + up(count * sizeof(ChipIsing));
+        const size_t o_s = o_r + up(nr * sizeof(ChipSweep)), total = o_s + up(ns * sizeof(ChipSum));
+        SPZ_TRY(slot.open(total));
+        TileOp *hp = (TileOp *)slot.host;
+        ChipSweep *hf = (ChipSweep *)(slot.host + o_f), *hr = (ChipSweep *)(slot.host + o_r);
+        ChipIsing *hi = (ChipIsing *)(slot.host + o_i);
+        ChipSum *hs = (ChipSum *)(slot.host + o_s);
+        const TileOp *dp = (const TileOp *)slot.dev;
+        // programs, states and partial sums of every circuit
+        struct Place {
+            double *psi, *part;
+            uint64_t amps;
+            size_t fwd, rev;  // first op
+        };
+        std::vector<Place> at(count);
+        double *amp = (double *)sc.states.p, *part = (double *)sc.parts.p;
+        size_t op = 0, sum = 0;
+        for (uint32_t c = 0; c < count; c++) {
+            const spz_batch_circuit &q = circuits[jobs[c].circuit];
+            const uint64_t t = tiles_of(q.n);
+            at[c] = {amp, part, t << kChipK, op, op + fwd[c].prog.size()};
+            for (const ChipPlan *p : {&fwd[c], &rev[c]}) {
+                if (!p->prog.empty()) memcpy(hp + op, p->prog.data(), p->prog.size() * sizeof(TileOp));
+                op += p->prog.size();
+            }
+            for (size_t k = 0; k < rev[c].grads.size(); k++)
+                hs[sum++] = {part + 2 * k * t * kChipRows, (uint32_t)(t * kChipRows),
+                             (uint32_t)(grad0 + q.grad_offset + rev[c].grads[k])};
+            double *ep = part + 2 * rev[c].grads.size() * t * kChipRows;
+            hs[sum++] = {ep, (uint32_t)t, slot0 + c};
+            const uint64_t A = at[c].amps;
+            hi[c] = {amp, amp + A, amp + 2 * A, amp + 3 * A, 1ull << q.n, ep, (uint32_t)t, q.n};
+            amp += 4 * A;
+            part = ep + 2 * t;
+        }
+        // descriptors, level by level
+        auto fill = [&](ChipSweep &d, uint32_t c, const ChipPlan::Sweep &s, size_t first_op) {
+            memset(&d, 0, sizeof d);
+            chip_geometry(s, circuits[jobs[c].circuit].n, SPZ_F64, d);
+            const uint64_t A = at[c].amps;
+            d.sr = d.pr = at[c].psi;
+            d.si = d.pi = at[c].psi + A;
+            d.qr = at[c].psi + 2 * A;
+            d.qi = at[c].psi + 3 * A;
+            d.ops = dp + first_op + s.op_begin;
+            d.part = at[c].part + 2 * (size_t)s.slot_begin * d.tiles * kChipRows;
+            d.width = jobs[c].width;
+            d.flags = CHIP_STORE;
+        };
+        struct Level {
+            size_t first;
+            uint32_t count;
+        };
+        std::vector<Level> levels_f, levels_r;
+        size_t k = 0;
+        for (size_t l = 0; l < lf; l++) {
+            levels_f.push_back({k, 0});
+            for (uint32_t c = 0; c < count; c++)
+                if (l < fwd[c].sweeps.size()) {
+                    fill(hf[k], c, fwd[c].sweeps[l], at[c].fwd);
+                    if (l == 0) hf[k].flags |= CHIP_INIT;
+                    k++;
+                }
+            levels_f.back().count = (uint32_t)(k - levels_f.back().first);
+        }
+        k = 0;
+        for (size_t l = 0; l < lr; l++) {
+            levels_r.push_back({k, 0});
+            for (uint32_t c = 0; c < count; c++)
+                if (l < rev[c].sweeps.size()) {
+                    fill(hr[k], c, rev[c].sweeps[l], at[c].rev);
+                    if (l + 1 == rev[c].sweeps.size()) hr[k].flags = 0;  // only its sums are used
+                    k++;
+                }
+            levels_r.back().count = (uint32_t)(k - levels_r.back().first);
+        }
+        hipStream_t st = rt().stream;
+        SPZ_HIP(hipEventRecord(begin, st));
+        SPZ_HIP(hipMemcpyAsync(slot.dev, slot.host, total, hipMemcpyHostToDevice, st));
+        int rc = SPZ_OK;
+        for (const Level &l : levels_f)
+            if (rc == SPZ_OK)
+                rc = launch_chip_sweeps(SPZ_F64, false, (const ChipSweep *)(slot.dev + o_f) + l.first,
+                                        l.count, width, lds);
+        if (rc == SPZ_OK)
+            rc = launch_chip_ising(SPZ_F64, (const ChipIsing *)(slot.dev + o_i), count, blocks, hx);
+        for (const Level &l : levels_r)
+            if (rc == SPZ_OK)
+                rc = launch_chip_sweeps(SPZ_F64, true, (const ChipSweep *)(slot.dev + o_r) + l.first,
+                                        l.count, width, lds);
+        if (rc == SPZ_OK)
+            rc = launch_chip_sums((const ChipSum *)(slot.dev + o_s), (uint32_t)ns,
+                                  (double *)sc.out.p);
+        SPZ_HIP(hipEventRecord(end, st));
+        SPZ_HIP(hipEventRecord(slot.done, st));
+        slot.busy = true;
+        return rc;
+    }
+};
 
 }  // namespace
 
@@ -585,15 +334,16 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
     SPZ_TRY(ensure_init());
     if (count == 0) return SPZ_OK;
     if (!circuits || !ops || !energies || !grads) return fail(SPZ_ERR_ARG, "null argument");
-    int wg_max = opts && opts->wg_max_qubits > 0 ? opts->wg_max_qubits
-                                                 : (g_wg_max_qubits > 0 ? g_wg_max_qubits : 14);
-    const int use_graph = opts ? opts->use_graph : 1;
-    // circuits above gq qubits run on groups of workgroups (gq >= 8 keeps
-    // every member's share of every gate's pairs non-empty)
+    const int wg_max = opts && opts->wg_max_qubits > 0
+                           ? opts->wg_max_qubits
+                           : (g_wg_max_qubits > 0 ? g_wg_max_qubits : 14);
+    // circuits above gq qubits run on 2^(n - gq) workgroups (at most one per tile)
     const int gq_opt = opts ? opts->group_qubits : 0;
-    const int gq = gq_opt < 0 ? 64 : (gq_opt == 0 ? 12 : std::max(gq_opt, 8));
-    std::vector<uint64_t> small, large;
-    uint64_t total_ops = 0;
+    const int gq = gq_opt < 0 ? 64 : (gq_opt == 0 ? kChipK : std::max(gq_opt, 8));
+    std::vector<Job> small;
+    std::vector<uint64_t> large;
+    int n_group = 0;
+    uint64_t gmax = 0;
     for (uint64_t i = 0; i < count; i++) {
         const spz_batch_circuit &c = circuits[i];
         if (c.n < 1 || c.n > 30 || c.n_ops < 0) return fail(SPZ_ERR_ARG, "bad circuit entry");
@@ -607,262 +357,126 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
                 return rc;
             }
         }
-        (c.n <= wg_max ? small : large).push_back(i);
-        total_ops += (uint64_t)c.n_ops;
+        if (c.n > wg_max || c.n > kBatchMaxQubits) {
+            large.push_back(i);
+            continue;
+        }
+        const uint64_t wgs = c.n > gq ? 1ull << (c.n - gq) : 1ull;
+        small.push_back({i, (uint32_t)std::min(wgs, tiles_of(c.n))});
+        n_group += c.n > gq;
+        gmax = std::max<uint64_t>(gmax, c.grad_offset + (uint64_t)c.n_ops);
     }
-    (void)total_ops;
+    if (small.size() + gmax >= 0xFFFFFFFFull) return fail(SPZ_ERR_ARG, "too many gradients");
     auto t0 = std::chrono::steady_clock::now();
     std::vector<double> lat(count, 0.0);
-    // ---- routing: circuits above group_qubits run on 2^(n - group_qubits)
-    // workgroups of one XCD; a group may take up to all of an XCD's resident
-    // workgroups (larger ones take the single-circuit path).  The grid never
-    // exceeds what is resident at once, and tickets are handed out in order,
-    // so a group's missing members are workgroups still finishing earlier
-    // tickets, none of which waits on a later one: every group fills.
-    int occ = 0;
-    SPZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_batch_adjoint, kW, 0));
-    // resident workgroups per CU (default 2): with fewer circuits sharing a CU a
-    // group's members keep pace with each other (1024 circuits, n 10..20, with
-    // groups up to a whole XCD: p99 87 -> 16 ms, 214k -> 253k grads/s)
-    const int cap = opts && opts->wg_per_cu != 0 ? opts->wg_per_cu : kWgPerCu;
-    if (cap > 0) occ = std::min(occ, cap);
-    const uint64_t grid = (uint64_t)rt().cu_count * std::max(occ, 1);
-    const int nx = (gq < 64 && !small.empty()) ? xcd_count() : 0;
-    const uint32_t nq = nx > 0 ? (uint32_t)nx : 1u;
-    const uint64_t per_q = grid / nq;
-    auto members = [&](int n) -> uint64_t { return (nx > 0 && n > gq) ? (1ull << (n - gq)) : 1ull; };
-    {
-        std::vector<uint64_t> keep;
-        for (uint64_t i : small) {
-            if (members(circuits[i].n) > 1 && members(circuits[i].n) > per_q) large.push_back(i);
-            else keep.push_back(i);
-        }
-        small.swap(keep);
+    // ---- circuits up to the switch point, largest first: circuits of one size
+    // share chunks, and the first chunk keeps the GPU busy longest
+    std::stable_sort(small.begin(), small.end(), [&](const Job &x, const Job &y) {
+        const spz_batch_circuit &a = circuits[x.circuit], &b = circuits[y.circuit];
+        return a.n != b.n ? a.n > b.n : a.n_ops > b.n_ops;
+    });
+    Scratch &sc = scratch();
+    // wg_per_cu > 0 caps the workgroups resident on a CU by padding their LDS
+    // (160 KiB per CU, 32 KiB used, at most 64 KiB per workgroup)
+    size_t lds = 0;
+    if (opts && opts->wg_per_cu > 0) {
+        const size_t share = std::min<size_t>(64 << 10, (160u << 10) / (size_t)opts->wg_per_cu);
+        lds = share > (32u << 10) ? share - (32u << 10) : 0;
     }
-    // ---- larger circuits: pre-size everything they need, so that no
-    // allocation or free (which would synchronise the device) happens while
-    // the small-circuit kernel runs beside them
+    int rc = SPZ_OK;
+    std::vector<size_t> first;  // first job of every chunk
+    if (!small.empty()) {
+        rc = sc.out.need((small.size() + gmax) * sizeof(double));
+        // (the gradients of ops without a parameter stay zero)
+        if (rc == SPZ_OK && hipMemsetAsync(sc.out.p, 0, (small.size() + gmax) * sizeof(double),
+                                           rt().stream) != hipSuccess)
+            rc = fail(SPZ_ERR_HIP, "batched adjoint clear failed");
+        Chunk ch{circuits, ops, hx, lds, small.size()};
+        for (size_t a = 0; rc == SPZ_OK && a < small.size();) {
+            size_t b = a;
+            uint64_t tiles = 0, nops = 0;
+            while (b < small.size()) {
+                const spz_batch_circuit &c = circuits[small[b].circuit];
+                tiles += tiles_of(c.n);
+                nops += 2 * (uint64_t)c.n_ops;
+                if (b > a && (tiles > kChunkTiles || nops > kChunkOps)) break;
+                b++;
+            }
+            const size_t k = first.size();
+            while (rc == SPZ_OK && sc.events.size() < 2 * (k + 1)) {
+                hipEvent_t e;
+                if (hipEventCreate(&e) != hipSuccess) rc = fail(SPZ_ERR_HIP, "event creation failed");
+                else sc.events.push_back(e);
+            }
+            if (rc == SPZ_OK)
+                rc = ch.run(&small[a], (uint32_t)(b - a), (uint32_t)a, sc, sc.slots[k & 1],
+                            sc.events[2 * k], sc.events[2 * k + 1]);
+            first.push_back(a);
+            a = b;
+        }
+    }
+    // ---- larger circuits: the single-circuit path, behind them on the stream ------
     std::stable_sort(large.begin(), large.end(),
                      [&](uint64_t x, uint64_t y) { return circuits[x].n < circuits[y].n; });
-    std::vector<spz_state> st_by_n(64, nullptr);
-    auto release = [&]() {
-        for (spz_state &x : st_by_n)
-            if (x) spz_state_destroy(x);
-    };
-    if (!large.empty()) {
-        int nmax = 0;
-        uint64_t opsmax = 0;
-        for (uint64_t i : large) {
-            nmax = std::max(nmax, circuits[i].n);
-            opsmax = std::max<uint64_t>(opsmax, (uint64_t)circuits[i].n_ops);
-        }
-        int rc = adjoint_reserve(nmax, SPZ_F64, opsmax);
-        for (uint64_t i : large)
-            if (rc == SPZ_OK && !st_by_n[circuits[i].n])
-                rc = spz_state_create(circuits[i].n, SPZ_F64, &st_by_n[circuits[i].n]);
-        if (rc != SPZ_OK) {
-            release();
-            return rc;
-        }
-    }
-    // ---- circuits up to the switch point: one persistent launch on the side stream
-    BatchCache &bcache = g_bc;
-    void *d_circ = nullptr, *d_ops = nullptr, *d_scr = nullptr, *d_cnt = nullptr, *d_e = nullptr,
-         *d_g = nullptr, *d_t = nullptr, *d_tk = nullptr, *d_q = nullptr, *d_pool = nullptr,
-         *d_parts = nullptr, *d_err = nullptr;
-    uint64_t gmax = 0;
-    hipStream_t st = side_stream() ? side_stream() : rt().stream;
-    int n_group = 0;
-    if (!small.empty()) {
-        // largest first: the long circuits start at once and the short ones
-        // fill the workgroups that finish early
-        std::stable_sort(small.begin(), small.end(), [&](uint64_t x, uint64_t y) {
-            const double cx = (double)circuits[x].n_ops * (double)(1ull << circuits[x].n);
-            const double cy = (double)circuits[y].n_ops * (double)(1ull << circuits[y].n);
-            return cx > cy;
-        });
-        std::vector<BCirc> bc(small.size());
-        std::vector<BOp> bo;
-        int nmax_single = 1;
-        uint64_t pool = 0, parts = 0;
-        uint32_t nbars = 0;
-        // queues: each circuit to the least-loaded queue, in cost order
-        std::vector<std::vector<BTicket>> qt(nq);
-        std::vector<double> qload(nq, 0.0);
-        for (size_t k = 0; k < small.size(); k++) {
-            const spz_batch_circuit &c = circuits[small[k]];
-            bc[k].n = c.n;
-            bc[k].nops = c.n_ops;
-            bc[k].op0 = bo.size();
-            bc[k].grad0 = c.grad_offset;
-            const uint64_t g = members(c.n);
-            if (g > 1) {
-                bc[k].region = pool;
-                bc[k].bar = nbars++;
-                bc[k].part = parts;
-                pool += 4ull << c.n;
-                parts += ((uint64_t)c.n_ops + 1) * g;
-                n_group++;
-            } else {
-                nmax_single = std::max(nmax_single, c.n);
-            }
-            for (int o = 0; o < c.n_ops; o++) {
-                BOp b;
-                int rc = lower_bop(ops[c.op_offset + o], &b);
-                if (rc != SPZ_OK) {
-                    release();
-                    return rc;
-                }
-                bo.push_back(b);
-            }
-            const uint32_t q = (uint32_t)(std::min_element(qload.begin(), qload.end()) - qload.begin());
-            qload[q] += (double)std::max(c.n_ops, 1) * (double)(1ull << c.n);
-            for (uint64_t m = 0; m < g; m++)
-                qt[q].push_back(BTicket{(uint32_t)k, (uint16_t)m, (uint16_t)g});
-        }
-        std::vector<BTicket> tk;
-        std::vector<uint32_t> qs(2 * nq);
-        for (uint32_t q = 0; q < nq; q++) {
-            qs[q] = (uint32_t)tk.size();
-            qs[nq + q] = (uint32_t)qt[q].size();
-            tk.insert(tk.end(), qt[q].begin(), qt[q].end());
-        }
-        const uint64_t slot = 1ull << nmax_single;
-        const uint64_t grid_used = std::min<uint64_t>(grid, nq == 1 ? tk.size() : grid);
-        // scratch: 4 arrays of 2^nmax doubles per workgroup for the one-workgroup circuits
-        const uint64_t scratch_bytes = grid_used * 4 * slot * sizeof(double);
-        for (uint64_t i : small) gmax = std::max<uint64_t>(gmax, circuits[i].grad_offset + circuits[i].n_ops);
-        const uint32_t ncnt = nq + nbars;
-        BatchCache &B = bcache;
-        if (!grow(B.circ, bc.size() * sizeof(BCirc)) || !grow(B.ops, bo.size() * sizeof(BOp)) ||
-            !grow(B.scr, scratch_bytes) || !grow(B.cnt, ncnt * sizeof(unsigned int)) ||
-            !grow(B.err, sizeof(int)) || !grow(B.tk, tk.size() * sizeof(BTicket)) ||
-            !grow(B.q, qs.size() * sizeof(uint32_t)) || !grow(B.pool, pool * sizeof(double)) ||
-            !grow(B.parts, 2 * parts * sizeof(double)) || !grow(B.e, small.size() * sizeof(double)) ||
-            !grow(B.g, gmax * sizeof(double)) ||
-            !grow(B.t, small.size() * 2 * sizeof(unsigned long long))) {
-            release();
-            return fail(SPZ_ERR_OOM, "batched adjoint scratch allocation failed");
-        }
-        d_circ = B.circ.p; d_ops = B.ops.p; d_scr = B.scr.p; d_cnt = B.cnt.p; d_err = B.err.p;
-        d_tk = B.tk.p; d_q = B.q.p; d_pool = B.pool.p; d_parts = B.parts.p; d_e = B.e.p;
-        d_g = B.g.p; d_t = B.t.p;
-        // the gradient slots of parameter-free ops stay zero
-        std::vector<double> zeros(std::max<uint64_t>(gmax, 1), 0.0);
-        if (hipMemcpy(d_circ, bc.data(), bc.size() * sizeof(BCirc), hipMemcpyHostToDevice) != hipSuccess ||
-            (bo.size() && hipMemcpy(d_ops, bo.data(), bo.size() * sizeof(BOp), hipMemcpyHostToDevice) != hipSuccess) ||
-            hipMemcpy(d_tk, tk.data(), tk.size() * sizeof(BTicket), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(d_q, qs.data(), qs.size() * sizeof(uint32_t), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(d_g, zeros.data(), zeros.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
-            release();
-            return fail(SPZ_ERR_HIP, "batched adjoint upload failed");
-        }
-        auto launch = [&]() {
-            hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, st, (unsigned int *)d_cnt, ncnt,
-                               (int *)d_err);
-            hipLaunchKernelGGL(k_batch_adjoint, dim3((unsigned)grid_used), dim3(kW), 0, st,
-                               (const BCirc *)d_circ, (const BTicket *)d_tk,
-                               (const uint32_t *)d_q, (const uint32_t *)d_q + nq, nq,
-                               (const BOp *)d_ops, hx, (double *)d_scr, slot, (double *)d_pool,
-                               (double *)d_parts, (unsigned int *)d_cnt, (int *)d_err,
-                               (double *)d_e, (double *)d_g, (unsigned long long *)d_t);
-        };
-        bool ok = true;
-        if (use_graph) {
-            // the captured launch is reused while every argument is the same
-            uint64_t hxb;
-            memcpy(&hxb, &hx, sizeof hxb);
-            std::vector<uint64_t> key = {grid_used, nq, ncnt, slot, hxb,
-                                         (uint64_t)(uintptr_t)d_circ, (uint64_t)(uintptr_t)d_ops,
-                                         (uint64_t)(uintptr_t)d_scr, (uint64_t)(uintptr_t)d_cnt,
-                                         (uint64_t)(uintptr_t)d_err, (uint64_t)(uintptr_t)d_tk,
-                                         (uint64_t)(uintptr_t)d_q, (uint64_t)(uintptr_t)d_pool,
-                                         (uint64_t)(uintptr_t)d_parts, (uint64_t)(uintptr_t)d_e,
-                                         (uint64_t)(uintptr_t)d_g, (uint64_t)(uintptr_t)d_t};
-            if (!(B.exec && B.key == key)) {
-                if (B.exec) (void)hipGraphExecDestroy(B.exec);
-                if (B.graph) (void)hipGraphDestroy(B.graph);
-                B.exec = nullptr;
-                B.graph = nullptr;
-                B.key.clear();
-                ok = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) == hipSuccess;
-                if (ok) {
-                    launch();
-                    ok = hipStreamEndCapture(st, &B.graph) == hipSuccess;
-                }
-                if (ok) ok = hipGraphInstantiate(&B.exec, B.graph, nullptr, nullptr, 0) == hipSuccess;
-                if (ok) B.key = key;
-            }
-            if (ok) ok = hipGraphLaunch(B.exec, st) == hipSuccess;
-        } else {
-            launch();
-            ok = hipGetLastError() == hipSuccess;
-        }
-        if (!ok) {
-            (void)hipGetLastError();
-            (void)hipStreamSynchronize(st);
-            if (B.exec) (void)hipGraphExecDestroy(B.exec);
-            if (B.graph) (void)hipGraphDestroy(B.graph);
-            B.exec = nullptr;
-            B.graph = nullptr;
-            B.key.clear();
-            release();
-            return fail(SPZ_ERR_HIP, "batched adjoint launch failed");
-        }
-    }
-    // ---- larger circuits: the single-circuit path on the library stream -----------
-    int rc_large = SPZ_OK;
+    spz_state st = nullptr;
+    int st_n = 0;
     for (uint64_t i : large) {
+        if (rc != SPZ_OK) break;
         const spz_batch_circuit &c = circuits[i];
-        spz_state s = st_by_n[c.n];
-        int rc = spz_state_set_basis(s, 0);
         auto a = std::chrono::steady_clock::now();
-        if (rc == SPZ_OK)
-            rc = adjoint_grad(s, ops + c.op_offset, (uint64_t)c.n_ops, hx, 0, grads + c.grad_offset,
-                              &energies[i], nullptr);
-        auto b = std::chrono::steady_clock::now();
-        if (rc != SPZ_OK) {
-            rc_large = rc;
-            break;
+        if (c.n != st_n) {
+            if (st) spz_state_destroy(st);
+            st = nullptr;
+            st_n = 0;
+            rc = spz_state_create(c.n, SPZ_F64, &st);
+            if (rc == SPZ_OK) st_n = c.n;
+        } else {
+            rc = spz_state_set_basis(st, 0);
         }
+        if (rc == SPZ_OK)
+            rc = adjoint_grad(st, ops + c.op_offset, (uint64_t)c.n_ops, hx, 0,
+                              grads + c.grad_offset, &energies[i], nullptr);
+        auto b = std::chrono::steady_clock::now();
         lat[i] = std::chrono::duration<double, std::milli>(b - a).count();
     }
-    // ---- collect the small circuits ---------------------------------------------
-    int rc_small = SPZ_OK;
-    if (!small.empty()) {
-        if (hipStreamSynchronize(st) != hipSuccess) rc_small = fail(SPZ_ERR_HIP, "batched adjoint kernel failed");
-        int kerr = 0;
-        if (rc_small == SPZ_OK &&
-            (hipMemcpy(&kerr, d_err, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess || kerr))
-            rc_small = fail(SPZ_ERR_HIP, "batched adjoint: a workgroup group barrier timed out");
-        if (rc_small == SPZ_OK) {
-            std::vector<double> e(small.size()), g(std::max<uint64_t>(gmax, 1));
-            std::vector<unsigned long long> t(2 * small.size());
-            if (hipMemcpy(e.data(), d_e, e.size() * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess ||
-                hipMemcpy(g.data(), d_g, g.size() * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess ||
-                hipMemcpy(t.data(), d_t, t.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost) != hipSuccess)
-                rc_small = fail(SPZ_ERR_HIP, "batched adjoint download failed");
-            int clk_khz = 100000;  // wall_clock64 runs at 100 MHz on gfx9
-            (void)hipDeviceGetAttribute(&clk_khz, hipDeviceAttributeWallClockRate, rt().device);
-            for (size_t k = 0; rc_small == SPZ_OK && k < small.size(); k++) {
-                const uint64_t i = small[k];
-                energies[i] = e[k];
+    if (st) spz_state_destroy(st);
+    // ---- collect -----------------------------------------------------------------
+    if (hipStreamSynchronize(rt().stream) != hipSuccess && rc == SPZ_OK)
+        rc = fail(SPZ_ERR_HIP, "batched adjoint failed");
+    if (rc == SPZ_OK && !small.empty()) {
+        std::vector<double> out(small.size() + gmax);
+        if (hipMemcpy(out.data(), sc.out.p, out.size() * sizeof(double), hipMemcpyDeviceToHost) !=
+            hipSuccess)
+            rc = fail(SPZ_ERR_HIP, "batched adjoint download failed");
+        for (size_t k = 0; rc == SPZ_OK && k < first.size(); k++) {
+            float ms = 0.f;  // a circuit's time is its chunk's
+            (void)hipEventElapsedTime(&ms, sc.events[2 * k], sc.events[2 * k + 1]);
+            const size_t b = k + 1 < first.size() ? first[k + 1] : small.size();
+            for (size_t j = first[k]; j < b; j++) {
+                const uint64_t i = small[j].circuit;
                 const spz_batch_circuit &c = circuits[i];
-                for (int o = 0; o < c.n_ops; o++) grads[c.grad_offset + o] = g[c.grad_offset + o];
-                lat[i] = (double)(t[2 * k + 1] - t[2 * k]) / (double)clk_khz;  // ms
+                energies[i] = out[j];
+                if (c.n_ops)
+                    memcpy(grads + c.grad_offset, out.data() + small.size() + c.grad_offset,
+                           (size_t)c.n_ops * sizeof(double));
+                lat[i] = ms;
             }
         }
     }
-    release();
-    if (rc_large != SPZ_OK) return rc_large;
-    if (rc_small != SPZ_OK) return rc_small;
+    if (sc.states.cap + sc.parts.cap + sc.out.cap + sc.slots[0].cap + sc.slots[1].cap > kKeep) {
+        for (Buf *b : {&sc.states, &sc.parts, &sc.out}) b->drop();
+        for (Slot &s : sc.slots) {
+            s.busy = false;  // (the stream was waited for)
+            s.drop();
+        }
+    }
+    if (rc != SPZ_OK) return rc;
     auto t1 = std::chrono::steady_clock::now();
     if (stats) {
-        std::vector<double> l = lat;
-        std::sort(l.begin(), l.end());
+        std::sort(lat.begin(), lat.end());
         stats->total_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
-        stats->p50_ms = l[(size_t)(0.50 * (l.size() - 1))];
-        stats->p99_ms = l[(size_t)(0.99 * (l.size() - 1))];
+        stats->p50_ms = lat[(size_t)(0.50 * (lat.size() - 1))];
+        stats->p99_ms = lat[(size_t)(0.99 * (lat.size() - 1))];
         stats->n_small = small.size();
         stats->n_large = large.size();
         stats->wg_max_qubits = wg_max;
@@ -874,19 +488,11 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
 int spz_batch_autotune(const spz_batch_circuit *circuits, uint64_t count, const spz_op *ops,
                        int *wg_max_qubits)
 {
-    // For every qubit count present: run up to 8 of its circuits concurrently
-    // in the persistent kernel (per-circuit latency L_wg) and one at a time on
-    // the single-circuit path (T_single each).  With m circuits of that size
-    // in the batch and `slots` resident workgroups, the persistent kernel needs
-    // about ceil(m / slots) * L_wg, the single path m * T_single.  The switch
-    // point is the largest n for which the persistent kernel wins.
+    // For every qubit count present: run up to 8 of its circuits batched and
+    // one at a time; the switch point is the largest n for which the batch wins.
     SPZ_API_LOCK;
     SPZ_TRY(ensure_init());
     if (!circuits || !ops) return fail(SPZ_ERR_ARG, "null argument");
-    int occ = 0;
-    SPZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_batch_adjoint, kW, 0));
-    occ = std::min(occ, kWgPerCu);  // the trial batches run with the default
-    const double slots = (double)rt().cu_count * std::max(occ, 1);
     std::vector<int> ns;
     for (uint64_t i = 0; i < count; i++) ns.push_back(circuits[i].n);
     std::sort(ns.begin(), ns.end());
@@ -894,12 +500,8 @@ int spz_batch_autotune(const spz_batch_circuit *circuits, uint64_t count, const 
     int best = 0;
     for (int n : ns) {
         std::vector<spz_batch_circuit> pick;
-        double m = 0;
-        for (uint64_t i = 0; i < count; i++)
-            if (circuits[i].n == n) {
-                m += 1;
-                if (pick.size() < 8) pick.push_back(circuits[i]);
-            }
+        for (uint64_t i = 0; i < count && pick.size() < 8; i++)
+            if (circuits[i].n == n) pick.push_back(circuits[i]);
         uint64_t gsz = 0;
         for (auto &c : pick) gsz = std::max<uint64_t>(gsz, c.grad_offset + c.n_ops);
         std::vector<double> e(std::max<uint64_t>(count, 1)), g(std::max<uint64_t>(gsz, 1));
@@ -907,13 +509,17 @@ int spz_batch_autotune(const spz_batch_circuit *circuits, uint64_t count, const 
         memset(&o, 0, sizeof o);
         o.use_graph = 1;
         spz_batch_stats sw, sl;
-        o.wg_max_qubits = 64;  // all in the persistent kernel
-        SPZ_TRY(spz_batch_adjoint(pick.data(), pick.size(), ops, 1.0, e.data(), g.data(), &o, &sw));
-        o.wg_max_qubits = n - 1;  // all on the single-circuit path
-        SPZ_TRY(spz_batch_adjoint(pick.data(), pick.size(), ops, 1.0, e.data(), g.data(), &o, &sl));
-        const double t_wg = std::ceil(m / slots) * sw.p99_ms;
-        const double t_single = m * (sl.total_ms / (double)pick.size());
-        if (t_wg <= t_single) best = n;
+        for (int pass = 0; pass < 2; pass++) {  // (the first sizes the scratch)
+            o.wg_max_qubits = 64;  // batched
+            SPZ_TRY(spz_batch_adjoint(pick.data(), pick.size(), ops, 1.0, e.data(), g.data(), &o,
+                                      &sw));
+            o.wg_max_qubits = n - 1;  // one at a time
+            if (n == 1) sl.total_ms = INFINITY;
+            else
+                SPZ_TRY(spz_batch_adjoint(pick.data(), pick.size(), ops, 1.0, e.data(), g.data(),
+                                          &o, &sl));
+        }
+        if (sw.total_ms <= sl.total_ms) best = n;
     }
     g_wg_max_qubits = best > 0 ? best : 1;
     if (wg_max_qubits) *wg_max_qubits = g_wg_max_qubits;

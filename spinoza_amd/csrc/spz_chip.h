@@ -28,7 +28,9 @@ struct ChipSweep {
     const TileOp *ops;
     double *part;         // gradient pairs: row r of slot k of tile t at
                           // part[2 ((k tiles + t) kChipRows + r)]
-    uint32_t nops, tiles, flags, pad;
+    uint32_t nops, tiles;
+    uint32_t width;       // workgroups of the circuit (they stride over its tiles)
+    uint32_t flags;
     int8_t spos[16];
     int8_t tin[16];
     uint64_t tg[8], gr[16], gs[16];
@@ -52,8 +54,8 @@ struct ChipSum {
 };
 
 // Launches on the library stream: `count` descriptors, of at most `width`
-// tiles (blocks) each; a circuit's workgroups stride over its tiles, `lds` pads
-// their LDS (a cap on how many are resident).
+// workgroups (blocks) each; `lds` pads the workgroups' LDS (a cap on how many
+// are resident).
 int launch_chip_sweeps(int prec, bool reverse, const ChipSweep *d, uint32_t count, uint32_t width,
                        size_t lds);
 int launch_chip_ising(int prec, const ChipIsing *d, uint32_t count, uint32_t width, double hx);

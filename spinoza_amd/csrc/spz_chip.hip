@@ -92,7 +92,8 @@ k_chip(const ChipSweep *__restrict__ sweeps)
     __shared__ double lds[1 << kChipK];
     const uint32_t tid = threadIdx.x;
     const ChipSweep &d = sweeps[blockIdx.y];
-    for (uint32_t tile = blockIdx.x; tile < d.tiles; tile += gridDim.x) {
+    if (blockIdx.x >= d.width) return;
+    for (uint32_t tile = blockIdx.x; tile < d.tiles; tile += d.width) {
         const uint64_t base = insert_zeros((uint64_t)tile, d.spos, kChipK);
         uint32_t lt = 0;
 #pragma unroll
@@ -272,6 +273,7 @@ void chip_geometry(const ChipPlan::Sweep &s, int n, int prec, ChipSweep &out)
     for (int i = 0; i < 8; i++) out.tg[i] = s.desc.tg[i];
     out.limit = 1ull << n;
     out.tiles = n > kChipK ? 1u << (n - kChipK) : 1u;
+    out.width = out.tiles;
     out.nops = s.op_count;
 }
 
