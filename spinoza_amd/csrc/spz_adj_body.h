@@ -256,20 +256,6 @@ __device__ __forceinline__ void adj_diag_lane_kinds(uint32_t gr, const Amps &s, 
     if (hit(gr & TG_RZ)) adj_diag_lane<R, AK_RZ, PRED>(s, k, bit, pm, g);
 }
 
-// One op, fetched whole into scalar registers off a uniform address (as in
-// k_tile).
-__device__ __forceinline__ TileOp fetch_op(uint64_t opa)
-{
-    const __attribute__((address_space(4))) uint64_t *w =
-        reinterpret_cast<const __attribute__((address_space(4))) uint64_t *>(opa);
-    uint64_t x[sizeof(TileOp) / 8];
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(TileOp) / 8); i++) x[i] = w[i];
-    TileOp op;
-    __builtin_memcpy(&op, x, sizeof(TileOp));
-    return op;
-}
-
 // An LDS change of layout: set() forms the addresses, move() takes one
 // register array through it.
 template <int R, int LOGW>

@@ -57,31 +57,6 @@ __device__ __forceinline__ void fwd_gate(const TileOp &cur, uint64_t base, uint3
     }
 }
 
-// With one workgroup to a CU nothing hides the op records' latency: a record is
-// two cold scalar lines, from HBM the first time (0.4 us of the 0.74 us that an
-// op took).  So the workgroup first pulls the program into the L2 with vector
-// loads, and each op touches the next one's lines while it runs.
-__device__ __forceinline__ void warm_program(const TileOp *ops, uint32_t nops, uint32_t tid)
-{
-    const char *p = reinterpret_cast<const char *>(ops);
-    uint32_t x = 0;
-    for (uint64_t o = (uint64_t)tid * 64; o < (uint64_t)nops * sizeof(TileOp); o += 64ull << kLogW)
-        x ^= *reinterpret_cast<const volatile uint32_t *>(p + o);
-    asm volatile("" ::"v"(x));
-}
-
-// One word of each line of the next op (the last op touches itself again),
-// loaded after the wait for this one.
-__device__ __forceinline__ uint64_t touch_next(const TileOp &cur, uint64_t opa, uint64_t ope)
-{
-    uint64_t nx = opa + sizeof(TileOp);
-    if (nx == ope) nx = opa;
-    asm volatile("" : "+s"(nx) : "s"(cur.grp));
-    const __attribute__((address_space(4))) uint32_t *w =
-        reinterpret_cast<const __attribute__((address_space(4))) uint32_t *>(nx);
-    return w[0] ^ ((uint64_t)w[16] << 32);
-}
-
 // Reverse sweeps hold two states (three waves per SIMD, as k_adj_tile),
 // forward sweeps one (four).
 template <typename T, bool REV>
@@ -126,7 +101,7 @@ k_chip(const ChipSweep *__restrict__ sweeps)
             }
         }
         const uint64_t ope = reinterpret_cast<uint64_t>(d.ops + d.nops);
-        warm_program(d.ops, d.nops, tid);
+        warm_program<kLogW>(d.ops, d.nops, tid);
         for (uint64_t opa = reinterpret_cast<uint64_t>(d.ops); opa != ope; opa += sizeof(TileOp)) {
             asm volatile("" : "+s"(opa));
             const TileOp cur = fetch_op(opa);

@@ -339,10 +339,59 @@ __device__ __forceinline__ uint64_t lane_offset(uint32_t x, const uint64_t *t)
     return ((uint64_t)hi << 32) | lo;
 }
 
+// One op, fetched whole into scalar registers off a uniform address (by
+// value, through the constant address space: its fields are scalar loads at
+// immediate offsets of one base that advances by one add per op, and selects
+// between its coefficients are value selects, never per-lane loads).
+__device__ __forceinline__ TileOp fetch_op(uint64_t opa)
+{
+    const __attribute__((address_space(4))) uint64_t *w =
+        reinterpret_cast<const __attribute__((address_space(4))) uint64_t *>(opa);
+    uint64_t x[sizeof(TileOp) / 8];
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(TileOp) / 8); i++) x[i] = w[i];
+    TileOp op;
+    __builtin_memcpy(&op, x, sizeof(TileOp));
+    return op;
+}
+
+// With few workgroups to a CU nothing hides the op records' latency: a record
+// is two cold scalar lines, from HBM the first time (0.2 to 0.4 us of an op's
+// 0.6).  So the workgroup first pulls the program into the L2 with vector
+// loads, and each op touches the next one's lines while it runs: a sweep of 17
+// qubits (32 tiles, about 60 gates) 37.6 -> 27 us, of the 20-qubit QFT (256
+// tiles) 68 -> 50; circuits of one tile, 152 gates, 127 -> 81 forward and 190 ->
+// 140 in reverse (spz_chip.hip).  k_tile does it up to kWarmTiles workgroups,
+// what is resident at once: with more of them the records stay in the scalar
+// caches and touching costs 1.3% (30 qubits).
+template <int LOGW>
+__device__ __forceinline__ void warm_program(const TileOp *ops, uint32_t nops, uint32_t tid)
+{
+    const char *p = reinterpret_cast<const char *>(ops);
+    uint32_t x = 0;
+    for (uint64_t o = (uint64_t)tid * 64; o < (uint64_t)nops * sizeof(TileOp); o += 64ull << LOGW)
+        x ^= *reinterpret_cast<const volatile uint32_t *>(p + o);
+    asm volatile("" ::"v"(x));
+}
+
+// One word of each line of the next op (the last op touches itself again),
+// loaded after the wait for this one.
+__device__ __forceinline__ uint64_t touch_next(const TileOp &cur, uint64_t opa, uint64_t ope)
+{
+    uint64_t nx = opa + sizeof(TileOp);
+    if (nx == ope) nx = opa;
+    asm volatile("" : "+s"(nx) : "s"(cur.grp));
+    const __attribute__((address_space(4))) uint32_t *w =
+        reinterpret_cast<const __attribute__((address_space(4))) uint32_t *>(nx);
+    return w[0] ^ ((uint64_t)w[16] << 32);
+}
+
 // Register budget: asking for 6 waves per SIMD makes the compiler fit the
 // kernel in ~108 VGPRs without spills (4 resident waves per SIMD instead of 3
 // at its unconstrained 138); the extra wave lets one workgroup's loads and
 // stores overlap the others' gate arithmetic.
+constexpr uint32_t kWarmTiles = 1024;
+
 template <typename T, int K, int LOGW, bool FAST>
 __global__ void __launch_bounds__(1 << LOGW) __attribute__((amdgpu_waves_per_eu(6, 6)))
 k_tile(T *__restrict__ re, T *__restrict__ im, const TileDesc d, const TileOp *__restrict__ ops)
@@ -376,22 +425,13 @@ k_tile(T *__restrict__ re, T *__restrict__ im, const TileDesc d, const TileOp *_
     }
 
     const uint64_t ope = reinterpret_cast<uint64_t>(ops + d.nops);
+    const bool few = gridDim.x <= kWarmTiles;
+    if (few) warm_program<LOGW>(ops, (uint32_t)d.nops, tid);
     for (uint64_t opa = reinterpret_cast<uint64_t>(ops); opa != ope; opa += sizeof(TileOp)) {
-        // by value: the op's fields come into scalar registers, so selects
-        // between its coefficients are value selects, never per-lane loads.
-        // The opaque address read through the constant address space gives
-        // scalar loads at immediate offsets of one base that advances by one
-        // add per op (not strength-reduced bases per field).
         asm volatile("" : "+s"(opa));
-        TileOp cur;
-        {
-            const __attribute__((address_space(4))) uint64_t *q =
-                reinterpret_cast<const __attribute__((address_space(4))) uint64_t *>(opa);
-            uint64_t w[sizeof(TileOp) / 8];
-#pragma unroll
-            for (int i = 0; i < (int)(sizeof(TileOp) / 8); i++) w[i] = q[i];
-            __builtin_memcpy(&cur, w, sizeof(TileOp));
-        }
+        const TileOp cur = fetch_op(opa);
+        uint64_t ahead = 0;
+        if (hit(few)) ahead = touch_next(cur, opa, ope);
         const uint32_t g = cur.grp;
         if (hit(g & TG_ANYLAYOUT)) {
         if (hit(g & (TG_SW16 | TG_SW32))) {
@@ -465,6 +505,7 @@ k_tile(T *__restrict__ re, T *__restrict__ im, const TileDesc d, const TileOp *_
                 }
             }
         }
+        asm volatile("" ::"s"(ahead));
     }
 
     // store layout: the lane part is where the last layout change left it;
