@@ -24,11 +24,16 @@ int launch_adj_sum(const double *part, uint64_t tiles, const uint32_t *d_idx, in
 // (more than one tile; a smaller one needs 2 kChipRows doubles per op).
 inline size_t adj_part_bytes(uint64_t N) { return (N >> kAdjK) * kAdjSlots * 2 * sizeof(double); }
 
-// Undo ops[lo, hi) (validated, hi > lo) on psi, whose
+// Undo ops[lo, hi) (validated, hi > lo, FP64 states) on psi, whose
 // amplitudes are taken from src (another state or psi itself), and on lam, and
 // write dE/dtheta of each parametric one to the device array grad[0, hi).
 int adjoint_undo(const spz_state_s *src, spz_state_s *psi, spz_state_s *lam, const spz_op *ops,
                  uint64_t lo, uint64_t hi, double *part, double *grad);
+
+// The same for FP32 storage (spz_adj_group.hip), in place, and its scratch.
+int adjoint_undo_groups(spz_state_s *psi, spz_state_s *lam, const spz_op *ops, uint64_t lo,
+                        uint64_t hi, double *part, double *grad);
+size_t adj_group_part_bytes(uint64_t N);
 
 // The inverse of one op.
 spz_op inverse_op(const spz_op &o);

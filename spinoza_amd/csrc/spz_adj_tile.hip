@@ -113,7 +113,8 @@ int launch_adj_tile(const spz_state_s *src, spz_state_s *psi, spz_state_s *lam, 
     const uint64_t tiles = psi->N >> kAdjK;
     if (tiles == 0 || tiles > (1ull << 31) - 1) return fail(SPZ_ERR_ARG, "tile grid out of range");
     if (slots < 0 || slots > kAdjSlots) return fail(SPZ_ERR_ARG, "too many gradients in a sweep");
-    const size_t esz = psi->prec == SPZ_F64 ? sizeof(double) : sizeof(float);
+    if (psi->prec != SPZ_F64) return fail(SPZ_ERR_ARG, "reverse sweeps take FP64 states");
+    const size_t esz = sizeof(double);
     TileDesc db = d;  // register terms as byte offsets
     for (int p = 0; p < 16; p++) {
         db.gr[p] *= esz;
@@ -121,13 +122,9 @@ int launch_adj_tile(const spz_state_s *src, spz_state_s *psi, spz_state_s *lam, 
     }
     LaunchTimer tm(SPZ_K_ADJOINT, 8.0 * (double)psi->N * (double)esz);
     const dim3 g((unsigned)tiles), b(1 << (kAdjK - 4));
-#define SPZ_ADJ(T)                                                                          \
-    hipLaunchKernelGGL((k_adj_tile<T, kAdjK>), g, b, 0, rt().stream, (const T *)src->re,      \
-                       (const T *)src->im, (T *)psi->re, (T *)psi->im, (T *)lam->re,          \
-                       (T *)lam->im, db, d_ops, slots, part)
-    if (psi->prec == SPZ_F64) SPZ_ADJ(double);
-    else SPZ_ADJ(float);
-#undef SPZ_ADJ
+    hipLaunchKernelGGL((k_adj_tile<double, kAdjK>), g, b, 0, rt().stream, (const double *)src->re,
+                       (const double *)src->im, (double *)psi->re, (double *)psi->im,
+                       (double *)lam->re, (double *)lam->im, db, d_ops, slots, part);
     SPZ_HIP(hipGetLastError());
     return SPZ_OK;
 }

@@ -9,7 +9,7 @@
 //
 // Reverse sweep.  Both states are undone together in tile sweeps
 // (spz_adj_tile.hip; states of at most 12 qubits are one tile and take one
-// launch, spz_chip.hip).
+// launch, spz_chip.hip); FP32 states in groups of gates (spz_adj_group.hip).
 #include <math.h>
 #include <string.h>
 
@@ -202,8 +202,10 @@ struct AdjScratch {
 
 size_t grad_bytes(uint64_t n_ops) { return std::max<uint64_t>(n_ops, 1) * sizeof(double); }
 
-size_t part_bytes(uint64_t N, uint64_t n_ops)
+size_t part_bytes(const spz_state_s *s, uint64_t n_ops)
 {
+    const uint64_t N = s->N;
+    if (s->prec == SPZ_F32) return adj_group_part_bytes(N);
     if (N > (1ull << kAdjK)) return adj_part_bytes(N);
     return std::max<uint64_t>(n_ops, 1) * 2 * kChipRows * sizeof(double);
 }
@@ -260,6 +262,11 @@ int adjoint_grad(spz_state_s *s, const spz_op *ops, uint64_t n_ops, double hx, i
     spz_exec_opts eo;
     memset(&eo, 0, sizeof eo);
     eo.mode = SPZ_EXEC_AUTO;
+    const bool f32 = s->prec == SPZ_F32;
+    if (f32 && s->n <= kChipK) {  // FP32: the rounding points stay (spz_adj_group.hip)
+        if (s->n <= 10) eo.mode = SPZ_EXEC_PLAIN;
+        else eo.tile_qubits = s->n - 1;
+    }
     const uint64_t step = ckpt_every > 0 ? (uint64_t)ckpt_every : std::max<uint64_t>(n_ops, 1);
     for (uint64_t done = 0; done < n_ops;) {
         const uint64_t len = std::min<uint64_t>(step, n_ops - done);
@@ -275,7 +282,7 @@ int adjoint_grad(spz_state_s *s, const spz_op *ops, uint64_t n_ops, double hx, i
     }
     // ---- lambda = H psi, energy (read with the gradients at the end) ----------
     SPZ_TRY(sc.states_like(s));
-    SPZ_TRY(sc.buffers(grad_bytes(n_ops), part_bytes(s->N, n_ops)));
+    SPZ_TRY(sc.buffers(grad_bytes(n_ops), part_bytes(s, n_ops)));
     spz_state_s *const wk = &sc.work, *const lm = &sc.lam;  // psi copy, lambda
     const double amp = s->prec == SPZ_F64 ? 16.0 : 8.0;
     double *const e_out = rt().h_result + (kResults - 1);
@@ -294,7 +301,12 @@ int adjoint_grad(spz_state_s *s, const spz_op *ops, uint64_t n_ops, double hx, i
     for (size_t seg = ckpts.size() + 1; seg-- > 0 && n_ops;) {
         const uint64_t lo = seg ? ckpt_at[seg - 1] + 1 : 0;
         const uint64_t hi = seg < ckpts.size() ? ckpt_at[seg] + 1 : n_ops;
-        SPZ_TRY(adjoint_undo(src, wk, lm, ops, lo, hi, part, gdev));
+        if (f32) {
+            SPZ_TRY(spz_state_copy(wk, const_cast<spz_state_s *>(src)));
+            SPZ_TRY(adjoint_undo_groups(wk, lm, ops, lo, hi, part, gdev));
+        } else {
+            SPZ_TRY(adjoint_undo(src, wk, lm, ops, lo, hi, part, gdev));
+        }
         if (!seg) break;
         // wk holds the uncomputed psi: compare it with the checkpoint, go on from that
         const spz_state_s *ck = ckpts[seg - 1];

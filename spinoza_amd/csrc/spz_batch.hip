@@ -303,7 +303,7 @@ struct Chunk {
                 rc = launch_chip_sweeps(SPZ_F64, false, (const ChipSweep *)(slot.dev + o_f) + l.first,
                                         l.count, width, lds);
         if (rc == SPZ_OK)
-            rc = launch_chip_ising(SPZ_F64, (const ChipIsing *)(slot.dev + o_i), count, blocks, hx);
+            rc = launch_chip_ising((const ChipIsing *)(slot.dev + o_i), count, blocks, hx);
         for (const Level &l : levels_r)
             if (rc == SPZ_OK)
                 rc = launch_chip_sweeps(SPZ_F64, true, (const ChipSweep *)(slot.dev + o_r) + l.first,

@@ -55,10 +55,10 @@ struct ChipSum {
 
 // Launches on the library stream: `count` descriptors, of at most `width`
 // workgroups (blocks) each; `lds` pads the workgroups' LDS (a cap on how many
-// are resident).
+// are resident).  Reverse sweeps and H psi take FP64 states.
 int launch_chip_sweeps(int prec, bool reverse, const ChipSweep *d, uint32_t count, uint32_t width,
                        size_t lds);
-int launch_chip_ising(int prec, const ChipIsing *d, uint32_t count, uint32_t width, double hx);
+int launch_chip_ising(const ChipIsing *d, uint32_t count, uint32_t width, double hx);
 int launch_chip_sums(const ChipSum *d, uint32_t count, double *out);
 
 // The sweeps of a circuit of validated ops: forward, or the undoing of its ops

@@ -205,25 +205,22 @@ int launch_chip_sweeps(int prec, bool reverse, const ChipSweep *d, uint32_t coun
     if (count > 65535) return fail(SPZ_ERR_ARG, "too many circuits in a launch");
     const dim3 g(width, count), b(1 << kLogW);
     hipStream_t st = rt().stream;
-    if (prec == SPZ_F64) {
-        if (reverse) hipLaunchKernelGGL((k_chip<double, true>), g, b, lds, st, d);
-        else hipLaunchKernelGGL((k_chip<double, false>), g, b, lds, st, d);
+    if (reverse) {
+        if (prec != SPZ_F64) return fail(SPZ_ERR_ARG, "reverse sweeps take FP64 states");
+        hipLaunchKernelGGL((k_chip<double, true>), g, b, lds, st, d);
+    } else if (prec == SPZ_F64) {
+        hipLaunchKernelGGL((k_chip<double, false>), g, b, lds, st, d);
     } else {
-        if (reverse) hipLaunchKernelGGL((k_chip<float, true>), g, b, lds, st, d);
-        else hipLaunchKernelGGL((k_chip<float, false>), g, b, lds, st, d);
+        hipLaunchKernelGGL((k_chip<float, false>), g, b, lds, st, d);
     }
     SPZ_HIP(hipGetLastError());
     return SPZ_OK;
 }
 
-int launch_chip_ising(int prec, const ChipIsing *d, uint32_t count, uint32_t width, double hx)
+int launch_chip_ising(const ChipIsing *d, uint32_t count, uint32_t width, double hx)
 {
     if (!count || !width) return SPZ_OK;
-    const dim3 g(width, count), b(kRT);
-    if (prec == SPZ_F64)
-        hipLaunchKernelGGL((k_chip_ising<double>), g, b, 0, rt().stream, d, hx);
-    else
-        hipLaunchKernelGGL((k_chip_ising<float>), g, b, 0, rt().stream, d, hx);
+    hipLaunchKernelGGL((k_chip_ising<double>), dim3(width, count), dim3(kRT), 0, rt().stream, d, hx);
     SPZ_HIP(hipGetLastError());
     return SPZ_OK;
 }
