@@ -1453,10 +1453,6 @@ void gate_matrix2(const Coef &k, double m[8])
     }
 }
 
-// Device buffer for block fragments (grown as needed, reused across calls).
-void *g_dfrag = nullptr;
-size_t g_dfrag_cap = 0;
-
 // Fuse runs of gates acting on at most 5 qubits into dense 32x32 blocks.
 int run_dense5(spz_state_s *s, const std::vector<SG> &run)
 {
@@ -1556,19 +1552,13 @@ int run_dense5(spz_state_s *s, const std::vector<SG> &run)
         }
         block5_fragments(U.data(), s->prec, f64, f32);
     }
-    const size_t bytes = s->prec == SPZ_F64 ? f64.size() * sizeof(double) : f32.size() * sizeof(float);
-    if (bytes) {
-        SPZ_HIP(hipStreamSynchronize(rt().stream));  // the previous fragments may still be in use
-        if (bytes > g_dfrag_cap) {
-            if (g_dfrag) SPZ_HIP(hipFree(g_dfrag));
-            g_dfrag = nullptr;
-            if (hipMalloc(&g_dfrag, bytes) != hipSuccess)
-                return fail(SPZ_ERR_OOM, "block fragment allocation failed");
-            g_dfrag_cap = bytes;
-        }
-        const void *src = s->prec == SPZ_F64 ? (const void *)f64.data() : (const void *)f32.data();
-        SPZ_HIP(hipMemcpyAsync(g_dfrag, src, bytes, hipMemcpyHostToDevice, rt().stream));
-    }
+    // fragments through the program ring: no wait before or after the launches
+    std::lock_guard<std::mutex> lk(g_slot_mu);
+    ProgSlot *slot = nullptr;
+    std::vector<char *> at;
+    const bool any = !f64.empty() || !f32.empty();
+    if (any) SPZ_TRY(upload({s->prec == SPZ_F64 ? bytes_of(f64) : bytes_of(f32)}, &slot, &at));
+    Release release{slot};
     size_t bi = 0;
     const size_t esz = s->prec == SPZ_F64 ? sizeof(double) : sizeof(float);
     for (const Blk &b : blocks) {
@@ -1578,10 +1568,9 @@ int run_dense5(spz_state_s *s, const std::vector<SG> &run)
             else SPZ_TRY(launch_pair(s, g.k, g.target, g.ones, g.zeros));
             continue;
         }
-        SPZ_TRY(launch_block5(s, b.q, (const char *)g_dfrag + bi * 4096 * esz));
+        SPZ_TRY(launch_block5(s, b.q, at[0] + bi * 4096 * esz));
         bi++;
     }
-    if (bytes) SPZ_HIP(hipStreamSynchronize(rt().stream));
     return SPZ_OK;
 }
 
