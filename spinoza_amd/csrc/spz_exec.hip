@@ -1237,6 +1237,15 @@ struct Planner {
             sw.desc.fzg = fr.z & ~smask;
             if (sw.desc.fzl || sw.desc.fzr || sw.desc.fzg) sw.desc.fflags |= TF_SIGN;
             if (w & 1) sw.desc.fflags |= TF_SIGN | TF_ODD;
+            // Without an LDS layout change nothing orders one wavefront's loads
+            // before another's stores: where amplitudes are not stored to the
+            // place their thread loaded, the kernel waits for all loads first.
+            bool lds = false, moved = xl != 0;
+            for (size_t o = sw.op_begin; o < prog.size(); o++) {
+                lds |= (prog[o].grp & TG_LAYOUT) != 0;
+                moved |= (prog[o].grp & (TG_SW16 | TG_SW32)) != 0;
+            }
+            if (moved && !lds) sw.desc.fflags |= TF_SYNC;
             // what a next sweep takes over if this one stores X^x phi only:
             // i^w X^x Z^z = i^(w + 2 |x & z|) Z^z X^x
             sw.can_carry = fast;

@@ -118,7 +118,8 @@ constexpr int kTileMaxR = 32;
 // fzl, on register bits the per-register parity mask fzr (bit p), outside the
 // tile fzg (global bits).  The real sign of w is folded into fzr; an
 // imaginary w (k odd) stores (-im, re).
-enum TileFrameFlags : uint32_t { TF_SIGN = 1u, TF_ODD = 2u, TF_PHASE = 4u };
+// TF_SYNC: every load of the tile lands before the first store.
+enum TileFrameFlags : uint32_t { TF_SIGN = 1u, TF_ODD = 2u, TF_PHASE = 4u, TF_SYNC = 8u };
 
 struct TileDesc {
     int8_t spos[16];          // qubit of local bit i (ascending), K entries

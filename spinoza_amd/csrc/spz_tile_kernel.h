@@ -514,6 +514,10 @@ k_tile(T *__restrict__ re, T *__restrict__ im, const TileDesc d, const TileOp *_
     // bits here, register bits folded into gs[]), the Z part and the phase
     // set its sign, and an imaginary phase stores (-im, re)
     const uint32_t lphi = lt;
+    if (d.fflags & TF_SYNC) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
     if constexpr (FAST) {
         lt ^= d.fxl;
         if (d.fflags & TF_PHASE) {  // the sweep's global factor (phases, H scale)
