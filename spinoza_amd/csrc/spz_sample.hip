@@ -12,10 +12,10 @@
 // dependent loads and additions at memory latency (859 us for 4096 samples of
 // 20 qubits, 734 us for 1000 of 17), with the block sums carried to the host
 // and back and six allocations around it.  Here the samples are counted into
-// their blocks (atomic ranks, one scan, one scatter) and one workgroup per
-// block that has any forms the block's 4096 running sums once in LDS (loads
+// their blocks (atomic ranks, one scan, one scatter) and for every 1024 samples
+// of a block a workgroup forms the block's 4096 running sums in LDS (loads
 // and squares by the whole workgroup, the chain by one lane at the FP64
-// addition latency) and answers all of its samples by bisection: a running
+// addition latency) and answers them by bisection: a running
 // sum of non-negative terms never decreases, so the first one above x is
 // where the walk stopped.  (A NaN or infinite weight makes the total NaN, no
 // sum compares above x, and every sample falls to the last index of positive
@@ -33,11 +33,13 @@ namespace {
 constexpr int kT = 256;
 constexpr uint32_t kBlock = 4096;      // indices per block of the sampling rule
 constexpr uint32_t kPiece = 1u << 20;  // uniforms per round (bounds the scratch)
+constexpr uint32_t kPer = 1024;        // samples a workgroup picks (4 per thread)
+constexpr uint32_t kFew = 64;          // blocks counted in LDS first
 
 struct SampleMeta {
     int64_t lastnz;    // last block with a positive weight (-1: none)
     double total;      // P_nb
-    uint32_t nslots;   // blocks that hold samples of this round
+    uint32_t nslots;   // workgroups' worth of samples of this round
     uint32_t pad;
 };
 
@@ -135,15 +137,25 @@ k_block_prefix(const double *__restrict__ pairs, uint64_t nb, double *__restrict
     }
 }
 
-// The block of every uniform, and its rank among the block's samples.
+// The block of every uniform, and its rank among the block's samples.  With few
+// blocks (kFew) a workgroup counts in LDS and takes its places at once: the
+// samples of a state of one block would queue at one address (10000 samples of
+// 4 qubits: 243 us a call with an atomic each and one workgroup to pick them, 78
+// so and in slots of kPer; 14 qubits 173 -> 108 us).
 __global__ void __launch_bounds__(kT)
 k_sample_block(const double *__restrict__ P, uint64_t nb, const SampleMeta *__restrict__ meta,
                const double *__restrict__ U, uint32_t k, uint32_t *__restrict__ counts,
                uint32_t *__restrict__ blk, uint32_t *__restrict__ rank)
 {
+    __shared__ uint32_t mine[kFew], first[kFew];
     const uint32_t s = blockIdx.x * kT + threadIdx.x;
-    if (s >= k || meta->lastnz < 0) return;
-    const double x = U[s] * meta->total;
+    if (meta->lastnz < 0) return;  // uniform over the grid
+    const bool few = nb <= kFew;
+    if (few) {
+        if (threadIdx.x < kFew) mine[threadIdx.x] = 0u;
+        __syncthreads();
+    }
+    const double x = s < k ? U[s] * meta->total : 0.0;
     uint64_t lo = 0, hi = nb;
     while (lo < hi) {
         const uint64_t mid = lo + (hi - lo) / 2;
@@ -151,12 +163,26 @@ k_sample_block(const double *__restrict__ P, uint64_t nb, const SampleMeta *__re
         else lo = mid + 1;
     }
     const uint32_t b = (uint32_t)(lo < nb ? lo : (uint64_t)meta->lastnz);
+    if (few) {
+        const uint32_t r = s < k ? atomicAdd(&mine[b], 1u) : 0u;
+        __syncthreads();
+        if (threadIdx.x < nb && mine[threadIdx.x])
+            first[threadIdx.x] = atomicAdd(&counts[threadIdx.x], mine[threadIdx.x]);
+        __syncthreads();
+        if (s < k) {
+            blk[s] = b;
+            rank[s] = first[b] + r;
+        }
+        return;
+    }
+    if (s >= k) return;
     blk[s] = b;
     rank[s] = atomicAdd(&counts[b], 1u);
 }
 
 // Exclusive scan of the counts (in place: counts[b] becomes the block's first
-// position) and the list of blocks that hold samples.  One workgroup.
+// position) and the list of the blocks' samples, at most kPer to a slot.  One
+// workgroup.
 __global__ void __launch_bounds__(kPT)
 k_sample_scan(uint32_t *__restrict__ counts, uint64_t nb, Slot *__restrict__ slots,
               SampleMeta *__restrict__ meta)
@@ -167,7 +193,7 @@ k_sample_scan(uint32_t *__restrict__ counts, uint64_t nb, Slot *__restrict__ slo
     for (uint64_t b0 = 0; b0 < nb; b0 += kPT) {
         const uint64_t b = b0 + tid;
         const uint32_t c = b < nb ? counts[b] : 0u;
-        uint32_t s = c, z = c ? 1u : 0u;  // inclusive scans over the wavefront
+        uint32_t s = c, z = (c + kPer - 1) / kPer;  // inclusive scans over the wavefront
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
             const uint32_t us = __shfl_up(s, d), uz = __shfl_up(z, d);
@@ -191,7 +217,9 @@ k_sample_scan(uint32_t *__restrict__ counts, uint64_t nb, Slot *__restrict__ slo
             base_z += wz[w];
         }
         if (b < nb) counts[b] = os + s - c;
-        if (c) slots[oz + z - 1] = Slot{(uint32_t)b, os + s - c, c};
+        const uint32_t nz = (c + kPer - 1) / kPer;
+        for (uint32_t i = 0; i < nz; i++)
+            slots[oz + z - nz + i] = Slot{(uint32_t)b, os + s - c + i * kPer, min(c - i * kPer, kPer)};
         __syncthreads();
     }
     if (tid == 0) meta->nslots = base_z;
@@ -206,8 +234,7 @@ k_sample_order(const uint32_t *__restrict__ starts, const SampleMeta *__restrict
     if (s < k && meta->lastnz >= 0) order[starts[blk[s]] + rank[s]] = s;
 }
 
-// One workgroup per block that holds samples; a sample bisects the group sums,
-// then walks its group.
+// One workgroup per slot; a sample bisects the group sums, then walks its group.
 template <typename T>
 __global__ void __launch_bounds__(kT)
 k_sample_pick(const T *__restrict__ re, const T *__restrict__ im, uint64_t N,
@@ -322,7 +349,7 @@ int sample_rounds(const spz_state_s *s, uint64_t nb, const double *uniforms, uin
                   uint64_t *out)
 {
     const uint32_t piece = (uint32_t)std::min<uint64_t>(k, kPiece);
-    const uint64_t slots_max = std::min<uint64_t>(piece, nb);
+    const uint64_t slots_max = std::min<uint64_t>(piece, nb + piece / kPer);
     // device layout: out and meta together (one copy back), then the rest
     const size_t o_out = 0, o_meta = up(piece * 8ull), o_u = o_meta + 256;
     const size_t o_blk = o_u + up(piece * 8ull), o_rank = o_blk + up(piece * 4ull);
@@ -352,7 +379,7 @@ int sample_rounds(const spz_state_s *s, uint64_t nb, const double *uniforms, uin
         hipLaunchKernelGGL(k_sample_scan, dim3(1), dim3(kPT), 0, st, counts, nb, slots, meta);
         hipLaunchKernelGGL(k_sample_order, dim3(g), dim3(kT), 0, st, counts, meta, blk, rank, m,
                            order);
-        const unsigned gs = (unsigned)std::min<uint64_t>(m, nb);
+        const unsigned gs = (unsigned)std::min<uint64_t>(m, nb + m / kPer);
         if (s->prec == SPZ_F64)
             hipLaunchKernelGGL((k_sample_pick<double>), dim3(gs), dim3(kT), 0, st,
                                (const double *)s->re, (const double *)s->im, s->N, P, meta, slots,
