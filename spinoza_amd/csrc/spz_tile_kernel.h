@@ -392,7 +392,39 @@ __device__ __forceinline__ uint64_t touch_next(const TileOp &cur, uint64_t opa, 
 // stores overlap the others' gate arithmetic.
 constexpr uint32_t kWarmTiles = 1024;
 
-template <typename T, int K, int LOGW, bool FAST>
+// Consecutive workgroups go to different XCDs.  In grids of kXcdTiles groups
+// and more the block index is permuted so that each XCD works on kXcdRun
+// consecutive tiles, about what its CUs hold at once (32 CUs, 4 workgroups
+// each): neighbouring runs of memory then meet in one L2.  FP32 tiles have runs
+// of 64 bytes, half a line: 27 and 29 qubits 800 -> 780 us and 4.03 -> 3.78 ms a
+// sweep; FP64, with the non-temporal accesses of launch_k, see there.  (Below,
+// nothing to gain: 21 qubits 34.2 and 34.3 us.)
+constexpr uint32_t kXcds = 8, kXcdRun = 128, kXcdTiles = kXcds * kXcdRun;
+
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t tiles)
+{
+    if (tiles < kXcdTiles) return b;  // (both powers of two)
+    return (b & ~(kXcdTiles - 1)) | ((b % kXcds) * kXcdRun) | ((b / kXcds) % kXcdRun);
+}
+
+// Amplitude accesses; NT: non-temporal (see launch_k).
+template <bool NT, typename T>
+__device__ __forceinline__ double load_amp(const char *p)
+{
+    const T *a = reinterpret_cast<const T *>(p);
+    if constexpr (NT) return (double)__builtin_nontemporal_load(a);
+    else return (double)*a;
+}
+
+template <bool NT, typename T>
+__device__ __forceinline__ void store_amp(char *p, double v)
+{
+    T *a = reinterpret_cast<T *>(p);
+    if constexpr (NT) __builtin_nontemporal_store((T)v, a);
+    else *a = (T)v;
+}
+
+template <typename T, int K, int LOGW, bool FAST, bool NT>
 __global__ void __launch_bounds__(1 << LOGW) __attribute__((amdgpu_waves_per_eu(6, 6)))
 k_tile(T *__restrict__ re, T *__restrict__ im, const TileDesc d, const TileOp *__restrict__ ops)
 {
@@ -403,7 +435,7 @@ k_tile(T *__restrict__ re, T *__restrict__ im, const TileDesc d, const TileOp *_
     const uint32_t tid = threadIdx.x;
 
     // global bits of the qubits outside S for this tile
-    const uint64_t base = insert_zeros((uint64_t)blockIdx.x, d.spos, K);
+    const uint64_t base = insert_zeros((uint64_t)xcd_tile(blockIdx.x, gridDim.x), d.spos, K);
     // thread part of the global index and of the local index (lane part)
     // (branch-free: the uniform table reads are issued together)
     uint32_t lt = 0;
@@ -420,8 +452,8 @@ k_tile(T *__restrict__ re, T *__restrict__ im, const TileDesc d, const TileOp *_
     const char *li = reinterpret_cast<const char *>(im + (base + gt));
 #pragma unroll
     for (int p = 0; p < R; p++) {
-        vr[p] = (double)*reinterpret_cast<const T *>(lr + d.gr[p]);
-        vi[p] = (double)*reinterpret_cast<const T *>(li + d.gr[p]);
+        vr[p] = load_amp<NT, T>(lr + d.gr[p]);
+        vi[p] = load_amp<NT, T>(li + d.gr[p]);
     }
 
     const uint64_t ope = reinterpret_cast<uint64_t>(ops + d.nops);
@@ -552,8 +584,8 @@ k_tile(T *__restrict__ re, T *__restrict__ im, const TileDesc d, const TileOp *_
                 a = flip_sign(a, sl ^ (decltype(odd)::value ? u ^ 0x80000000u : u));
                 b = flip_sign(b, sl ^ u);
             }
-            *reinterpret_cast<T *>(sr + d.gs[p]) = (T)a;
-            *reinterpret_cast<T *>(si + d.gs[p]) = (T)b;
+            store_amp<NT, T>(sr + d.gs[p], a);
+            store_amp<NT, T>(si + d.gs[p], b);
         }
     };
     using F = std::false_type;
@@ -582,7 +614,22 @@ int launch_k(spz_state_s *s, const TileDesc &d, const TileOp *d_ops)
         db.gs[p] *= sizeof(T);
     }
     LaunchTimer tm(SPZ_K_TILE, bytes);
-    hipLaunchKernelGGL((k_tile<T, K, LOGW, FAST>), dim3((unsigned)tiles), dim3(1 << LOGW), 0,
+    // FP64 states from the size of the last-level cache (256 MiB, 2^24
+    // amplitudes) up are streamed: non-temporal loads and stores.  With them (and
+    // xcd_tile) a sweep takes, 25 qubits 378 -> 348 us, 28 qubits 2.76 -> 2.52 ms
+    // (ansatz layers), 30 qubits 7.39 -> 7.13 ms (random gates); a smaller state
+    // is still in the cache for the next sweep (23 qubits 90 -> 92 us), and FP32
+    // tiles, whose runs are half a line, lose (27 qubits 800 -> 860 us).
+    constexpr bool may = sizeof(T) == 8 && K == 12;
+    if constexpr (may) {
+        if (s->n >= 24) {
+            hipLaunchKernelGGL((k_tile<T, K, LOGW, FAST, true>), dim3((unsigned)tiles),
+                               dim3(1 << LOGW), 0, rt().stream, (T *)s->re, (T *)s->im, db, d_ops);
+            SPZ_HIP(hipGetLastError());
+            return SPZ_OK;
+        }
+    }
+    hipLaunchKernelGGL((k_tile<T, K, LOGW, FAST, false>), dim3((unsigned)tiles), dim3(1 << LOGW), 0,
                        rt().stream, (T *)s->re, (T *)s->im, db, d_ops);
     SPZ_HIP(hipGetLastError());
     return SPZ_OK;
