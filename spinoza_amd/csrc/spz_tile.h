@@ -124,6 +124,8 @@ enum TileFrameFlags : uint32_t { TF_SIGN = 1u, TF_ODD = 2u, TF_PHASE = 4u, TF_SY
 struct TileDesc {
     int8_t spos[16];          // qubit of local bit i (ascending), K entries
     int8_t tin[16];           // local bit of thread-index bit i in the load layout
+    int8_t sout[16];          // qubit that local bit i is stored to: spos, permuted by the
+                              // sweep's SWAPs
     uint64_t gr[kTileMaxR];   // global offset of register index p in the load layout
     uint64_t gs[kTileMaxR];   // ... and in the store layout (its lane part follows the
                               // program's last layout change); in amplitudes on the

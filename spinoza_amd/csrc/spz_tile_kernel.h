@@ -559,7 +559,7 @@ k_tile(T *__restrict__ re, T *__restrict__ im, const TileDesc d, const TileOp *_
     }
     uint64_t gsb[K];
 #pragma unroll
-    for (int b = 0; b < K; b++) gsb[b] = 1ull << d.spos[b];
+    for (int b = 0; b < K; b++) gsb[b] = 1ull << d.sout[b];
     const uint64_t gs = lane_offset<K>(lt, gsb);
     char *sr = reinterpret_cast<char *>(re + (base + gs));
     char *si = reinterpret_cast<char *>(im + (base + gs));
