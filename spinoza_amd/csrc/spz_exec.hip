@@ -1678,6 +1678,20 @@ int run_dense5(spz_state_s *s, const std::vector<SG> &run)
 
 }  // namespace
 
+// A dense block (arguments checked): its matrix goes through the program ring, so
+// the call neither allocates nor waits.
+int run_dense(spz_state_s *s, int m, const double *u_re, const double *u_im, int t, int control)
+{
+    std::vector<double> coef;
+    dense_coefs(s, m, u_re, u_im, coef);
+    std::lock_guard<std::mutex> lk(g_slot_mu);
+    ProgSlot *slot = nullptr;
+    std::vector<char *> at;
+    SPZ_TRY(upload({bytes_of(coef)}, &slot, &at));
+    Release release{slot};
+    return launch_dense(s, m, (const double *)at[0], t, control);
+}
+
 // A SWAP as three CX, the middle one with the SWAP's controls.
 void swap_as_cx(const spz_op &o, spz_op out[3])
 {

@@ -254,8 +254,11 @@ int launch_pair(spz_state_s *s, const Coef &k, int target, uint64_t ones, uint64
 int launch_diag(spz_state_s *s, const Coef &k, int target, uint64_t ones, uint64_t zeros);
 int launch_swap(spz_state_s *s, int q0, int q1, uint64_t ones, uint64_t zeros);
 int launch_collapse(spz_state_s *s, int target, int outcome, int reset, double scale);
-int launch_dense(spz_state_s *s, int m, const double *u_re, const double *u_im, int t,
-                 int control);
+void dense_coefs(const spz_state_s *s, int m, const double *ur, const double *ui,
+                 std::vector<double> &out);
+int launch_dense(spz_state_s *s, int m, const double *coef, int t, int control);
+// (spz_exec.hip) the same with the matrix on the host
+int run_dense(spz_state_s *s, int m, const double *u_re, const double *u_im, int t, int control);
 int launch_fill_basis(spz_state_s *s, uint64_t index);
 
 // Reductions: term kinds

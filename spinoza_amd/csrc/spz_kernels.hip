@@ -239,6 +239,95 @@ k_dense(T *__restrict__ re, T *__restrict__ im, uint64_t units, int t, int contr
     }
 }
 
+// Blocks of 8 amplitudes and more: a workgroup takes 64 vectors, staged in LDS,
+// and each of its wavefronts a quarter of the rows (the same additions in the same
+// order), with the coefficients in scalar registers.  Bound by one read and write
+// of the state and, from m = 4 on, by 2^(m+3) unfused FP64 operations per
+// amplitude.  One thread per vector left 1024 wavefronts for a 32-amplitude block
+// of 21 qubits, read low blocks at a stride of the vector's length and took every
+// coefficient from LDS.  m = 3, 4, 5, then and now: 21 qubits FP64 18-33, 68-84,
+// 76-131 us, now 13-15, 17-18, 29-32; 26 qubits 494-824, 1990-2290, 2170-3240 us,
+// now 360-400, 395-420, 517-546 (6.0, 5.4, 4.0 TB/s); 27 qubits FP32 0.94-2.1,
+// 3.8-5.1, 4.5-5.8 ms, now 0.46-0.49, 0.58, 1.0; 12 qubits 6.2, 23, 44 us, now 6.2,
+// 10, 26.
+// coef: [wavefront][column][row of the wavefront][re, im] (dense_coefs).
+template <typename T, int M>
+__global__ void __launch_bounds__(kThreads)
+k_dense_rows(T *__restrict__ re, T *__restrict__ im, int t, int control,
+             const double *__restrict__ coef)
+{
+    constexpr int D = 1 << M, ROWS = D / 4, LD = 65;  // (65: low blocks spread over the banks)
+    __shared__ T vr[D * LD], vi[D * LD];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint64_t u0 = (uint64_t)blockIdx.x * 64, u = u0 + lane;
+    const uint64_t mine = ((u >> t) << (t + M)) | (u & ((1ull << t) - 1ull));
+    const bool on = control < 0 || ((mine >> control) & 1);
+    if (!__ballot(on)) return;  // the same for all four wavefronts
+    // with t < 6 the 64 vectors are one run of memory: local index i holds
+    // column (i >> t) % D of vector (i % 2^t) + (i >> (t + M)) 2^t
+    auto place = [&](uint32_t i) {
+        const uint32_t v = (i & ((1u << t) - 1u)) | ((i >> (t + M)) << t);
+        return ((i >> t) & (D - 1)) * LD + v;
+    };
+    if (t >= 6) {
+#pragma unroll
+        for (int k = 0; k < ROWS; k++) {
+            const uint32_t j = k * 4 + wave;
+            const uint64_t g = mine + ((uint64_t)j << t);
+            vr[j * LD + lane] = re[g];
+            vi[j * LD + lane] = im[g];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < ROWS; k++) {
+            const uint32_t i = k * kThreads + tid, o = place(i);
+            vr[o] = re[(u0 << M) + i];
+            vi[o] = im[(u0 << M) + i];
+        }
+    }
+    __syncthreads();
+    double dr[ROWS], di[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) dr[r] = di[r] = 0.0;
+    const double *c = coef + wave * (2 * ROWS * D);
+#pragma unroll 2
+    for (int col = 0; col < D; col++, c += 2 * ROWS) {
+        const double x = vr[col * LD + lane], y = vi[col * LD + lane];
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const double a = c[2 * r], b = c[2 * r + 1];
+            dr[r] += a * x - b * y;
+            di[r] += a * y + b * x;
+        }
+    }
+    if (t >= 6) {
+        if (!on) return;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const uint64_t g = mine + ((uint64_t)(wave * ROWS + r) << t);
+            re[g] = (T)dr[r];
+            im[g] = (T)di[r];
+        }
+        return;
+    }
+    __syncthreads();
+    if (on) {
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            vr[(wave * ROWS + r) * LD + lane] = (T)dr[r];
+            vi[(wave * ROWS + r) * LD + lane] = (T)di[r];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < ROWS; k++) {
+        const uint32_t i = k * kThreads + tid, o = place(i);
+        re[(u0 << M) + i] = vr[o];
+        im[(u0 << M) + i] = vi[o];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Fixed-tree compensated reduction (spz_reduce.h).
 // ---------------------------------------------------------------------------
@@ -490,30 +579,72 @@ int launch_fill_basis(spz_state_s *s, uint64_t index)
     return SPZ_OK;
 }
 
-template <typename T>
-static int dense_dispatch(spz_state_s *s, int m, const double *dur, const double *dui, int t,
-                          int control)
+// Whether a block runs on k_dense_rows: 8 amplitudes and more, and at least the 64
+// vectors of a workgroup.  (Blocks of 4 are at the memory rate with a thread per
+// vector, 9-19 us at 21 qubits, and have one row to a wavefront here.)
+static bool dense_by_rows(const spz_state_s *s, int m) { return m >= 3 && (s->N >> m) >= 64; }
+
+// The block's matrix (row-major) in the order its kernel reads it.
+void dense_coefs(const spz_state_s *s, int m, const double *ur, const double *ui,
+                 std::vector<double> &out)
 {
-    uint64_t units = s->N >> m;
+    const size_t D = (size_t)1 << m, rows = D / 4;
+    out.resize(2 * D * D);
+    for (size_t row = 0; row < D; row++)
+        for (size_t col = 0; col < D; col++) {
+            const double a = ur[row * D + col], b = ui[row * D + col];
+            if (dense_by_rows(s, m)) {
+                double *o = &out[2 * (((row / rows) * D + col) * rows + row % rows)];
+                o[0] = a;
+                o[1] = b;
+            } else {
+                out[row * D + col] = a;
+                out[D * D + row * D + col] = b;
+            }
+        }
+}
+
+template <typename T>
+static int dense_dispatch(spz_state_s *s, int m, const double *coef, int t, int control)
+{
+    const uint64_t units = s->N >> m;
     hipStream_t st = rt().stream;
     T *re = (T *)s->re, *im = (T *)s->im;
+    const double *ui = coef + ((size_t)1 << (2 * m));
     LaunchTimer tm(SPZ_K_DENSE, 2.0 * (double)s->N * amp_bytes(s));
-    switch (m) {
-    case 1: hipLaunchKernelGGL((k_dense<T, 1>), dim3(grid_for(units)), dim3(kThreads), 0, st, re, im, units, t, control, dur, dui); break;
-    case 2: hipLaunchKernelGGL((k_dense<T, 2>), dim3(grid_for(units)), dim3(kThreads), 0, st, re, im, units, t, control, dur, dui); break;
-    case 3: hipLaunchKernelGGL((k_dense<T, 3>), dim3(grid_for(units)), dim3(kThreads), 0, st, re, im, units, t, control, dur, dui); break;
-    case 4: hipLaunchKernelGGL((k_dense<T, 4>), dim3(grid_for(units)), dim3(kThreads), 0, st, re, im, units, t, control, dur, dui); break;
-    case 5: hipLaunchKernelGGL((k_dense<T, 5>), dim3(grid_for(units)), dim3(kThreads), 0, st, re, im, units, t, control, dur, dui); break;
-    default: return fail(SPZ_ERR_ARG, "dense block wider than 5 qubits");
+#define SPZ_DENSE(M)                                                                            \
+    hipLaunchKernelGGL((k_dense<T, M>), dim3(grid_for(units)), dim3(kThreads), 0, st, re, im,     \
+                       units, t, control, coef, ui)
+#define SPZ_DENSE_ROWS(M)                                                                       \
+    hipLaunchKernelGGL((k_dense_rows<T, M>), dim3((unsigned)(units / 64)), dim3(kThreads), 0, st, \
+                       re, im, t, control, coef)
+    if (dense_by_rows(s, m)) {
+        switch (m) {
+        case 3: SPZ_DENSE_ROWS(3); break;
+        case 4: SPZ_DENSE_ROWS(4); break;
+        case 5: SPZ_DENSE_ROWS(5); break;
+        default: return fail(SPZ_ERR_ARG, "dense block wider than 5 qubits");
+        }
+    } else {
+        switch (m) {
+        case 1: SPZ_DENSE(1); break;
+        case 2: SPZ_DENSE(2); break;
+        case 3: SPZ_DENSE(3); break;
+        case 4: SPZ_DENSE(4); break;
+        case 5: SPZ_DENSE(5); break;
+        default: return fail(SPZ_ERR_ARG, "dense block wider than 5 qubits");
+        }
     }
+#undef SPZ_DENSE
+#undef SPZ_DENSE_ROWS
     SPZ_HIP(hipGetLastError());
     return SPZ_OK;
 }
 
-int launch_dense(spz_state_s *s, int m, const double *dur, const double *dui, int t, int control)
+int launch_dense(spz_state_s *s, int m, const double *coef, int t, int control)
 {
-    if (s->prec == SPZ_F64) return dense_dispatch<double>(s, m, dur, dui, t, control);
-    return dense_dispatch<float>(s, m, dur, dui, t, control);
+    if (s->prec == SPZ_F64) return dense_dispatch<double>(s, m, coef, t, control);
+    return dense_dispatch<float>(s, m, coef, t, control);
 }
 
 // ---------------------------------------------------------------------------

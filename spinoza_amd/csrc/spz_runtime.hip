@@ -495,17 +495,7 @@ int spz_transform_u(spz_state s, int m, const double *u_re, const double *u_im, 
     if (control >= 0 && (control >= s->n || (control >= t && control < t + m)))
         return fail(SPZ_ERR_QUBIT, "control must be a qubit outside the block");
     if (control < -1) return fail(SPZ_ERR_QUBIT, "bad control");
-    size_t dd = (size_t)1 << (2 * m);
-    double *d = nullptr;
-    SPZ_HIP(hipMalloc(&d, 2 * dd * sizeof(double)));
-    hipError_t e1 = hipMemcpyAsync(d, u_re, dd * sizeof(double), hipMemcpyHostToDevice, g_rt.stream);
-    hipError_t e2 = hipMemcpyAsync(d + dd, u_im, dd * sizeof(double), hipMemcpyHostToDevice,
-                                   g_rt.stream);
-    int rc = (e1 == hipSuccess && e2 == hipSuccess) ? launch_dense(s, m, d, d + dd, t, control)
-                                                    : fail(SPZ_ERR_HIP, "matrix upload failed");
-    hipStreamSynchronize(g_rt.stream);
-    hipFree(d);
-    return rc;
+    return run_dense(s, m, u_re, u_im, t, control);
 }
 
 int spz_execute(spz_state s, const spz_op *ops, uint64_t n_ops, spz_tracker *tracker,
