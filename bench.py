@@ -78,12 +78,12 @@ def parse():
     p.add_argument("--no-batch", action="store_true", help="skip the batched adjoint leg")
     p.add_argument("--batch-count", type=int, default=1024)
     p.add_argument("--batch-group-qubits", type=int, default=0,
-                   help="circuits above this many qubits count as n_group "
-                        "(0: the library default, < 0: none)")
+                   help="circuits above this many qubits run on several workgroups "
+                        "(0: the library default, < 0: never)")
     p.add_argument("--batch-wg-max", type=int, default=0,
                    help="switch point to the single-circuit path (0: autotuned)")
     p.add_argument("--batch-wg-per-cu", type=int, default=0,
-                   help="spz_batch_opts.wg_per_cu (accepted, without effect)")
+                   help="most resident workgroups per CU (<= 0: as many as fit)")
     p.add_argument("--no-qft", action="store_true", help="skip the 20q QFT leg")
     return p.parse_args()
 
