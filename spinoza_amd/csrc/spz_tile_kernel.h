@@ -363,7 +363,9 @@ __device__ __forceinline__ TileOp fetch_op(uint64_t opa)
 // tiles) 68 -> 50; circuits of one tile, 152 gates, 127 -> 81 forward and 190 ->
 // 140 in reverse (spz_chip.hip).  k_tile does it up to kWarmTiles workgroups,
 // what is resident at once: with more of them the records stay in the scalar
-// caches and touching costs 1.3% (30 qubits).
+// caches and touching costs 1.3% (30 qubits).  The test for it is two scalar
+// instructions per op, so the streamed instances (NT) are without: 7.73 -> 7.61
+// ms a sweep of the 30-qubit random circuit.
 template <int LOGW>
 __device__ __forceinline__ void warm_program(const TileOp *ops, uint32_t nops, uint32_t tid)
 {
@@ -457,7 +459,7 @@ k_tile(T *__restrict__ re, T *__restrict__ im, const TileDesc d, const TileOp *_
     }
 
     const uint64_t ope = reinterpret_cast<uint64_t>(ops + d.nops);
-    const bool few = gridDim.x <= kWarmTiles;
+    const bool few = !NT && gridDim.x <= kWarmTiles;  // (NT grids have 4096 and more)
     if (few) warm_program<LOGW>(ops, (uint32_t)d.nops, tid);
     for (uint64_t opa = reinterpret_cast<uint64_t>(ops); opa != ope; opa += sizeof(TileOp)) {
         asm volatile("" : "+s"(opa));
