@@ -750,15 +750,18 @@ struct Planner {
         return cnt;
     }
 
-    // Register targets still to run, weighted by readiness.
+    // Register targets still to run, weighted by readiness: a ready gate counts
+    // for more than all the waiting ones together, so that the best-scored bit
+    // always has a ready gate (a gate that waits never outranks what it waits for).
     void pair_score(const std::vector<Todo> &todo, std::vector<long> &score) const
     {
+        const long ready_weight = std::max<long>(1000, (long)todo.size() + 1);
         score.assign(K, 0);
         uint64_t bnd = 0, bd = 0;
         for (const Todo &g : todo) {
             if (g.need) {
                 const bool ready = !(g.nd & (bnd | bd)) && !(g.dm & bnd);
-                score[__builtin_ctz(g.need)] += ready ? 1000 : 1;
+                score[__builtin_ctz(g.need)] += ready ? ready_weight : 1;
             }
             bnd |= g.nd;
             bd |= g.dm;
@@ -832,9 +835,9 @@ struct Planner {
         }
         std::vector<int> out;
         if (best_val == -1e30) {
-            // nothing runs under any candidate (cannot happen while a ready
-            // pair gate's target is among the best-scored bits): take the top
-            // bits, which hold every ready target
+            // nothing runs under any candidate: possible only for the load
+            // layout, where every ready target may be a low bit (from lo = 0 the
+            // best-scored bit has a ready gate); take the top bits
             for (int i = 0; i < RB && i < (int)bits.size(); i++) out.push_back(bits[i]);
             std::sort(out.begin(), out.end());
             return out;
