@@ -24,6 +24,10 @@ int launch_adj_sum(const double *part, uint64_t tiles, const uint32_t *d_idx, in
 // (more than one tile; a smaller one needs 2 kChipRows doubles per op).
 inline size_t adj_part_bytes(uint64_t N) { return (N >> kAdjK) * kAdjSlots * 2 * sizeof(double); }
 
+// The sweeps that undo ops[lo, hi) (validated; host only).
+struct ChipPlan;
+int adjoint_plan(int n, const spz_op *ops, uint64_t lo, uint64_t hi, ChipPlan &out);
+
 // Undo ops[lo, hi) (validated, hi > lo, FP64 states) on psi, whose
 // amplitudes are taken from src (another state or psi itself), and on lam, and
 // write dE/dtheta of each parametric one to the device array grad[0, hi).

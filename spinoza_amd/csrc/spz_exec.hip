@@ -157,6 +157,9 @@ int env_int(const char *name, int dflt)
     return (e && *e) ? atoi(e) : dflt;
 }
 
+// How many of the lowest qubits are always in the tile (at most `most`).
+int tile_klo(int most) { return std::max(0, std::min(env_int("SPZ_TILE_KLO", 4), most)); }
+
 struct Sweep {
     bool tile;                 // false: a single gate on the plain path
     int gate;                  // plain: index into the run
@@ -1356,6 +1359,10 @@ struct Planner {
         while (!rem.empty()) {
             uint64_t smask;
             std::vector<int> order = collect(run, rem, smask);
+            if (order.empty() && (max_grads || quick)) {  // (a tile without a free slot)
+                bad = true;
+                return;
+            }
             if (order.size() >= 2) endgame(run, rem, smask, order);
             if (max_grads) {  // a prefix of the order is a valid sweep
                 int left = max_grads;
@@ -1477,7 +1484,7 @@ int run_fused(spz_state_s *s, const std::vector<SG> &run, int K, bool strict)
     pl.K = K;
     pl.LOGW = K - 4;
     pl.RB = 4;
-    pl.klo = std::min(env_int("SPZ_TILE_KLO", 4), K);
+    pl.klo = tile_klo(K);
     pl.improve = env_int("SPZ_TILE_SEARCH", 16);
     pl.strict = strict;
     pl.fast = !strict;
@@ -1749,6 +1756,20 @@ enum class Swaps { BARRIER, AS_CX, RELABEL };
 static int collect_run(const spz_state_s *s, const spz_op *ops, uint64_t n_ops,
                        const spz_tracker *trk, Swaps how, uint64_t *j, std::vector<SG> &run);
 
+// Plans a run whose sweeps are all tile sweeps.
+static int plan_tiles(Planner &pl, const std::vector<SG> &run, ChipPlan &out)
+{
+    pl.plan(run);
+    if (pl.bad) return fail(SPZ_ERR_ARG, "tile planner produced a gate outside the register layout");
+    out.sweeps.clear();
+    for (const Sweep &sw : pl.sweeps)
+        out.sweeps.push_back({sw.desc, (uint32_t)sw.op_begin, (uint32_t)sw.op_count,
+                              (uint32_t)sw.slot_begin, (uint32_t)sw.slots});
+    out.prog.swap(pl.prog);
+    out.grads.swap(pl.grads);
+    return SPZ_OK;
+}
+
 static int plan_chip(int n, const std::vector<SG> &run, bool strict, bool reverse, ChipPlan &out)
 {
     Planner pl;
@@ -1760,15 +1781,7 @@ static int plan_chip(int n, const std::vector<SG> &run, bool strict, bool revers
     pl.strict = strict;
     pl.quick = true;
     if (reverse) pl.max_grads = 1 << 30;
-    pl.plan(run);
-    if (pl.bad) return fail(SPZ_ERR_ARG, "tile planner produced a gate outside the register layout");
-    out.sweeps.clear();
-    for (const Sweep &sw : pl.sweeps)
-        out.sweeps.push_back({sw.desc, (uint32_t)sw.op_begin, (uint32_t)sw.op_count,
-                              (uint32_t)sw.slot_begin, (uint32_t)sw.slots});
-    out.prog.swap(pl.prog);
-    out.grads.swap(pl.grads);
-    return SPZ_OK;
+    return plan_tiles(pl, run, out);
 }
 
 // (spz_chip.h)
@@ -1813,15 +1826,29 @@ static int run_chip(spz_state_s *s, const std::vector<SG> &run)
 }
 
 // (spz_adj_tile.h)
+int adjoint_plan(int n, const spz_op *ops, uint64_t lo, uint64_t hi, ChipPlan &out)
+{
+    std::vector<SG> run;
+    SPZ_TRY(lower_run(std::max(n, kChipK), ops, lo, hi, true, run));
+    if (n <= kChipK) return plan_chip(n, run, false, true, out);
+    Planner pl;
+    pl.n = n;
+    pl.K = kAdjK;
+    pl.LOGW = kAdjK - 4;
+    pl.RB = 4;
+    pl.klo = tile_klo(kAdjK - 1);  // every gate runs in a sweep: one slot for its target
+    pl.improve = env_int("SPZ_TILE_SEARCH", 16);
+    pl.strict = false;
+    pl.max_grads = kAdjSlots;
+    return plan_tiles(pl, run, out);
+}
+
 int adjoint_undo(const spz_state_s *src, spz_state_s *psi, spz_state_s *lam, const spz_op *ops,
                  uint64_t lo, uint64_t hi, double *part, double *grad)
 {
-    std::vector<SG> run;
-    const bool chip = psi->n <= kChipK;
-    SPZ_TRY(lower_run(chip ? kChipK : psi->n, ops, lo, hi, true, run));
-    if (chip) {
-        ChipPlan cp;
-        SPZ_TRY(plan_chip(psi->n, run, false, true, cp));
+    ChipPlan cp;
+    SPZ_TRY(adjoint_plan(psi->n, ops, lo, hi, cp));
+    if (psi->n <= kChipK) {
         std::vector<ChipSweep> d(cp.sweeps.size());
         std::vector<ChipSum> sums;
         const size_t o_d = aligned(cp.prog.size() * sizeof(TileOp));
@@ -1858,26 +1885,15 @@ int adjoint_undo(const spz_state_s *src, spz_state_s *psi, spz_state_s *lam, con
         }
         return launch_chip_sums((const ChipSum *)(slot->dev + o_s), (uint32_t)sums.size(), grad);
     }
-    Planner pl;
-    pl.n = psi->n;
-    pl.K = kAdjK;
-    pl.LOGW = kAdjK - 4;
-    pl.RB = 4;
-    pl.klo = std::min(env_int("SPZ_TILE_KLO", 4), kAdjK);
-    pl.improve = env_int("SPZ_TILE_SEARCH", 16);
-    pl.strict = false;
-    pl.max_grads = kAdjSlots;
-    pl.plan(run);
-    if (pl.bad) return fail(SPZ_ERR_ARG, "tile planner produced a gate outside the register layout");
     std::lock_guard<std::mutex> lk(g_slot_mu);
     ProgSlot *slot = nullptr;
     std::vector<char *> at;
-    SPZ_TRY(upload({bytes_of(pl.prog), bytes_of(pl.grads)}, &slot, &at));
+    SPZ_TRY(upload({bytes_of(cp.prog), bytes_of(cp.grads)}, &slot, &at));
     Release release{slot};
     const TileOp *d_prog = (const TileOp *)at[0];
     const uint32_t *d_idx = (const uint32_t *)at[1];
     const uint64_t tiles = psi->N >> kAdjK;
-    for (const Sweep &sw : pl.sweeps) {
+    for (const ChipPlan::Sweep &sw : cp.sweeps) {
         SPZ_TRY(launch_adj_tile(src, psi, lam, sw.desc, d_prog + sw.op_begin, sw.slots, part));
         SPZ_TRY(launch_adj_sum(part, tiles, d_idx + sw.slot_begin, sw.slots, grad));
         src = psi;
@@ -1982,7 +1998,7 @@ int plan_info(int n, int prec, const spz_op *ops, uint64_t n_ops, const spz_exec
         pl.K = K;
         pl.LOGW = K - 4;
         pl.RB = 4;
-        pl.klo = std::min(env_int("SPZ_TILE_KLO", 4), K);
+        pl.klo = tile_klo(K);
         pl.improve = env_int("SPZ_TILE_SEARCH", 16);
         pl.strict = mode == SPZ_EXEC_STRICT;
         pl.fast = !pl.strict;

@@ -20,20 +20,29 @@ def held_up(heavy, per):
     return [op(N.H, 0)] + ops + [op(N.H, 0)]
 
 
-def chip_plan(n, ops, reverse):
-    """The plan of batched circuits and of states of at most 12 qubits
-    (spz::chip_plan, an inner function of the library): the gates of its program."""
-    f = N.lib()._ZN3spz9chip_planEiPK6spz_opmbRNS_8ChipPlanE
-    f.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_uint64, ctypes.c_bool, ctypes.c_void_p]
+def planned(fn, n, ops, *args):
+    """The gates in the program that an inner planning function of the library makes."""
     arr, keep = encode_ops(ops)
     plan = (ctypes.c_uint64 * 9)()  # three empty std::vector: program, sweeps, gradients
-    rc = f(n, ctypes.addressof(arr), len(ops), reverse, ctypes.addressof(plan))
+    rc = fn(ctypes.c_int(n), arr, *args, plan)
     del keep
     if rc:
         raise N.SpinozaError(rc, N.lib().spz_last_error().decode())
     raw = ctypes.string_at(plan[0], plan[1] - plan[0])
     types = np.frombuffer(raw, dtype=np.int32).reshape(-1, TILE_OP // 4)[:, 0]
     return int(np.sum(types != LAYOUT))
+
+
+def chip_plan(n, ops, reverse):
+    """Batched circuits, forward or reverse (spz::chip_plan)."""
+    return planned(N.lib()._ZN3spz9chip_planEiPK6spz_opmbRNS_8ChipPlanE, n, ops,
+                   ctypes.c_uint64(len(ops)), ctypes.c_bool(reverse))
+
+
+def adjoint_plan(n, ops):
+    """The reverse sweeps of one gradient (spz::adjoint_plan)."""
+    return planned(N.lib()._ZN3spz12adjoint_planEiPK6spz_opmmRNS_8ChipPlanE, n, ops,
+                   ctypes.c_uint64(0), ctypes.c_uint64(len(ops)))
 
 
 @pytest.mark.parametrize("reverse", [False, True])
@@ -50,3 +59,22 @@ def test_tile_plans_of_held_up_gates(n, heavy, per, mode):
     ops = held_up(heavy, per)
     st = plan_stats(n, ops, mode=mode)
     assert st["tile_gates"] + st["plain_gates"] == len(ops)
+
+
+@pytest.mark.parametrize("n,heavy,per", [(6, 5, 1005), (13, 12, 1100), (16, 15, 1100), (20, 3, 1200)])
+def test_reverse_plans_of_held_up_gates(n, heavy, per):
+    ops = held_up(heavy, per)
+    assert adjoint_plan(n, ops) == len(ops)
+
+
+@pytest.mark.parametrize("klo", [-3, 0, 1, 8, 9, 11, 12, 13, 40])
+def test_plans_for_every_number_of_low_qubits(monkeypatch, klo):
+    """SPZ_TILE_KLO outside its range counts as the nearest number in it; a
+    reverse sweep always has room for a gate on any qubit."""
+    monkeypatch.setenv("SPZ_TILE_KLO", str(klo))
+    ops = [op([N.RX, N.RZ, N.H][q % 3], q, theta=0.1 * q, ones=1 << ((q + 5) % 18))
+           for r in range(3) for q in range(18)]
+    swaps = [op(N.SWAP, q, t1=17 - q) for q in range(9)]
+    assert adjoint_plan(18, ops + swaps) == len(ops) + 3 * len(swaps)
+    st = plan_stats(18, ops + swaps)
+    assert st["tile_gates"] + st["plain_gates"] == len(ops) + len(swaps)
