@@ -251,16 +251,17 @@ k_dense(T *__restrict__ re, T *__restrict__ im, uint64_t units, int t, int contr
 // 3.8-5.1, 4.5-5.8 ms, now 0.46-0.49, 0.58, 1.0; 12 qubits 6.2, 23, 44 us, now 6.2,
 // 10, 26.
 // coef: [wavefront][column][row of the wavefront][re, im] (dense_coefs).
+// first: the launch's first workgroup of the whole (dense_dispatch).
 template <typename T, int M>
 __global__ void __launch_bounds__(kThreads)
-k_dense_rows(T *__restrict__ re, T *__restrict__ im, int t, int control,
+k_dense_rows(T *__restrict__ re, T *__restrict__ im, uint64_t first, int t, int control,
              const double *__restrict__ coef)
 {
     constexpr int D = 1 << M, ROWS = D / 4, LD = 65;  // (65: low blocks spread over the banks)
     __shared__ T vr[D * LD], vi[D * LD];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint64_t u0 = (uint64_t)blockIdx.x * 64, u = u0 + lane;
+    const uint64_t u0 = (first + blockIdx.x) * 64, u = u0 + lane;
     const uint64_t mine = ((u >> t) << (t + M)) | (u & ((1ull << t) - 1ull));
     const bool on = control < 0 || ((mine >> control) & 1);
     if (!__ballot(on)) return;  // the same for all four wavefronts
@@ -615,9 +616,13 @@ static int dense_dispatch(spz_state_s *s, int m, const double *coef, int t, int 
 #define SPZ_DENSE(M)                                                                            \
     hipLaunchKernelGGL((k_dense<T, M>), dim3(grid_for(units)), dim3(kThreads), 0, st, re, im,     \
                        units, t, control, coef, ui)
+    // workgroups of 64 vectors, at most 2^23 of them to a launch: 2^31 work-items,
+    // where a dispatch takes fewer than 2^32 (a 3-qubit block of 33 qubits has 2^24)
+    const uint64_t groups = units / 64, most = 1ull << 23;
 #define SPZ_DENSE_ROWS(M)                                                                       \
-    hipLaunchKernelGGL((k_dense_rows<T, M>), dim3((unsigned)(units / 64)), dim3(kThreads), 0, st, \
-                       re, im, t, control, coef)
+    for (uint64_t f = 0; f < groups; f += most)                                                   \
+        hipLaunchKernelGGL((k_dense_rows<T, M>), dim3((unsigned)std::min(groups - f, most)),       \
+                           dim3(kThreads), 0, st, re, im, f, t, control, coef)
     if (dense_by_rows(s, m)) {
         switch (m) {
         case 3: SPZ_DENSE_ROWS(3); break;
