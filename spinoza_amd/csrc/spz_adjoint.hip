@@ -97,9 +97,12 @@ constexpr size_t kCkptKeep = (size_t)4 << 30;
 
 struct CkptPool {
     std::vector<std::unique_ptr<OwnedState>> st;
+    size_t used = 0;  // by the call that is running
 
+    // The i-th checkpoint of a call (i = 0, 1, ...).
     int get(size_t i, const spz_state_s *like, spz_state_s **out)
     {
+        used = i;
         if (!st.empty() && (st[0]->s->n != like->n || st[0]->s->prec != like->prec)) st.clear();
         while (st.size() <= i) {
             auto o = std::make_unique<OwnedState>();
@@ -107,11 +110,20 @@ struct CkptPool {
             st.push_back(std::move(o));
         }
         *out = st[i]->s;
+        used = i + 1;
         return SPZ_OK;
+    }
+
+    bool drop_unused()
+    {
+        if (st.size() <= used) return false;
+        st.resize(used);
+        return true;
     }
 
     void trim()
     {
+        used = 0;
         if (st.empty()) return;
         const size_t each = (size_t)st[0]->s->N * (st[0]->s->prec == SPZ_F64 ? 16 : 8);
         if (each * st.size() > kCkptKeep) st.clear();
@@ -131,6 +143,27 @@ struct AdjScratch {
     void *grad = nullptr, *part = nullptr, *dmax = nullptr;
     size_t grad_cap = 0, part_cap = 0;
     CkptPool ckpts;
+    bool in_use = false;  // a call is running
+
+    // Free what no call uses (a running one: checkpoint states beyond its own).
+    bool give_back()
+    {
+        bool any = ckpts.drop_unused();
+        if (in_use) return any;
+        for (void *&a : arr) drop(&a, any);
+        drop(&grad, any);
+        drop(&part, any);
+        arr_cap = grad_cap = part_cap = 0;
+        return any;
+    }
+
+    static void drop(void **p, bool &any)
+    {
+        if (!*p) return;
+        (void)hipFree(*p);
+        *p = nullptr;
+        any = true;
+    }
 
     int reserve_states(int n, int prec)
     {
@@ -143,8 +176,7 @@ struct AdjScratch {
                 }
             arr_cap = 0;
             for (void *&a : arr)
-                if (hipMalloc(&a, bytes) != hipSuccess) {
-                    (void)hipGetLastError();
+                if (device_alloc(&a, bytes) != hipSuccess) {
                     for (void *&b : arr)
                         if (b) {
                             (void)hipFree(b);
@@ -176,11 +208,8 @@ struct AdjScratch {
         if (*p) SPZ_HIP(hipFree(*p));
         *p = nullptr;
         *cap = 0;
-        if (hipMalloc(p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            *p = nullptr;
+        if (device_alloc(p, bytes) != hipSuccess)
             return fail(SPZ_ERR_OOM, "adjoint scratch allocation failed");
-        }
         *cap = bytes;
         return SPZ_OK;
     }
@@ -190,11 +219,8 @@ struct AdjScratch {
         SPZ_TRY(grow(&grad, &grad_cap, grad_bytes));
         SPZ_TRY(grow(&part, &part_cap, part_bytes));
         if (!dmax) {
-            if (hipMalloc(&dmax, sizeof(unsigned long long)) != hipSuccess) {
-                (void)hipGetLastError();
-                dmax = nullptr;
+            if (device_alloc(&dmax, sizeof(unsigned long long)) != hipSuccess)
                 return fail(SPZ_ERR_OOM, "adjoint scratch allocation failed");
-            }
         }
         return SPZ_OK;
     }
@@ -217,6 +243,8 @@ AdjScratch &adj_scratch()
 }
 
 }  // namespace
+
+bool adjoint_give_back() { return adj_scratch().give_back(); }
 
 // The ops a differentiated circuit may hold: unitary single-target gates H..U
 // (and SWAP where allowed) with 1- and 0-controls; every qubit in range, the
@@ -252,10 +280,15 @@ int adjoint_grad(spz_state_s *s, const spz_op *ops, uint64_t n_ops, double hx, i
     for (uint64_t i = 0; i < n_ops; i++) SPZ_TRY(validate_adjoint_op(s->n, ops[i], i, true, 64));
     AdjScratch &sc = adj_scratch();
     std::lock_guard<std::mutex> lock(sc.mu);
-    struct Trim {
-        CkptPool &p;
-        ~Trim() { p.trim(); }
-    } trim{sc.ckpts};
+    struct Running {
+        AdjScratch &s;
+        explicit Running(AdjScratch &a) : s(a) { s.in_use = true; }
+        ~Running()
+        {
+            s.ckpts.trim();
+            s.in_use = false;
+        }
+    } running(sc);
     // ---- forward pass with checkpoints ---------------------------------------
     std::vector<spz_state_s *> ckpts;
     std::vector<uint64_t> ckpt_at;  // checkpoint j holds psi after op ckpt_at[j]

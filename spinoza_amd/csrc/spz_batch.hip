@@ -57,11 +57,8 @@ struct Buf {
     {
         if (bytes <= cap) return SPZ_OK;
         drop();
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            p = nullptr;
+        if (device_alloc(&p, bytes) != hipSuccess)
             return fail(SPZ_ERR_OOM, "batched adjoint scratch allocation failed");
-        }
         cap = bytes;
         return SPZ_OK;
     }
@@ -91,7 +88,7 @@ struct Slot {
         if (!done) SPZ_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
         if (bytes <= cap) return SPZ_OK;
         drop();
-        if (hipMalloc(&dev, bytes) != hipSuccess ||
+        if (device_alloc((void **)&dev, bytes) != hipSuccess ||
             hipHostMalloc(&host, bytes, hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
             drop();
@@ -114,6 +111,20 @@ struct Scratch {
     Buf states, parts, out;
     Slot slots[2];
     std::vector<hipEvent_t> events;  // pairs of timing events, one per chunk
+    bool in_use = false;             // a call is running
+
+    void drop()  // (the stream was waited for, or the frees wait for it)
+    {
+        for (Buf *b : {&states, &parts, &out}) b->drop();
+        for (Slot &s : slots) {
+            s.busy = false;
+            s.drop();
+        }
+    }
+    size_t bytes() const
+    {
+        return states.cap + parts.cap + out.cap + slots[0].cap + slots[1].cap;
+    }
 };
 Scratch &scratch()
 {
@@ -320,6 +331,14 @@ struct Chunk {
 
 }  // namespace
 
+bool batch_give_back()
+{
+    Scratch &sc = scratch();
+    if (sc.in_use || !sc.bytes()) return false;
+    sc.drop();
+    return true;
+}
+
 }  // namespace spz
 
 using namespace spz;
@@ -376,6 +395,11 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
         return a.n != b.n ? a.n > b.n : a.n_ops > b.n_ops;
     });
     Scratch &sc = scratch();
+    struct InUse {
+        bool &flag;
+        explicit InUse(bool &f) : flag(f) { flag = true; }
+        ~InUse() { flag = false; }
+    } in_use(sc.in_use);
     // wg_per_cu > 0 caps the workgroups resident on a CU by padding their LDS
     // (160 KiB per CU, 32 KiB used, at most 64 KiB per workgroup)
     size_t lds = 0;
@@ -463,13 +487,7 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
             }
         }
     }
-    if (sc.states.cap + sc.parts.cap + sc.out.cap + sc.slots[0].cap + sc.slots[1].cap > kKeep) {
-        for (Buf *b : {&sc.states, &sc.parts, &sc.out}) b->drop();
-        for (Slot &s : sc.slots) {
-            s.busy = false;  // (the stream was waited for)
-            s.drop();
-        }
-    }
+    if (sc.bytes() > kKeep) sc.drop();
     if (rc != SPZ_OK) return rc;
     auto t1 = std::chrono::steady_clock::now();
     if (stats) {

@@ -1430,7 +1430,7 @@ int reserve_slot(size_t total, ProgSlot **out)
         sl.host = nullptr;
         sl.cap = 0;
         const size_t cap = std::max(total, 4096 * sizeof(TileOp));
-        if (hipMalloc(&sl.dev, cap) != hipSuccess ||
+        if (device_alloc((void **)&sl.dev, cap) != hipSuccess ||
             hipHostMalloc(&sl.host, cap, hipHostMallocDefault) != hipSuccess)
             return fail(SPZ_ERR_OOM, "tile program allocation failed");
         sl.cap = cap;

@@ -73,6 +73,15 @@ std::recursive_mutex &api_mutex();
 #define SPZ_API_LOCK std::lock_guard<std::recursive_mutex> spz_api_lock_(::spz::api_mutex())
 int ensure_partials(size_t pairs);
 
+// Device memory, under the library lock.  When an allocation fails, what finished
+// calls keep for later ones is given back (gradients: working states, checkpoint
+// states of up to 4 GiB; batches: buffers of up to 1 GiB) and it is tried again.
+hipError_t device_alloc(void **p, size_t bytes);
+// Free the kept memory that no call uses; whether there was any.
+bool adjoint_give_back();
+bool batch_give_back();
+extern int g_alloc_failures;  // (tests) so many attempts to come count as failed
+
 // Bracket a kernel launch with events when profiling is on.
 struct LaunchTimer {
     int cls;

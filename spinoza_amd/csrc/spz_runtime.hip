@@ -50,6 +50,28 @@ int ensure_init()
     return SPZ_OK;
 }
 
+int g_alloc_failures = 0;
+
+static hipError_t try_alloc(void **p, size_t bytes)
+{
+    hipError_t e = hipErrorOutOfMemory;
+    if (g_alloc_failures > 0) g_alloc_failures--;
+    else e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
+hipError_t device_alloc(void **p, size_t bytes)
+{
+    const hipError_t e = try_alloc(p, bytes);
+    if (e == hipSuccess) return e;
+    const bool a = adjoint_give_back(), b = batch_give_back();
+    return a || b ? try_alloc(p, bytes) : e;
+}
+
 int ensure_partials(size_t pairs)
 {
     if (pairs <= g_rt.partial_cap) return SPZ_OK;
@@ -59,7 +81,7 @@ int ensure_partials(size_t pairs)
         g_rt.d_partials = nullptr;
     }
     size_t cap = std::max<size_t>(pairs, 1024);
-    if (hipMalloc(&g_rt.d_partials, cap * 2 * sizeof(double)) != hipSuccess)
+    if (device_alloc((void **)&g_rt.d_partials, cap * 2 * sizeof(double)) != hipSuccess)
         return fail(SPZ_ERR_OOM, "reduction scratch allocation failed");
     g_rt.partial_cap = cap;
     return SPZ_OK;
@@ -298,13 +320,11 @@ int spz_state_create(int n, int precision, spz_state *out)
     s->prec = precision;
     s->N = 1ull << n;
     size_t bytes = (size_t)s->N * (precision == SPZ_F64 ? 8 : 4);
-    if (hipMalloc(&s->re, bytes) != hipSuccess) {
-        hipGetLastError();
+    if (device_alloc(&s->re, bytes) != hipSuccess) {
         delete s;
         return fail(SPZ_ERR_OOM, "state allocation failed (reals)");
     }
-    if (hipMalloc(&s->im, bytes) != hipSuccess) {
-        hipGetLastError();
+    if (device_alloc(&s->im, bytes) != hipSuccess) {
         hipFree(s->re);
         delete s;
         return fail(SPZ_ERR_OOM, "state allocation failed (imags)");

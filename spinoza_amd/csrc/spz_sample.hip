@@ -355,11 +355,8 @@ int reserve(size_t dev_bytes, size_t host_bytes)
         if (g_scr.dev) SPZ_HIP(hipFree(g_scr.dev));
         g_scr.dev = nullptr;
         g_scr.dev_cap = 0;
-        if (hipMalloc(&g_scr.dev, dev_bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            g_scr.dev = nullptr;
+        if (device_alloc(&g_scr.dev, dev_bytes) != hipSuccess)
             return fail(SPZ_ERR_OOM, "sampling scratch allocation failed");
-        }
         g_scr.dev_cap = dev_bytes;
     }
     if (host_bytes > g_scr.host_cap) {
