@@ -79,6 +79,7 @@ int ensure_partials(size_t pairs)
         SPZ_HIP(hipStreamSynchronize(g_rt.stream));
         SPZ_HIP(hipFree(g_rt.d_partials));
         g_rt.d_partials = nullptr;
+        g_rt.partial_cap = 0;
     }
     size_t cap = std::max<size_t>(pairs, 1024);
     if (device_alloc((void **)&g_rt.d_partials, cap * 2 * sizeof(double)) != hipSuccess)

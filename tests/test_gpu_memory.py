@@ -2,8 +2,10 @@
 the allocation tried again; a second failure raises, and the calls after it
 are right.  Failures are counted down by the library, no memory is filled."""
 import ctypes
+import os
+import subprocess
+import sys
 
-import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -79,3 +81,32 @@ def test_failures_inside_calls(failures):
     assert err.value.code == N.ERR_OOM
     failures.value = 0
     assert gradient(20, 5) == ref[20] and gradient(18, 5) == ref[18] and batch() == b0
+
+
+REDUCTION = """
+import ctypes
+import spinoza_amd as spz
+from spinoza_amd import _native as N
+failures = ctypes.c_int.in_dll(N.lib(), "_ZN3spz16g_alloc_failuresE")
+small, large = spz.State(13), spz.State(26)
+want = small.norm()  # the smallest scratch
+failures.value = 2
+try:
+    spz.xyz_expectation_value("z", large, list(range(8)))
+    raise SystemExit("no error")
+except N.SpinozaError as e:
+    assert e.code == N.ERR_OOM, e
+failures.value = 0
+assert small.norm() == want == 1.0
+assert spz.xyz_expectation_value("z", large, list(range(8))) == [1.0] * 8
+"""
+
+
+def test_reduction_scratch_after_a_failure():
+    """The scratch of reductions is freed before it grows: after a failure it
+    has no size left (a process of its own, where it is still small)."""
+    print("case reduction scratch", flush=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", REDUCTION], cwd=root, capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
