@@ -47,6 +47,8 @@ constexpr size_t kKeep = (size_t)1 << 30;  // scratch kept between calls
 
 int g_wg_max_qubits = -1;  // autotuned switch point (-1: not tuned yet)
 
+int switch_point() { return g_wg_max_qubits > 0 ? g_wg_max_qubits : 14; }
+
 // Grow-only device buffers, given back at the end of a call that needed more
 // than kKeep bytes of them (a free synchronises the device).
 struct Buf {
@@ -148,6 +150,21 @@ ChipPlan::Sweep empty_sweep()
     }
     for (uint64_t p = 0; p < 16; p++) s.desc.gr[p] = s.desc.gs[p] = p << (kChipK - 4);
     return s;
+}
+
+// One rule for both paths (the switch point must not decide whether a circuit
+// is accepted): gates H..U, at most kMaxControls controls.
+int check_circuit(const spz_batch_circuit &c, const spz_op *ops, uint64_t i)
+{
+    if (c.n < 1 || c.n > 30 || c.n_ops < 0) return fail(SPZ_ERR_ARG, "bad circuit entry");
+    for (int o = 0; o < c.n_ops; o++) {
+        const int rc = validate_adjoint_op(c.n, ops[c.op_offset + o], (uint64_t)o, false, kMaxControls);
+        if (rc != SPZ_OK) {
+            set_error("circuit " + std::to_string(i) + ": " + spz_last_error());
+            return rc;
+        }
+    }
+    return SPZ_OK;
 }
 
 struct Job {
@@ -355,7 +372,7 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
     if (!circuits || !ops || !energies || !grads) return fail(SPZ_ERR_ARG, "null argument");
     const int wg_max = opts && opts->wg_max_qubits > 0
                            ? opts->wg_max_qubits
-                           : (g_wg_max_qubits > 0 ? g_wg_max_qubits : 14);
+                           : switch_point();
     // circuits above gq qubits run on 2^(n - gq) workgroups (at most one per tile)
     const int gq_opt = opts ? opts->group_qubits : 0;
     const int gq = gq_opt < 0 ? 64 : (gq_opt == 0 ? kChipK : std::max(gq_opt, 8));
@@ -365,17 +382,7 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
     uint64_t gmax = 0;
     for (uint64_t i = 0; i < count; i++) {
         const spz_batch_circuit &c = circuits[i];
-        if (c.n < 1 || c.n > 30 || c.n_ops < 0) return fail(SPZ_ERR_ARG, "bad circuit entry");
-        // one rule for both paths (the switch point must not decide whether
-        // a circuit is accepted): gates H..U, at most kMaxControls controls
-        for (int o = 0; o < c.n_ops; o++) {
-            const int rc = validate_adjoint_op(c.n, ops[c.op_offset + o], (uint64_t)o, false,
-                                               kMaxControls);
-            if (rc != SPZ_OK) {
-                set_error("circuit " + std::to_string(i) + ": " + spz_last_error());
-                return rc;
-            }
-        }
+        SPZ_TRY(check_circuit(c, ops, i));
         if (c.n > wg_max || c.n > kBatchMaxQubits) {
             large.push_back(i);
             continue;
@@ -506,13 +513,18 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
 int spz_batch_autotune(const spz_batch_circuit *circuits, uint64_t count, const spz_op *ops,
                        int *wg_max_qubits)
 {
-    // For every qubit count present: run up to 8 of its circuits batched and
-    // one at a time; the switch point is the largest n for which the batch wins.
+    // For every qubit count present that can run batched: run up to 8 of its
+    // circuits batched and one at a time; the switch point is the largest n for
+    // which the batch wins.  (Larger circuits take the same path in both runs, so
+    // only noise would decide; with none but those the switch point stays.)
     SPZ_API_LOCK;
     SPZ_TRY(ensure_init());
     if (!circuits || !ops) return fail(SPZ_ERR_ARG, "null argument");
     std::vector<int> ns;
-    for (uint64_t i = 0; i < count; i++) ns.push_back(circuits[i].n);
+    for (uint64_t i = 0; i < count; i++) {
+        SPZ_TRY(check_circuit(circuits[i], ops, i));
+        if (circuits[i].n <= kBatchMaxQubits) ns.push_back(circuits[i].n);
+    }
     std::sort(ns.begin(), ns.end());
     ns.erase(std::unique(ns.begin(), ns.end()), ns.end());
     int best = 0;
@@ -539,8 +551,8 @@ int spz_batch_autotune(const spz_batch_circuit *circuits, uint64_t count, const 
         }
         if (sw.total_ms <= sl.total_ms) best = n;
     }
-    g_wg_max_qubits = best > 0 ? best : 1;
-    if (wg_max_qubits) *wg_max_qubits = g_wg_max_qubits;
+    if (!ns.empty()) g_wg_max_qubits = best > 0 ? best : 1;
+    if (wg_max_qubits) *wg_max_qubits = switch_point();
     return SPZ_OK;
 }
 
