@@ -420,6 +420,12 @@ struct Planner {
     // Cheap planning (spz_chip.h): every sweep is a tile sweep, the next register
     // bits are simply the best-scored ones.
     bool quick = false;
+    // ... and of at most so many gates (0: any number): choosing layouts passes over
+    // a sweep's remaining gates at every change, which is quadratic in their
+    // number.  Circuits of 8 to 12 qubits are otherwise one sweep: 10000 gates
+    // 25 ms and 30000 gates 250 ms a direction, now 6 and 20 ms; a further sweep
+    // costs a launch and a pass over the tile, about 10 us for 1024 gates' 500.
+    size_t max_gates = 0;
     std::vector<uint32_t> grads;  // the sweeps' gradients, slot by slot
     uint64_t frame_gates = 0;  // gates absorbed into Pauli frames
     uint64_t split_ops = 0;    // second halves of gates run as two half-angle ops
@@ -473,6 +479,7 @@ struct Planner {
             }
             if (ok) {
                 order.push_back(idx);
+                if (order.size() == max_gates) break;
             } else {
                 if (strict) break;
                 bnd |= g.nd;
@@ -1781,6 +1788,7 @@ static int plan_chip(int n, const std::vector<SG> &run, bool strict, bool revers
     pl.strict = strict;
     pl.quick = true;
     if (reverse) pl.max_grads = 1 << 30;
+    if (!strict) pl.max_gates = 1024;
     return plan_tiles(pl, run, out);
 }
 

@@ -2,6 +2,7 @@
 holds each gate once, also where one qubit with few gates holds up more than a
 thousand gates on each of the others."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -78,3 +79,24 @@ def test_plans_for_every_number_of_low_qubits(monkeypatch, klo):
     assert adjoint_plan(18, ops + swaps) == len(ops) + 3 * len(swaps)
     st = plan_stats(18, ops + swaps)
     assert st["tile_gates"] + st["plain_gates"] == len(ops) + len(swaps)
+
+
+@pytest.mark.parametrize("reverse", [False, True])
+def test_batched_planning_time_is_linear(reverse):
+    """Four times the gates of a 10-qubit circuit: 4 times the time where a sweep
+    has a bounded number of gates, 16 times where a circuit is one sweep."""
+    rng = np.random.default_rng(3)
+    ops = []
+    for _ in range(24000):
+        a, b = (int(q) for q in rng.permutation(10)[:2])
+        kind = [N.RX, N.RY, N.RZ, N.X][int(rng.integers(4))]
+        ops.append(op(kind, a, theta=0.1, ones=1 << b if kind == N.X else 0))
+    took = []
+    for part in (ops[:6000], ops):
+        best = float("inf")
+        for _ in range(3):
+            t = time.process_time()
+            assert chip_plan(10, part, reverse) == len(part)
+            best = min(best, time.process_time() - t)
+        took.append(best)
+    assert took[1] < 8 * took[0], took
