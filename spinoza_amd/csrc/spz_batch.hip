@@ -41,7 +41,11 @@ namespace {
 constexpr int kMaxControls = 7;
 constexpr int kBatchMaxQubits = 20;     // larger circuits fill the GPU on their own
 constexpr uint64_t kChunkTiles = 768;   // three reverse workgroups on each of 256 CUs
-constexpr uint64_t kChunkOps = 20000;   // bounds a chunk's program (128 bytes per op)
+// A chunk ends at so many ops once every CU has a workgroup, and at 256 MiB of
+// program (128 bytes per op) in any case.  (Ended at kChunkOps whatever its tiles,
+// long circuits ran one after another: 64 of 10 qubits and 10000 ops 996 ms, now
+// 65; 256 of 1000 ops 45 and 21 ms; 128 of 10 to 18 qubits 10.3 and 9.6 ms.)
+constexpr uint64_t kChunkOps = 20000, kChunkFull = 256, kChunkMax = 1u << 21;
 constexpr int kPlanThreads = 8;
 constexpr size_t kKeep = (size_t)1 << 30;  // scratch kept between calls
 
@@ -197,7 +201,8 @@ int plan_chunk(const spz_batch_circuit *circuits, const spz_op *ops, const Job *
         }
     };
     const unsigned cores = std::max(1u, std::thread::hardware_concurrency());
-    const uint64_t want = std::min<uint64_t>({(uint64_t)kPlanThreads, cores, count, nops / 1000 + 1});
+    const uint64_t cost = 8ull * count + nops / 2;  // us, both directions
+    const uint64_t want = std::min<uint64_t>({(uint64_t)kPlanThreads, cores, count, cost / 150 + 1});
     std::vector<std::thread> pool;
     pool.reserve(kPlanThreads);
     try {
@@ -430,7 +435,9 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
                 const spz_batch_circuit &c = circuits[small[b].circuit];
                 tiles += tiles_of(c.n);
                 nops += 2 * (uint64_t)c.n_ops;
-                if (b > a && (tiles > kChunkTiles || nops > kChunkOps)) break;
+                if (b > a && (tiles > kChunkTiles || nops > kChunkMax ||
+                              (nops > kChunkOps && tiles > kChunkFull)))
+                    break;
                 b++;
             }
             const size_t k = first.size();
