@@ -48,6 +48,7 @@ constexpr uint64_t kChunkTiles = 768;   // three reverse workgroups on each of 2
 constexpr uint64_t kChunkOps = 20000, kChunkFull = 256, kChunkMax = 1u << 21;
 constexpr int kPlanThreads = 8;
 constexpr size_t kKeep = (size_t)1 << 30;  // scratch kept between calls
+constexpr size_t kKeepPlans = (size_t)64 << 20;
 
 int g_wg_max_qubits = -1;  // autotuned switch point (-1: not tuned yet)
 
@@ -117,6 +118,7 @@ struct Scratch {
     Buf states, parts, out;
     Slot slots[2];
     std::vector<hipEvent_t> events;  // pairs of timing events, one per chunk
+    std::vector<ChipPlan> fwd, rev;  // a chunk's plans
     bool in_use = false;             // a call is running
 
     void drop()  // (the stream was waited for, or the frees wait for it)
@@ -126,6 +128,19 @@ struct Scratch {
             s.busy = false;
             s.drop();
         }
+    }
+    // Plans keep their memory from chunk to chunk and call to call (allocated anew, its
+    // page faults cost several threads more than planning small circuits does), at
+    // most kKeepPlans of it.
+    void trim_plans()
+    {
+        size_t n = 0;
+        for (const auto *v : {&fwd, &rev})
+            for (const ChipPlan &p : *v)
+                n += p.prog.capacity() * sizeof(TileOp) + p.sweeps.capacity() * sizeof(ChipPlan::Sweep);
+        if (n <= kKeepPlans) return;
+        fwd = std::vector<ChipPlan>();
+        rev = std::vector<ChipPlan>();
     }
     size_t bytes() const
     {
@@ -176,10 +191,11 @@ struct Job {
     uint32_t width;     // workgroups it may use
 };
 
-// Forward and reverse plans of a chunk's circuits.  Planning costs about 0.1 us
-// per op and direction, more than the GPU takes for circuits of up to 12 qubits
-// (180 of them: 6.0 ms planned by one thread, 0.6 ms of sweeps), so a chunk is
-// planned by several threads once it has enough ops to pay for starting them.
+// Forward and reverse plans of a chunk's circuits.  Planning costs about half a
+// microsecond per circuit and 0.06 to 0.2 us per op in each direction, more than
+// the GPU takes for circuits of up to 12 qubits (180 of them: 6.0 ms planned by one
+// thread, 0.6 ms of sweeps), so a chunk is planned by several threads once there
+// is enough to pay for starting them (20 to 40 us each).
 int plan_chunk(const spz_batch_circuit *circuits, const spz_op *ops, const Job *jobs,
                uint32_t count, std::vector<ChipPlan> &fwd, std::vector<ChipPlan> &rev)
 {
@@ -201,7 +217,7 @@ int plan_chunk(const spz_batch_circuit *circuits, const spz_op *ops, const Job *
         }
     };
     const unsigned cores = std::max(1u, std::thread::hardware_concurrency());
-    const uint64_t cost = 8ull * count + nops / 2;  // us, both directions
+    const uint64_t cost = count + nops / 4;  // about so many us, both directions
     const uint64_t want = std::min<uint64_t>({(uint64_t)kPlanThreads, cores, count, cost / 150 + 1});
     std::vector<std::thread> pool;
     pool.reserve(kPlanThreads);
@@ -228,7 +244,11 @@ struct Chunk {
     int run(const Job *jobs, uint32_t count, uint32_t slot0, Scratch &sc, Slot &slot,
             hipEvent_t begin, hipEvent_t end)
     {
-        std::vector<ChipPlan> fwd(count), rev(count);
+        if (sc.fwd.size() < count) {
+            sc.fwd.resize(count);
+            sc.rev.resize(count);
+        }
+        std::vector<ChipPlan> &fwd = sc.fwd, &rev = sc.rev;
         uint64_t amps = 0, pairs = 0, nops = 0;
         size_t nf = 0, nr = 0, ns = 0, lf = 0, lr = 0;
         uint32_t width = 0, blocks = 0;
@@ -502,6 +522,7 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
         }
     }
     if (sc.bytes() > kKeep) sc.drop();
+    sc.trim_plans();
     if (rc != SPZ_OK) return rc;
     auto t1 = std::chrono::steady_clock::now();
     if (stats) {

@@ -197,10 +197,47 @@ uint32_t kind_bit(int ak)
 // A change of register layout inside a sweep: an LDS transpose to any
 // layout, or in-wavefront swaps of register-index bits with lane bits 4 and 5
 // (v_permlane16/32_swap), which move no data through LDS.
+// A few values in place (a tile has at most kTileMaxK bits): planning a small
+// circuit is otherwise mostly malloc and free.
+template <typename T>
+struct Few {
+    static constexpr int kMost = 16;
+    static_assert(kTileMaxK <= kMost, "a value per tile bit");
+    T v[kMost];
+    int n = 0;
+
+    Few() = default;
+    explicit Few(int count, T x = T()) { assign(count, x); }
+    Few(const T *b, const T *e) { while (b != e) push_back(*b++); }
+    void assign(int count, T x)
+    {
+        n = count;
+        for (int i = 0; i < n; i++) v[i] = x;
+    }
+    void push_back(T x) { v[n++] = x; }
+    void clear() { n = 0; }
+    void erase(T *at)
+    {
+        std::copy(at + 1, end(), at);
+        n--;
+    }
+    size_t size() const { return (size_t)n; }
+    bool empty() const { return n == 0; }
+    T *begin() { return v; }
+    T *end() { return v + n; }
+    const T *begin() const { return v; }
+    const T *end() const { return v + n; }
+    T &operator[](size_t i) { return v[i]; }
+    const T &operator[](size_t i) const { return v[i]; }
+    bool operator!=(const Few &o) const { return !std::equal(begin(), end(), o.begin(), o.end()); }
+};
+using Bits = Few<int>;
+using Scores = Few<long>;
+
 struct Change {
     bool lds = true;
-    std::vector<int> rs;                    // register slot -> local bit after it
-    std::vector<int> thr;                   // thread-index bit -> local bit after it
+    Bits rs;                    // register slot -> local bit after it
+    Bits thr;                   // thread-index bit -> local bit after it
     std::vector<std::pair<int, int>> sw;    // (register slot, lane bit), in order
 };
 
@@ -407,6 +444,18 @@ void ush_form(Coef &k, double *gr, double *gi, bool *zafter)
     *gi = ai;
 }
 
+// A stable sort (std::stable_sort allocates).
+template <typename Before>
+void sort_bits(Bits &v, Before before)
+{
+    for (size_t i = 1; i < v.size(); i++) {
+        const int x = v[i];
+        size_t j = i;
+        for (; j && before(x, v[j - 1]); j--) v[j] = v[j - 1];
+        v[j] = x;
+    }
+}
+
 struct Planner {
     int n, K, LOGW, RB, klo;
     int improve = 0;  // local-search passes over the tile set (AUTO only)
@@ -432,7 +481,7 @@ struct Planner {
     uint64_t swap_gates = 0;   // SWAPs that a sweep's store carries out
     // The local bits stored to qubits 0..klo-1 by the sweep being built (they end
     // on the low lanes, so that stores are contiguous), and their mask.
-    std::vector<int> outlow;
+    Bits outlow;
     uint32_t outmask = 0;
     std::vector<TileOp> prog;
     std::vector<Sweep> sweeps;
@@ -461,6 +510,7 @@ struct Planner {
                              uint64_t &smask)
     {
         std::vector<int> order;
+        order.reserve(std::min<size_t>(rem.size(), 64));
         smask = (klo >= 64) ? ~0ull : ((1ull << klo) - 1);
         int free_slots = K - klo;
         uint64_t bnd = 0, bd = 0;
@@ -584,7 +634,8 @@ struct Planner {
     static std::vector<int> minus(const std::vector<int> &rem, const std::vector<int> &ord)
     {
         std::vector<int> out;
-        out.reserve(rem.size());
+        if (ord.size() == rem.size()) return out;
+        out.reserve(rem.size() - ord.size());
         size_t k = 0;
         for (int idx : rem) {
             if (k < ord.size() && ord[k] == idx) { k++; continue; }
@@ -637,8 +688,8 @@ struct Planner {
         }
     }
 
-    void emit_layout(const std::vector<int> &oldRS, const std::vector<int> &RSv,
-                     const std::vector<int> &thr)
+    void emit_layout(const Bits &oldRS, const Bits &RSv,
+                     const Bits &thr)
     {
         TileOp op;
         memset(&op, 0, sizeof op);
@@ -675,26 +726,25 @@ struct Planner {
     // bits in ascending order, after those that are stored to the low qubits.
     // (lo: bits below it may not go to lanes 4, 5, used for the load layout,
     // whose lanes 0..klo-1 must hold the low bits.)
-    std::vector<int> thread_layout(const std::vector<int> &rs, const std::vector<long> *score,
+    Bits thread_layout(const Bits &rs, const Scores *score,
                                    int lo) const
     {
-        std::vector<int> avail;
+        Bits avail;
         for (int b = 0; b < K; b++)
             if (std::find(rs.begin(), rs.end(), b) == rs.end()) avail.push_back(b);
-        std::vector<int> thr(LOGW, -1);
+        Bits thr(LOGW, -1);
         if (swaps && LOGW >= 6 && score) {
-            std::vector<int> cand;
+            Bits cand;
             for (int b : avail)
                 if (b >= lo && (*score)[b] > 0) cand.push_back(b);
-            std::stable_sort(cand.begin(), cand.end(),
-                             [&](int x, int y) { return (*score)[x] > (*score)[y]; });
+            sort_bits(cand, [&](int x, int y) { return (*score)[x] > (*score)[y]; });
             for (int i = 0; i < 2 && i < (int)cand.size(); i++) {
                 thr[4 + i] = cand[i];
                 avail.erase(std::find(avail.begin(), avail.end(), cand[i]));
             }
         }
         if (!lo)
-            std::stable_sort(avail.begin(), avail.end(), [&](int x, int y) {
+            sort_bits(avail, [&](int x, int y) {
                 return std::find(outlow.begin(), outlow.end(), x) <
                        std::find(outlow.begin(), outlow.end(), y);
             });
@@ -706,11 +756,11 @@ struct Planner {
 
     // Swaps that turn register set rs (slots) into one holding exactly the
     // bits of `want`, if every missing bit sits on lane bit 4 or 5.
-    bool swap_path(const std::vector<int> &rs, const std::vector<int> &thr,
-                   const std::vector<int> &want, std::vector<std::pair<int, int>> *sw) const
+    bool swap_path(const Bits &rs, const Bits &thr,
+                   const Bits &want, std::vector<std::pair<int, int>> *sw) const
     {
         if (!swaps || LOGW < 6) return false;
-        std::vector<int> in, out;
+        Bits in, out;
         for (int b : want)
             if (std::find(rs.begin(), rs.end(), b) == rs.end()) in.push_back(b);
         for (int j = 0; j < RB; j++)
@@ -724,7 +774,7 @@ struct Planner {
         return true;
     }
 
-    void apply_swaps(std::vector<int> &rs, std::vector<int> &thr,
+    void apply_swaps(Bits &rs, Bits &thr,
                      const std::vector<std::pair<int, int>> &sw) const
     {
         for (auto [j, tb] : sw) std::swap(rs[j], thr[tb]);
@@ -763,7 +813,7 @@ struct Planner {
     // Register targets still to run, weighted by readiness: a ready gate counts
     // for more than all the waiting ones together, so that the best-scored bit
     // always has a ready gate (a gate that waits never outranks what it waits for).
-    void pair_score(const std::vector<Todo> &todo, std::vector<long> &score) const
+    void pair_score(const std::vector<Todo> &todo, Scores &score) const
     {
         const long ready_weight = std::max<long>(1000, (long)todo.size() + 1);
         score.assign(K, 0);
@@ -785,17 +835,16 @@ struct Planner {
     // swaps is charged less than one that needs an LDS transpose (in gates
     // that could have run: a transpose costs about four gates, a swap about
     // half of one).
-    std::vector<int> best_set(const std::vector<Todo> &todo, const std::vector<long> &score, int lo,
-                              const std::vector<int> *cur_rs = nullptr,
-                              const std::vector<int> *cur_thr = nullptr) const
+    Bits best_set(const std::vector<Todo> &todo, const Scores &score, int lo,
+                              const Bits *cur_rs = nullptr,
+                              const Bits *cur_thr = nullptr) const
     {
         const int left = (int)todo.size();
-        std::vector<int> bits;
+        Bits bits;
         for (int b = lo; b < K; b++) bits.push_back(b);
-        std::stable_sort(bits.begin(), bits.end(),
-                         [&](int x, int y) { return score[x] > score[y]; });
+        sort_bits(bits, [&](int x, int y) { return score[x] > score[y]; });
         if (quick) {
-            std::vector<int> out(bits.begin(), bits.begin() + RB);
+            Bits out(bits.begin(), bits.begin() + RB);
             std::sort(out.begin(), out.end());
             return out;
         }
@@ -805,7 +854,7 @@ struct Planner {
         long best_sc = -1;
         uint64_t all = 0;
         for (const Todo &g : todo) all |= g.nd | g.dm;
-        std::vector<int> want;
+        Bits want;
         std::vector<std::pair<int, int>> sw;
         for (uint32_t sub = 0; sub < (1u << T); sub++) {
             if (__builtin_popcount(sub) != RB) continue;
@@ -843,7 +892,7 @@ struct Planner {
                 best_sc = sc;
             }
         }
-        std::vector<int> out;
+        Bits out;
         if (best_val == -1e30) {
             // nothing runs under any candidate: possible only for the load
             // layout, where every ready target may be a low bit (from lo = 0 the
@@ -867,11 +916,12 @@ struct Planner {
     // the most ready pair gates, and lane bits 4 and 5 holding the next
     // best-scored bits).
     void sequence(const std::vector<SG> &run, const std::vector<int> &order, const int *lbit,
-                  std::vector<int> &seq, std::vector<Change> &changes, std::vector<int> &rs_in,
-                  std::vector<int> &thr_in)
+                  std::vector<int> &seq, std::vector<Change> &changes, Bits &rs_in,
+                  Bits &thr_in)
     {
         const int m = (int)order.size();
-        std::vector<int> RS(RB);
+        seq.reserve(m + m / 2 + 8);
+        Bits RS(RB);
         for (int j = 0; j < RB; j++) RS[j] = LOGW + j;
         auto in_rs = [&](int b) {
             for (int j = 0; j < RB; j++)
@@ -883,23 +933,23 @@ struct Planner {
             const SG &g = run[order[a]];
             todo[a] = {g.nd, g.dm, needs_reg(g) ? 1u << lbit[g.target] : 0u, a};
         }
-        std::vector<long> score0;
+        Scores score0;
         pair_score(todo, score0);
         if (!strict && K - klo >= RB) RS = best_set(todo, score0, klo);
-        std::vector<int> THR = thread_layout(RS, &score0, klo);
+        Bits THR = thread_layout(RS, &score0, klo);
         rs_in = RS;
         thr_in = THR;
         // move to register bits `nx` (slot order as given): swaps when they
         // reach it, else an LDS transpose whose lane bits 4, 5 get the
         // best-scored free bits
-        auto change_to = [&](const std::vector<int> &nx, const std::vector<long> &score) {
+        auto change_to = [&](const Bits &nx, const Scores &score) {
             Change ch;
             if (swap_path(RS, THR, nx, &ch.sw)) {
                 ch.lds = false;
                 apply_swaps(RS, THR, ch.sw);
             } else {
                 // keep bits that stay in place in their old slots
-                std::vector<int> slotted(RB, -1);
+                Bits slotted(RB, -1);
                 for (int j = 0; j < RB; j++)
                     if (std::find(nx.begin(), nx.end(), RS[j]) != nx.end()) slotted[j] = RS[j];
                 for (int b : nx) {
@@ -919,8 +969,8 @@ struct Planner {
             for (int pos = 0; pos < m; pos++) {
                 const SG &g = run[order[pos]];
                 if (!g.diag && !in_rs(lbit[g.target])) {
-                    std::vector<int> nx;
-                    std::vector<long> score(K, 0);
+                    Bits nx;
+                    Scores score(K, 0);
                     for (int p2 = pos; p2 < m; p2++) {
                         // (scores only place lanes 4 and 5, for swaps)
                         if (!swaps && (int)nx.size() == RB) break;
@@ -955,7 +1005,8 @@ struct Planner {
             return;
         }
         std::vector<Todo> stuck;
-        std::vector<long> score;
+        Scores score;
+        stuck.reserve(m);
         for (;;) {
             // every gate that runs under the current register bits, in order
             uint32_t rs = 0;
@@ -978,7 +1029,7 @@ struct Planner {
             // scored bits, take the one under which the most gates run
             // before the next change, less the cost of reaching it
             pair_score(todo, score);
-            std::vector<int> nx = best_set(todo, score, 0, &RS, &THR);
+            Bits nx = best_set(todo, score, 0, &RS, &THR);
             change_to(nx, score);
             if ((int)changes.size() > 2 * m + 8) {  // every change runs a gate: cannot happen
                 bad = true;
@@ -1062,11 +1113,12 @@ struct Planner {
         }
         sw.op_begin = prog.size();
         sw.slot_begin = grads.size();
-        std::vector<int> seq, RS, THR;
+        std::vector<int> seq;
+        Bits RS, THR;
         std::vector<Change> changes;
         sequence(run, order, lbit, seq, changes, RS, THR);
         // load layout: register bits RS, thread bits THR
-        auto reg_offsets = [&](const std::vector<int> &rs, const int8_t *qubit, uint64_t *out) {
+        auto reg_offsets = [&](const Bits &rs, const int8_t *qubit, uint64_t *out) {
             for (int p = 0; p < (1 << RB); p++) {
                 uint64_t g = 0;
                 for (int j = 0; j < RB; j++)
@@ -1288,7 +1340,7 @@ struct Planner {
         // (then those register bits are swapped for unused high bits) or the
         // low lane bits do not hold the low local bits in order
         {
-            std::vector<int> st = RS;
+            Bits st = RS;
             uint32_t used = 0;
             for (int b : RS) used |= 1u << b;
             int nb = K - 1;
@@ -1363,6 +1415,7 @@ struct Planner {
     {
         std::vector<int> rem(run.size());
         for (size_t i = 0; i < run.size(); i++) rem[i] = (int)i;
+        prog.reserve(run.size() + run.size() / 4 + 8);
         while (!rem.empty()) {
             uint64_t smask;
             std::vector<int> order = collect(run, rem, smask);
@@ -1766,9 +1819,14 @@ static int collect_run(const spz_state_s *s, const spz_op *ops, uint64_t n_ops,
 // Plans a run whose sweeps are all tile sweeps.
 static int plan_tiles(Planner &pl, const std::vector<SG> &run, ChipPlan &out)
 {
+    out.prog.clear();
+    out.grads.clear();
+    pl.prog.swap(out.prog);  // (their memory is used again)
+    pl.grads.swap(out.grads);
     pl.plan(run);
     if (pl.bad) return fail(SPZ_ERR_ARG, "tile planner produced a gate outside the register layout");
     out.sweeps.clear();
+    out.sweeps.reserve(pl.sweeps.size());
     for (const Sweep &sw : pl.sweeps)
         out.sweeps.push_back({sw.desc, (uint32_t)sw.op_begin, (uint32_t)sw.op_count,
                               (uint32_t)sw.slot_begin, (uint32_t)sw.slots});
