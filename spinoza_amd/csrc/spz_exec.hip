@@ -2008,6 +2008,20 @@ static bool plain_swap(const spz_op &o, int n)
     return !(c & sw) && !(o.ones & o.zeros) && !(c >> n);
 }
 
+// A run of so few ops goes op by op in small states too: the one launch costs its
+// program's copy and a workgroup's start.  3 to 12 qubits, one op 4.2 us and (in
+// one launch) 12-13.5, four 12.0 and 14-17, five 14.6 and 14.6-17, six 17.3 and
+// 15-19, eight 22.3 and 16-19.6; waited for after each call 12.5 and 21 (one op),
+// 22.6 and 23.5 (five), 25 and 24 (six).
+constexpr int kShortRun = 5;
+
+static int ops_of(const std::vector<SG> &run)
+{
+    int n = 0;  // (a SWAP is several gates)
+    for (size_t i = 0; i < run.size(); i++) n += i == 0 || run[i].op_index != run[i - 1].op_index;
+    return n;
+}
+
 // How a run takes SWAPs: one launch as CX, tile sweeps as a relabelling where no
 // qubit controls it.
 static bool takes_swap(const spz_op &o, int n, Swaps how)
@@ -2047,7 +2061,9 @@ int plan_info(int n, int prec, const spz_op *ops, uint64_t n_ops, const spz_exec
         uint64_t j = i;
         SPZ_TRY(collect_run(&st, ops, n_ops, nullptr, how, &j, run));
         if (small) {
-            if (!run.empty()) {
+            if (ops_of(run) <= kShortRun) {
+                out->plain_gates += ops_of(run);
+            } else {
                 ChipPlan cp;
                 SPZ_TRY(plan_chip(n, run, true, false, cp));
                 out->sweeps += cp.sweeps.size();
@@ -2159,9 +2175,12 @@ int execute_ops(spz_state_s *s, const spz_op *ops, uint64_t n_ops, spz_tracker *
         std::vector<SG> run;
         uint64_t j = i;
         SPZ_TRY(collect_run(s, ops, n_ops, trk, how, &j, run));
-        if (!run.empty())
+        if (small && ops_of(run) <= kShortRun) {
+            for (; i < j; i++) SPZ_TRY(exec_one_plain(s, ops[i], trk, nullptr));
+        } else if (!run.empty()) {
             SPZ_TRY(small ? run_chip(s, run)
                           : dense5 ? run_dense5(s, run) : run_fused(s, run, K, strict));
+        }
         i = j;
     }
     return SPZ_OK;
