@@ -59,14 +59,30 @@ __device__ __forceinline__ void expect_reg(const double *a, const double *b, dou
         add_term(s, c, expect_term<OBS>((e & BIT) != 0, a[e], b[e], a[e ^ BIT], b[e ^ BIT]));
 }
 
-template <typename T, char OBS>
+// Which of j and its partner over q forms the sum of both: for q = 6 and 7 the one
+// with the bit clear; for the block bits above 12 in even blocks that one, in odd
+// blocks the other, so that both halves of a state, which run on different XCDs
+// (xcd_block), have as much to do (qubit 21 of 22 alone, a whole call: 40 us with
+// the clear side only, 30 now; 34 when every amplitude formed its own).
+__device__ __forceinline__ bool forms_sum(uint64_t j, int q)
+{
+    const uint64_t odd = q > 12 ? j >> 12 : 0;
+    return (((j >> q) ^ odd) & 1) == 0;
+}
+
+// G: the most targets of the launch.  One alone needs 4 KiB of LDS instead of 32,
+// so more workgroups share a CU (x on qubit 0, a whole call: 23 qubits FP64 42 ->
+// 38 us, 25 qubits FP32 76 -> 59), and blocks whose sum the partner forms end at once.
+template <typename T, char OBS, int G>
 __global__ void __launch_bounds__(kRT)
 k_expect(const T *__restrict__ re, const T *__restrict__ im, uint64_t nb, Targets tg,
          double *__restrict__ partials)
 {
-    __shared__ double S[kExpectGroup][kRT], C[kExpectGroup][kRT];
+    __shared__ double S[G][kRT], C[G][kRT];
     const uint32_t tid = threadIdx.x;
     const uint64_t blk = xcd_block(blockIdx.x, nb), base = blk * kRB;
+    if constexpr (G == 1 && OBS != 'z')  // (a block whose only sum its partner forms)
+        if (tg.q[0] >= 12 && !forms_sum(base, tg.q[0])) return;
     double a[kRE], b[kRE];
 #pragma unroll
     for (int e = 0; e < kRE; e++) {
@@ -77,7 +93,8 @@ k_expect(const T *__restrict__ re, const T *__restrict__ im, uint64_t nb, Target
 #pragma unroll
         for (int e = 0; e < kRE; e++) a[e] = a[e] * a[e] + b[e] * b[e];
     }
-    for (int t = 0; t < tg.count; t++) {
+    const int count = G == 1 ? 1 : tg.count;
+    for (int t = 0; t < count; t++) {
         const int q = tg.q[t];
         double s = 0.0, c = 0.0;
         if constexpr (OBS == 'z') {  // a (-a) + b (-b) is exactly -(a a + b b)
@@ -108,11 +125,12 @@ k_expect(const T *__restrict__ re, const T *__restrict__ im, uint64_t nb, Target
         } else {
             // An amplitude and its partner have the same X and Y term, so a
             // thread and its partner thread (q = 6, 7: another wavefront),
-            // and a block and its partner block, have the same sums: the
-            // side with the bit clear forms them for both.
+            // and a block and its partner block, have the same sums: one
+            // side (forms_sum) forms them for both.
             const uint64_t j0 = base + tid;
-            if ((j0 >> q) & 1) continue;
-            const uint64_t p0 = j0 | (1ull << q);
+            if (!forms_sum(j0, q)) continue;
+            const uint64_t p0 = j0 ^ (1ull << q);
+            const bool bit = ((j0 >> q) & 1) != 0;
             T x[kRE], y[kRE];
 #pragma unroll
             for (int e = 0; e < kRE; e++) {
@@ -121,7 +139,7 @@ k_expect(const T *__restrict__ re, const T *__restrict__ im, uint64_t nb, Target
             }
 #pragma unroll
             for (int e = 0; e < kRE; e++)
-                add_term(s, c, expect_term<OBS>(false, a[e], b[e], x[e], y[e]));
+                add_term(s, c, expect_term<OBS>(bit, a[e], b[e], x[e], y[e]));
             if (q < 8) {
                 S[t][tid | (1u << q)] = s;
                 C[t][tid | (1u << q)] = c;
@@ -134,7 +152,7 @@ k_expect(const T *__restrict__ re, const T *__restrict__ im, uint64_t nb, Target
     // the halving tree of every target at once
     for (int lh = 7; lh >= 0; lh--) {
         const uint32_t h = 1u << lh;
-        for (uint32_t i = tid; i < (uint32_t)tg.count << lh; i += kRT) {
+        for (uint32_t i = tid; i < (uint32_t)count << lh; i += kRT) {
             const uint32_t t = i >> lh, k = i & (h - 1);
             double ns, e;
             two_sum(S[t][k], S[t][k + h], ns, e);
@@ -143,14 +161,14 @@ k_expect(const T *__restrict__ re, const T *__restrict__ im, uint64_t nb, Target
         }
         __syncthreads();
     }
-    if ((int)tid < tg.count) {
+    if ((int)tid < count) {
         const int q = tg.q[tid];
         double *p = partials + 2 * (uint64_t)tid * nb;
-        if (OBS == 'z' || q < 12 || !((base >> q) & 1)) {
+        if (OBS == 'z' || q < 12 || forms_sum(base, q)) {
             p[2 * blk] = S[tid][0];
             p[2 * blk + 1] = C[tid][0];
             if (OBS != 'z' && q >= 12) {
-                const uint64_t other = blk | (1ull << (q - 12));
+                const uint64_t other = blk ^ (1ull << (q - 12));
                 p[2 * other] = S[tid][0];
                 p[2 * other + 1] = C[tid][0];
             }
@@ -200,12 +218,18 @@ void launch_expect(const spz_state_s *s, char obs, uint64_t nb, const Targets &t
     const T *re = (const T *)s->re, *im = (const T *)s->im;
     const dim3 g((unsigned)nb), b(kRT);
     hipStream_t st = rt().stream;
-    if (obs == 'x')
-        hipLaunchKernelGGL((k_expect<T, 'x'>), g, b, 0, st, re, im, nb, tg, part);
-    else if (obs == 'y')
-        hipLaunchKernelGGL((k_expect<T, 'y'>), g, b, 0, st, re, im, nb, tg, part);
-    else
-        hipLaunchKernelGGL((k_expect<T, 'z'>), g, b, 0, st, re, im, nb, tg, part);
+#define SPZ_EX(OBS)                                                                          \
+    do {                                                                                     \
+        if (tg.count == 1)                                                                     \
+            hipLaunchKernelGGL((k_expect<T, OBS, 1>), g, b, 0, st, re, im, nb, tg, part);          \
+        else                                                                                 \
+            hipLaunchKernelGGL((k_expect<T, OBS, kExpectGroup>), g, b, 0, st, re, im, nb, tg,       \
+                               part);                                                        \
+    } while (0)
+    if (obs == 'x') SPZ_EX('x');
+    else if (obs == 'y') SPZ_EX('y');
+    else SPZ_EX('z');
+#undef SPZ_EX
 }
 
 }  // namespace
