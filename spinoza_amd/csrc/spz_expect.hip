@@ -189,12 +189,13 @@ k_finish(const double *__restrict__ partials, uint64_t nb, double *__restrict__ 
 //
 // Bound: the partner loads of the qubits above the block (one state read each,
 // from L2 where the partner block is in flight on the same XCD, else from the
-// memory-side cache): 11 reads of 134 MB at 23 qubits in 192 us (195 with one
-// thread per term; wavefront, register and loaded partners cost the same
-// there).  With H psi kept, 24 qubits: 464 us for both, where a pass for H psi
-// (504) and one for the energy (99) took 603.
+// memory-side cache): 11 reads of 134 MB at 23 qubits.  Whole calls for the energy
+// and for both with H psi, FP64: 23 qubits 190 and 218 us, 24 qubits 390-402 and 445,
+// 28 qubits 8.6 and 9.1 ms.  Two waves per SIMD, whose 256 registers hold the block
+// and the partners on their way, not three (168): 211 and 245, 430 and 488 us, 8.8
+// and 9.3 ms.  One thread per term: 210 and 346, 403 and 730 us, 9.9 and 13.6 ms.
 template <typename T, bool STORE>
-__global__ void __launch_bounds__(kRT) __attribute__((amdgpu_waves_per_eu(3, 3)))
+__global__ void __launch_bounds__(kRT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_ising(const T *__restrict__ re, const T *__restrict__ im, T *__restrict__ lr,
         T *__restrict__ li, uint64_t nb, int n, double hx, double *__restrict__ partials)
 {

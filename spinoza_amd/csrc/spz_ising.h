@@ -42,7 +42,7 @@ __device__ __forceinline__ void ising_block(const T *__restrict__ re, const T *_
     }
     auto far = [&](int q) {
         const uint64_t p0 = (base + tid) ^ (1ull << q);
-        // a quarter of the block at a time keeps three waves per SIMD
+        // a quarter of the block at a time (half of it measured the same)
 #pragma unroll
         for (int h = 0; h < kRE; h += kRE / 4) {
             T x[kRE / 4], y[kRE / 4];
