@@ -35,6 +35,8 @@ constexpr uint32_t kBlock = 4096;      // indices per block of the sampling rule
 constexpr uint32_t kPiece = 1u << 20;  // uniforms per round (bounds the scratch)
 constexpr uint32_t kPer = 1024;        // samples a workgroup picks (4 per thread)
 constexpr uint32_t kFew = 64;          // blocks counted in LDS first
+constexpr uint64_t kHostBlocks = 1u << 12;  // blocks whose sums the host forms
+constexpr uint64_t kHostPiece = 1u << 20;   // ... so many at a time
 constexpr uint32_t kDirect = 1u << 14; // samples a call reads and writes in pinned memory
 
 struct SampleMeta {
@@ -140,6 +142,35 @@ k_block_prefix(const double *__restrict__ pairs, uint64_t nb, double *__restrict
     }
 }
 
+// The same for many blocks, whose sums the host forms (block_prefix_on_host): their
+// way to pinned memory and back, and the start of a round.
+__global__ void __launch_bounds__(kT)
+k_block_sums(const double *__restrict__ pairs, uint64_t cnt, double *__restrict__ host_v)
+{
+    const uint64_t b = (uint64_t)blockIdx.x * kT + threadIdx.x;
+    if (b < cnt) host_v[b] = pairs[2 * b] + pairs[2 * b + 1];
+}
+
+__global__ void __launch_bounds__(kT)
+k_take_sums(const double *__restrict__ host_v, uint64_t cnt, double *__restrict__ P)
+{
+    const uint64_t b = (uint64_t)blockIdx.x * kT + threadIdx.x;
+    if (b < cnt) P[b] = host_v[b];
+}
+
+__global__ void __launch_bounds__(kT)
+k_sample_begin(uint32_t *__restrict__ counts, uint64_t nb, double *__restrict__ P,
+               SampleMeta *__restrict__ meta, SampleMeta *__restrict__ host_meta, SampleMeta m)
+{
+    const uint64_t b = (uint64_t)blockIdx.x * kT + threadIdx.x;
+    if (b < nb) counts[b] = 0u;
+    if (b == 0) {
+        P[nb] = m.total;
+        *meta = m;
+        if (host_meta) host_meta->lastnz = m.lastnz;
+    }
+}
+
 // The block of every uniform, and its rank among the block's samples.  With few
 // blocks (kFew) a workgroup counts in LDS and takes its places at once: the
 // samples of a state of one block would queue at one address (10000 samples of
@@ -185,7 +216,10 @@ k_sample_block(const double *__restrict__ P, uint64_t nb, const SampleMeta *__re
 
 // Exclusive scan of the counts (in place: counts[b] becomes the block's first
 // position) and the list of the blocks' samples, at most kPer to a slot.  One
-// workgroup.
+// workgroup, kScan blocks to a thread at a time (one to a thread took 0.1 ms more
+// for 2^18 blocks).
+constexpr int kScan = 8;
+
 __global__ void __launch_bounds__(kPT)
 k_sample_scan(uint32_t *__restrict__ counts, uint64_t nb, Slot *__restrict__ slots,
               SampleMeta *__restrict__ meta)
@@ -193,10 +227,17 @@ k_sample_scan(uint32_t *__restrict__ counts, uint64_t nb, Slot *__restrict__ slo
     __shared__ uint32_t ws[kPT / 64], wz[kPT / 64];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     uint32_t base_s = 0, base_z = 0;
-    for (uint64_t b0 = 0; b0 < nb; b0 += kPT) {
-        const uint64_t b = b0 + tid;
-        const uint32_t c = b < nb ? counts[b] : 0u;
-        uint32_t s = c, z = (c + kPer - 1) / kPer;  // inclusive scans over the wavefront
+    for (uint64_t b0 = 0; b0 < nb; b0 += kPT * kScan) {
+        const uint64_t b = b0 + (uint64_t)tid * kScan;
+        uint32_t c[kScan], cs = 0, cz = 0;
+#pragma unroll
+        for (int i = 0; i < kScan; i++) c[i] = b + i < nb ? counts[b + i] : 0u;
+#pragma unroll
+        for (int i = 0; i < kScan; i++) {
+            cs += c[i];
+            cz += (c[i] + kPer - 1) / kPer;
+        }
+        uint32_t s = cs, z = cz;  // inclusive scans over the wavefront
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
             const uint32_t us = __shfl_up(s, d), uz = __shfl_up(z, d);
@@ -210,7 +251,7 @@ k_sample_scan(uint32_t *__restrict__ counts, uint64_t nb, Slot *__restrict__ slo
             wz[wave] = z;
         }
         __syncthreads();
-        uint32_t os = base_s, oz = base_z;
+        uint32_t os = base_s + s - cs, oz = base_z + z - cz;
         for (uint32_t w = 0; w < kPT / 64; w++) {
             if (w < wave) {
                 os += ws[w];
@@ -219,10 +260,13 @@ k_sample_scan(uint32_t *__restrict__ counts, uint64_t nb, Slot *__restrict__ slo
             base_s += ws[w];
             base_z += wz[w];
         }
-        if (b < nb) counts[b] = os + s - c;
-        const uint32_t nz = (c + kPer - 1) / kPer;
-        for (uint32_t i = 0; i < nz; i++)
-            slots[oz + z - nz + i] = Slot{(uint32_t)b, os + s - c + i * kPer, min(c - i * kPer, kPer)};
+#pragma unroll
+        for (int i = 0; i < kScan; i++) {
+            if (b + i < nb) counts[b + i] = os;
+            for (uint32_t at = 0; at < c[i]; at += kPer)
+                slots[oz++] = Slot{(uint32_t)(b + i), os + at, min(c[i] - at, kPer)};
+            os += c[i];
+        }
         __syncthreads();
     }
     if (tid == 0) meta->nslots = base_z;
@@ -406,6 +450,38 @@ int sample_one(const spz_state_s *s, const double *uniforms, uint64_t k, uint64_
     return SPZ_OK;
 }
 
+// P[0..nb-1] in device memory, the total and the last positive block from the level-1
+// pairs in rt().d_partials, the additions by the host in the same order: it makes
+// one in 1.2 ns where a lane of the GPU takes 5.5, which pays for the blocks' sums
+// crossing the bus twice from kHostBlocks blocks on (one sample, the GPU's lane and
+// the host: 23 qubits 95 us both, 24 qubits 130 and 118, 26 360 and 270, 28 1260 and
+// 860, 30 5.0 and 3.3 ms, 32 in FP32 15.1 and 8.4).  `v`: pinned, kHostPiece values.
+int block_prefix_on_host(uint64_t nb, double *P, double *v, SampleMeta *m)
+{
+    hipStream_t st = rt().stream;
+    double acc = 0.0;
+    m->lastnz = -1;
+    m->nslots = 0;
+    m->pad = 0;
+    for (uint64_t at = 0; at < nb; at += kHostPiece) {
+        const uint64_t cnt = std::min(kHostPiece, nb - at);
+        const dim3 g((unsigned)((cnt + kT - 1) / kT)), t(kT);
+        hipLaunchKernelGGL(k_block_sums, g, t, 0, st, rt().d_partials + 2 * at, cnt, v);
+        SPZ_HIP(hipGetLastError());
+        SPZ_HIP(hipStreamSynchronize(st));
+        for (uint64_t b = 0; b < cnt; b++) {
+            const double w = v[b];
+            v[b] = acc;
+            acc = acc + w;
+            if (w > 0.0) m->lastnz = (int64_t)(at + b);
+        }
+        hipLaunchKernelGGL(k_take_sums, g, t, 0, st, v, cnt, P + at);
+        SPZ_HIP(hipGetLastError());
+    }
+    m->total = acc;
+    return SPZ_OK;
+}
+
 int sample_rounds(const spz_state_s *s, uint64_t nb, const double *uniforms, uint64_t k,
                   uint64_t *out)
 {
@@ -421,7 +497,9 @@ int sample_rounds(const spz_state_s *s, uint64_t nb, const double *uniforms, uin
     // (16 to 20 qubits, one sample 71 -> 65 us, 4096 103 -> 76, 16384 118 -> 106;
     // the picks' scattered stores over the bus catch up with the copies there)
     const bool direct = k <= kDirect;
-    SPZ_TRY(reserve(dev_bytes, direct ? o_u + up(piece * 8ull) : o_u));
+    const bool on_host = nb >= kHostBlocks;
+    const size_t o_stage = direct ? o_u + up(piece * 8ull) : o_u;
+    SPZ_TRY(reserve(dev_bytes, o_stage + (on_host ? std::min(nb, kHostPiece) * sizeof(double) : 0)));
     char *d = (char *)g_scr.dev, *h = (char *)g_scr.host;
     SampleMeta *meta = (SampleMeta *)(d + o_meta);
     double *U = (double *)((direct ? h : d) + o_u), *P = (double *)(d + o_p);
@@ -432,6 +510,11 @@ int sample_rounds(const spz_state_s *s, uint64_t nb, const double *uniforms, uin
     SampleMeta *host_meta = (SampleMeta *)(h + o_meta);
     hipStream_t st = rt().stream;
     LaunchTimer tm(SPZ_K_OTHER, 0.0);
+    SampleMeta first;
+    if (on_host) {
+        SPZ_TRY(block_prefix_on_host(nb, P, (double *)(h + o_stage), &first));
+        if (first.lastnz < 0) return fail(SPZ_ERR_PROB, "sampling a zero state");
+    }
     for (uint64_t at = 0; at < k; at += piece) {
         const uint32_t m = (uint32_t)std::min<uint64_t>(piece, k - at);
         // (the previous round was waited for: the staging buffer is free)
@@ -439,8 +522,12 @@ int sample_rounds(const spz_state_s *s, uint64_t nb, const double *uniforms, uin
         if (!direct)
             SPZ_HIP(hipMemcpyAsync(U, h, m * sizeof(double), hipMemcpyHostToDevice, st));
         const unsigned g = (m + kT - 1) / kT;
-        hipLaunchKernelGGL(k_block_prefix, dim3(1), dim3(kPT), 0, st, rt().d_partials, nb, P,
-                           counts, meta, direct ? host_meta : nullptr);
+        if (on_host)
+            hipLaunchKernelGGL(k_sample_begin, dim3((unsigned)((nb + kT - 1) / kT)), dim3(kT), 0, st,
+                               counts, nb, P, meta, direct ? host_meta : nullptr, first);
+        else
+            hipLaunchKernelGGL(k_block_prefix, dim3(1), dim3(kPT), 0, st, rt().d_partials, nb, P,
+                               counts, meta, direct ? host_meta : nullptr);
         hipLaunchKernelGGL(k_sample_block, dim3(g), dim3(kT), 0, st, P, nb, meta, U, m, counts,
                            blk, rank);
         hipLaunchKernelGGL(k_sample_scan, dim3(1), dim3(kPT), 0, st, counts, nb, slots, meta);
