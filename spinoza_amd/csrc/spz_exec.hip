@@ -1537,8 +1537,17 @@ struct Release {
     }
 };
 
+// One gate of a run by itself.
+int run_one(spz_state_s *s, const SG &g)
+{
+    if (g.kind == SPZ_SWAP) return launch_swap(s, g.target, g.t1, 0, 0);
+    return g.diag ? launch_diag(s, g.k, g.target, g.ones, g.zeros)
+                  : launch_pair(s, g.k, g.target, g.ones, g.zeros);
+}
+
 int run_fused(spz_state_s *s, const std::vector<SG> &run, int K, bool strict)
 {
+    if (run.size() == 1) return run_one(s, run[0]);  // (what its plan would say)
     Planner pl;
     pl.n = s->n;
     pl.K = K;
@@ -1596,10 +1605,7 @@ int run_fused(spz_state_s *s, const std::vector<SG> &run, int K, bool strict)
         if (sw.tile) {
             SPZ_TRY(launch_tile(s, K, sw.desc, d_prog + sw.op_begin, pl.fast));
         } else {
-            const SG &g = run[sw.gate];
-            if (g.kind == SPZ_SWAP) SPZ_TRY(launch_swap(s, g.target, g.t1, 0, 0));
-            else if (g.diag) SPZ_TRY(launch_diag(s, g.k, g.target, g.ones, g.zeros));
-            else SPZ_TRY(launch_pair(s, g.k, g.target, g.ones, g.zeros));
+            SPZ_TRY(run_one(s, run[sw.gate]));
         }
     }
     return SPZ_OK;
@@ -2015,19 +2021,21 @@ static bool plain_swap(const spz_op &o, int n)
 // 22.6 and 23.5 (five), 25 and 24 (six).
 constexpr int kShortRun = 5;
 
-static int ops_of(const std::vector<SG> &run)
-{
-    int n = 0;  // (a SWAP is several gates)
-    for (size_t i = 0; i < run.size(); i++) n += i == 0 || run[i].op_index != run[i - 1].op_index;
-    return n;
-}
-
 // How a run takes SWAPs: one launch as CX, tile sweeps as a relabelling where no
 // qubit controls it.
 static bool takes_swap(const spz_op &o, int n, Swaps how)
 {
     return how != Swaps::BARRIER && plain_swap(o, n) &&
            (how == Swaps::AS_CX || !(o.ones | o.zeros));
+}
+
+// The end of the run at `i` if it has at most kShortRun ops, else `i`.
+static uint64_t short_run(const spz_op *ops, uint64_t i, uint64_t n_ops, int n, Swaps how)
+{
+    uint64_t e = i;
+    for (; e < n_ops && (!is_barrier(ops[e]) || takes_swap(ops[e], n, how)); e++)
+        if (e - i == (uint64_t)kShortRun) return i;
+    return e;
 }
 
 // Planning only (no device work): how the tile executor would split `ops`.
@@ -2061,8 +2069,8 @@ int plan_info(int n, int prec, const spz_op *ops, uint64_t n_ops, const spz_exec
         uint64_t j = i;
         SPZ_TRY(collect_run(&st, ops, n_ops, nullptr, how, &j, run));
         if (small) {
-            if (ops_of(run) <= kShortRun) {
-                out->plain_gates += ops_of(run);
+            if (j - i <= (uint64_t)kShortRun) {
+                out->plain_gates += j - i;
             } else {
                 ChipPlan cp;
                 SPZ_TRY(plan_chip(n, run, true, false, cp));
@@ -2172,15 +2180,22 @@ int execute_ops(spz_state_s *s, const spz_op *ops, uint64_t n_ops, spz_tracker *
             i++;
             continue;
         }
+        if (const uint64_t end = small ? short_run(ops, i, n_ops, s->n, how) : i; end > i) {
+            for (; i < end; i++) {
+                const int rc = exec_one_plain(s, ops[i], trk, nullptr);
+                if (rc != SPZ_OK) {
+                    set_error("op " + std::to_string(i) + ": " + spz_last_error());
+                    return rc;
+                }
+            }
+            continue;
+        }
         std::vector<SG> run;
         uint64_t j = i;
         SPZ_TRY(collect_run(s, ops, n_ops, trk, how, &j, run));
-        if (small && ops_of(run) <= kShortRun) {
-            for (; i < j; i++) SPZ_TRY(exec_one_plain(s, ops[i], trk, nullptr));
-        } else if (!run.empty()) {
+        if (!run.empty())
             SPZ_TRY(small ? run_chip(s, run)
                           : dense5 ? run_dense5(s, run) : run_fused(s, run, K, strict));
-        }
         i = j;
     }
     return SPZ_OK;
