@@ -22,8 +22,10 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <condition_variable>
+#include <functional>
+#include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -191,43 +193,108 @@ struct Job {
     uint32_t width;     // workgroups it may use
 };
 
+// Threads that help the caller with a chunk's host work (plans, then the copies of
+// programs and descriptors to pinned memory, each by whoever is free), started when
+// they are first wanted and ended with the batch.  1000 circuits of 5 qubits, 10 and
+// 40 gates: threads started for every chunk's plans and copies by the caller alone
+// took 1.5 and 3.1 ms, this 1.04 and 2.5; 128 of 10 to 18 qubits the same 9.7.
+class Crew {
+    std::vector<std::thread> pool;
+    std::mutex mu;
+    std::condition_variable wake, idle;
+    std::function<void()> job;
+    uint64_t turn = 0;     // of the job that is up
+    unsigned places = 0;   // helpers the job still takes
+    unsigned working = 0;
+    bool stop = false;
+
+    void help()
+    {
+        uint64_t seen = 0;
+        std::unique_lock<std::mutex> lk(mu);
+        for (;;) {
+            wake.wait(lk, [&] { return stop || turn != seen; });
+            if (stop) return;
+            seen = turn;
+            if (!places) continue;
+            places--;
+            working++;
+            lk.unlock();
+            job();
+            lk.lock();
+            if (!--working) idle.notify_one();
+        }
+    }
+
+public:
+    ~Crew()
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            stop = true;
+        }
+        wake.notify_all();
+        for (std::thread &t : pool) t.join();
+    }
+
+    // Runs f here and on up to want - 1 helpers; f shares out the work by itself, ends
+    // when there is none left, and does not throw.
+    void run(uint64_t want, const std::function<void()> &f)
+    {
+        if (want > 1) {
+            try {
+                while (pool.size() + 1 < want) pool.emplace_back([this] { help(); });
+            } catch (const std::exception &) {
+                // no more threads to be had: the ones there are do the work
+            }
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                job = f;
+                turn++;
+                places = (unsigned)std::min<uint64_t>(want - 1, pool.size());
+            }
+            wake.notify_all();
+        }
+        f();
+        std::unique_lock<std::mutex> lk(mu);
+        places = 0;  // (whoever has not started need not)
+        idle.wait(lk, [&] { return !working; });
+    }
+};
+
+uint64_t most_threads(uint32_t count)
+{
+    const unsigned cores = std::max(1u, std::thread::hardware_concurrency());
+    return std::min<uint64_t>({(uint64_t)kPlanThreads, cores, count});
+}
+
 // Forward and reverse plans of a chunk's circuits.  Planning costs about half a
 // microsecond per circuit and 0.06 to 0.2 us per op in each direction, more than
 // the GPU takes for circuits of up to 12 qubits (180 of them: 6.0 ms planned by one
 // thread, 0.6 ms of sweeps), so a chunk is planned by several threads once there
 // is enough to pay for starting them (20 to 40 us each).
-int plan_chunk(const spz_batch_circuit *circuits, const spz_op *ops, const Job *jobs,
+int plan_chunk(Crew &crew, const spz_batch_circuit *circuits, const spz_op *ops, const Job *jobs,
                uint32_t count, std::vector<ChipPlan> &fwd, std::vector<ChipPlan> &rev)
 {
     uint64_t nops = 0;
     for (uint32_t c = 0; c < count; c++) nops += (uint64_t)circuits[jobs[c].circuit].n_ops;
     std::atomic<uint32_t> next{0};
     std::atomic<int> status{SPZ_OK};
-    auto work = [&]() {
+    const uint64_t cost = count + nops / 4;  // about so many us, both directions
+    crew.run(std::min(most_threads(count), cost / 150 + 1), [&]() {
         try {
             for (uint32_t c; status == SPZ_OK && (c = next++) < count;) {
                 const spz_batch_circuit &q = circuits[jobs[c].circuit];
                 const spz_op *o = ops + q.op_offset;
                 int rc = chip_plan(q.n, o, (uint64_t)q.n_ops, false, fwd[c]);
                 if (rc == SPZ_OK) rc = chip_plan(q.n, o, (uint64_t)q.n_ops, true, rev[c]);
+                if (rc == SPZ_OK && fwd[c].sweeps.empty()) fwd[c].sweeps.push_back(empty_sweep());
                 if (rc != SPZ_OK) status = rc;
             }
         } catch (const std::bad_alloc &) {
             status = SPZ_ERR_OOM;
         }
-    };
-    const unsigned cores = std::max(1u, std::thread::hardware_concurrency());
-    const uint64_t cost = count + nops / 4;  // about so many us, both directions
-    const uint64_t want = std::min<uint64_t>({(uint64_t)kPlanThreads, cores, count, cost / 150 + 1});
-    std::vector<std::thread> pool;
-    pool.reserve(kPlanThreads);
-    try {
-        for (uint64_t t = 1; t < want; t++) pool.emplace_back(work);
-    } catch (const std::system_error &) {
-        // no more threads to be had: the ones there are do the work
-    }
-    work();
-    for (std::thread &t : pool) t.join();
+    });
     if (status != SPZ_OK) return fail(status, "batched adjoint: planning failed");
     return SPZ_OK;
 }
@@ -240,6 +307,7 @@ struct Chunk {
     double hx;
     size_t lds;
     uint64_t grad0;
+    Crew &crew;
 
     int run(const Job *jobs, uint32_t count, uint32_t slot0, Scratch &sc, Slot &slot,
             hipEvent_t begin, hipEvent_t end)
@@ -252,10 +320,9 @@ struct Chunk {
         uint64_t amps = 0, pairs = 0, nops = 0;
         size_t nf = 0, nr = 0, ns = 0, lf = 0, lr = 0;
         uint32_t width = 0, blocks = 0;
-        SPZ_TRY(plan_chunk(circuits, ops, jobs, count, fwd, rev));
+        SPZ_TRY(plan_chunk(crew, circuits, ops, jobs, count, fwd, rev));
         for (uint32_t c = 0; c < count; c++) {
             const spz_batch_circuit &q = circuits[jobs[c].circuit];
-            if (fwd[c].sweeps.empty()) fwd[c].sweeps.push_back(empty_sweep());
             const uint64_t t = tiles_of(q.n);
             amps += 4 * (t << kChipK);
             pairs += rev[c].grads.size() * t * kChipRows + t;
@@ -279,34 +346,43 @@ struct Chunk {
         ChipIsing *hi = (ChipIsing *)(slot.host + o_i);
         ChipSum *hs = (ChipSum *)(slot.host + o_s);
         const TileOp *dp = (const TileOp *)slot.dev;
-        // programs, states and partial sums of every circuit
+        // where every circuit's programs, states and sums go, and its descriptors,
+        // which are in the order of the levels
         struct Place {
             double *psi, *part;
             uint64_t amps;
-            size_t fwd, rev;  // first op
+            size_t fwd, rev, sum;    // first op, first sum
+            size_t fwd_at, rev_at;   // in `order`
+        };
+        struct Level {
+            size_t first;
+            uint32_t count;
         };
         std::vector<Place> at(count);
-        double *amp = (double *)sc.states.p, *part = (double *)sc.parts.p;
-        size_t op = 0, sum = 0;
-        for (uint32_t c = 0; c < count; c++) {
-            const spz_batch_circuit &q = circuits[jobs[c].circuit];
-            const uint64_t t = tiles_of(q.n);
-            at[c] = {amp, part, t << kChipK, op, op + fwd[c].prog.size()};
-            for (const ChipPlan *p : {&fwd[c], &rev[c]}) {
-                if (!p->prog.empty()) memcpy(hp + op, p->prog.data(), p->prog.size() * sizeof(TileOp));
-                op += p->prog.size();
+        std::vector<Level> levels_f(lf, {0, 0}), levels_r(lr, {0, 0});
+        std::vector<size_t> order(nf + nr);  // a sweep's place among its level's
+        {
+            double *amp = (double *)sc.states.p, *part = (double *)sc.parts.p;
+            size_t op = 0, sum = 0, k = 0;
+            for (uint32_t c = 0; c < count; c++) {
+                const uint64_t t = tiles_of(circuits[jobs[c].circuit].n);
+                at[c] = {amp, part, t << kChipK, op, op + fwd[c].prog.size(), sum, k,
+                         k + fwd[c].sweeps.size()};
+                for (size_t l = 0; l < fwd[c].sweeps.size(); l++) order[k++] = levels_f[l].count++;
+                for (size_t l = 0; l < rev[c].sweeps.size(); l++) order[k++] = levels_r[l].count++;
+                op += fwd[c].prog.size() + rev[c].prog.size();
+                sum += rev[c].grads.size() + 1;
+                amp += 4 * at[c].amps;
+                part += 2 * (rev[c].grads.size() * t * kChipRows + t);
             }
-            for (size_t k = 0; k < rev[c].grads.size(); k++)
-                hs[sum++] = {part + 2 * k * t * kChipRows, (uint32_t)(t * kChipRows),
-                             (uint32_t)(grad0 + q.grad_offset + rev[c].grads[k])};
-            double *ep = part + 2 * rev[c].grads.size() * t * kChipRows;
-            hs[sum++] = {ep, (uint32_t)t, slot0 + c};
-            const uint64_t A = at[c].amps;
-            hi[c] = {amp, amp + A, amp + 2 * A, amp + 3 * A, 1ull << q.n, ep, (uint32_t)t, q.n};
-            amp += 4 * A;
-            part = ep + 2 * t;
+            for (auto *ls : {&levels_f, &levels_r}) {
+                size_t first = 0;
+                for (Level &l : *ls) {
+                    l.first = first;
+                    first += l.count;
+                }
+            }
         }
-        // descriptors, level by level
         auto fill = [&](ChipSweep &d, uint32_t c, const ChipPlan::Sweep &s, size_t first_op) {
             memset(&d, 0, sizeof d);
             chip_geometry(s, circuits[jobs[c].circuit].n, SPZ_F64, d);
@@ -320,33 +396,36 @@ struct Chunk {
             d.width = jobs[c].width;
             d.flags = CHIP_STORE;
         };
-        struct Level {
-            size_t first;
-            uint32_t count;
+        auto write = [&](uint32_t c) {
+            const spz_batch_circuit &q = circuits[jobs[c].circuit];
+            const uint64_t t = tiles_of(q.n), A = at[c].amps;
+            const ChipPlan &f = fwd[c], &r = rev[c];
+            if (!f.prog.empty()) memcpy(hp + at[c].fwd, f.prog.data(), f.prog.size() * sizeof(TileOp));
+            if (!r.prog.empty()) memcpy(hp + at[c].rev, r.prog.data(), r.prog.size() * sizeof(TileOp));
+            ChipSum *sum = hs + at[c].sum;
+            for (size_t k = 0; k < r.grads.size(); k++)
+                *sum++ = {at[c].part + 2 * k * t * kChipRows, (uint32_t)(t * kChipRows),
+                          (uint32_t)(grad0 + q.grad_offset + r.grads[k])};
+            double *ep = at[c].part + 2 * r.grads.size() * t * kChipRows, *psi = at[c].psi;
+            *sum = {ep, (uint32_t)t, slot0 + c};
+            hi[c] = {psi, psi + A, psi + 2 * A, psi + 3 * A, 1ull << q.n, ep, (uint32_t)t, q.n};
+            for (size_t l = 0; l < f.sweeps.size(); l++) {
+                ChipSweep &d = hf[levels_f[l].first + order[at[c].fwd_at + l]];
+                fill(d, c, f.sweeps[l], at[c].fwd);
+                if (l == 0) d.flags |= CHIP_INIT;
+            }
+            for (size_t l = 0; l < r.sweeps.size(); l++) {
+                ChipSweep &d = hr[levels_r[l].first + order[at[c].rev_at + l]];
+                fill(d, c, r.sweeps[l], at[c].rev);
+                if (l + 1 == r.sweeps.size()) d.flags = 0;  // only its sums are used
+            }
         };
-        std::vector<Level> levels_f, levels_r;
-        size_t k = 0;
-        for (size_t l = 0; l < lf; l++) {
-            levels_f.push_back({k, 0});
-            for (uint32_t c = 0; c < count; c++)
-                if (l < fwd[c].sweeps.size()) {
-                    fill(hf[k], c, fwd[c].sweeps[l], at[c].fwd);
-                    if (l == 0) hf[k].flags |= CHIP_INIT;
-                    k++;
-                }
-            levels_f.back().count = (uint32_t)(k - levels_f.back().first);
-        }
-        k = 0;
-        for (size_t l = 0; l < lr; l++) {
-            levels_r.push_back({k, 0});
-            for (uint32_t c = 0; c < count; c++)
-                if (l < rev[c].sweeps.size()) {
-                    fill(hr[k], c, rev[c].sweeps[l], at[c].rev);
-                    if (l + 1 == rev[c].sweeps.size()) hr[k].flags = 0;  // only its sums are used
-                    k++;
-                }
-            levels_r.back().count = (uint32_t)(k - levels_r.back().first);
-        }
+        std::atomic<uint32_t> next{0};
+        crew.run(std::min(most_threads(count), (uint64_t)total / (256 << 10) + 1), [&]() {
+            constexpr uint32_t kAtOnce = 8;
+            for (uint32_t c; (c = next.fetch_add(kAtOnce)) < count;)
+                for (uint32_t e = std::min(c + kAtOnce, count); c < e; c++) write(c);
+        });
         hipStream_t st = rt().stream;
         SPZ_HIP(hipEventRecord(begin, st));
         SPZ_HIP(hipMemcpyAsync(slot.dev, slot.host, total, hipMemcpyHostToDevice, st));
@@ -447,7 +526,8 @@ int spz_batch_adjoint(const spz_batch_circuit *circuits, uint64_t count, const s
         if (rc == SPZ_OK && hipMemsetAsync(sc.out.p, 0, (small.size() + gmax) * sizeof(double),
                                            rt().stream) != hipSuccess)
             rc = fail(SPZ_ERR_HIP, "batched adjoint clear failed");
-        Chunk ch{circuits, ops, hx, lds, small.size()};
+        Crew crew;
+        Chunk ch{circuits, ops, hx, lds, small.size(), crew};
         for (size_t a = 0; rc == SPZ_OK && a < small.size();) {
             size_t b = a;
             uint64_t tiles = 0, nops = 0;
