@@ -11,7 +11,17 @@
 //          into each sweep; floating-point results then differ from PLAIN only
 //          by rounding (the same products in a different order).
 //
-// Measurements, SWAPs and dense blocks end a run and execute on their own.
+// States of at most 12 qubits (no tile width asked for) keep program order and
+// STRICT arithmetic in AUTO too: a run of more than five ops is one launch
+// (spz_chip.hip), a shorter one goes op by op.  (At 11 and 12 qubits sweeps of
+// narrower tiles are faster, since they reorder: 96 random gates of 11 qubits 48
+// us against 69.  tile_qubits = 10 takes them.)
+//
+// Measurements and dense blocks end a run and execute on their own.  So do, above
+// 12 qubits, SWAPs with controls, and in DENSE5 every SWAP; SWAPs without controls
+// are a relabelling inside a sweep (FP32: only among themselves).  States of at
+// most 12 qubits take SWAPs, controlled ones too, as three CX.  A SWAP under
+// classical control always executes on its own.
 #include <stdlib.h>
 #include <string.h>
 

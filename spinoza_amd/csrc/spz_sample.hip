@@ -216,10 +216,9 @@ k_sample_block(const double *__restrict__ P, uint64_t nb, const SampleMeta *__re
 
 // Exclusive scan of the counts (in place: counts[b] becomes the block's first
 // position) and the list of the blocks' samples, at most kPer to a slot.  One
-// workgroup, kScan blocks to a thread at a time (one to a thread took 0.1 ms more
-// for 2^18 blocks).
-constexpr int kScan = 8;
-
+// workgroup, `kScan` blocks to a thread at a time: one, and eight where there are
+// more blocks than threads (one there took 0.1 ms more for 2^18 blocks).
+template <int kScan>
 __global__ void __launch_bounds__(kPT)
 k_sample_scan(uint32_t *__restrict__ counts, uint64_t nb, Slot *__restrict__ slots,
               SampleMeta *__restrict__ meta)
@@ -530,7 +529,10 @@ int sample_rounds(const spz_state_s *s, uint64_t nb, const double *uniforms, uin
                                counts, meta, direct ? host_meta : nullptr);
         hipLaunchKernelGGL(k_sample_block, dim3(g), dim3(kT), 0, st, P, nb, meta, U, m, counts,
                            blk, rank);
-        hipLaunchKernelGGL(k_sample_scan, dim3(1), dim3(kPT), 0, st, counts, nb, slots, meta);
+        if (nb <= kPT)
+            hipLaunchKernelGGL((k_sample_scan<1>), dim3(1), dim3(kPT), 0, st, counts, nb, slots, meta);
+        else
+            hipLaunchKernelGGL((k_sample_scan<8>), dim3(1), dim3(kPT), 0, st, counts, nb, slots, meta);
         hipLaunchKernelGGL(k_sample_order, dim3(g), dim3(kT), 0, st, counts, meta, blk, rank, m,
                            order);
         const unsigned gs = (unsigned)std::min<uint64_t>(m, nb + m / kPer);
