@@ -239,7 +239,9 @@ int spz_sample(spz_state s, const double *uniforms, uint64_t k, uint64_t *out);
  * dE/dtheta of op i for RX/RY/RZ/P ops (controlled or not) and 0 for other
  * ops.  ckpt_every > 0 stores |psi> every ckpt_every ops during the forward
  * pass and restores it in the reverse sweep; *drift (may be NULL) receives
- * the largest |psi_uncomputed - psi_checkpoint| seen. */
+ * the largest |psi_uncomputed - psi_checkpoint| seen.  Working states and up to
+ * 4 GiB of checkpoints stay allocated for the next call; any allocation of the
+ * library that fails gives them back and is tried again. */
 int spz_adjoint_grad(spz_state s, const spz_op *ops, uint64_t n_ops, double hx,
                      int ckpt_every, double *grad, double *energy, double *drift);
 

@@ -14,7 +14,7 @@
 // What bounded it: a persistent kernel that moved every gate's pairs through
 // the L2 (one workgroup, or a group of workgroups of one XCD with a barrier
 // around every gate that crossed their blocks): 33.3 ms of device time for 128
-// circuits of 10 to 18 qubits, 6.7 ms now (whole call 50.8 -> 10.3 ms).  Chunks
+// circuits of 10 to 18 qubits, 6.7 ms now (whole call 50.8 -> 9.7 ms).  Chunks
 // of 192 to 1536 tiles measured within 5% of each other.
 #include <math.h>
 #include <string.h>

@@ -13,7 +13,7 @@
 // and one wait per target (23 qubits: 69 passes of 22-28 us and 70 round
 // trips for x, y and z).  Now kExpectGroup targets share a pass, all targets of
 // a call share one second-level launch per pass and one wait, and results land
-// in pinned memory.  x, y and z of all 23 qubits and the energy: 3.08 -> 0.75
+// in pinned memory.  x, y and z of all 23 qubits and the energy: 3.08 -> 0.73
 // ms; a pass of 8 targets takes 28 us for z (one state read, then additions)
 // and 64 us for x or y.
 #include <algorithm>
